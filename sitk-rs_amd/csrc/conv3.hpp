@@ -1,0 +1,700 @@
+// The 3-D convolutions of the learned initializer on the gfx950 BF16 matrix
+// cores (v_mfma_f32_16x16x32_bf16, FP32 accumulation): forward, input gradient
+// and weight gradient of the stride-2 layers, and the two-channel first layer.
+//
+// Every kernel stages the voxels that a tile of output positions reads, zero
+// padding included, in LDS once for all 27 taps, and builds its matrix
+// operands from there. Voxels are channels-last, so a forward or input-
+// gradient operand (K = channels) is one 16-byte LDS read; the weight
+// gradient's K runs over positions, which channels-last does not keep
+// together, and its operands come through ds_read_b64_tr_b16, which hands
+// each lane four consecutive rows of its column out of a 4 x 16 block.
+// Voxels are spaced 2 C + 16 bytes apart in LDS: with stride-2 positions that
+// puts eight neighbouring rows' 32-byte pieces on different banks for
+// C = 16, 32, 64 and 128.
+//
+// MFMA 16x16x32 lane layout: lane l supplies row (A) or column (B) l mod 16,
+// K group 8 (l / 16) .. + 7, and receives D rows 4 (l / 16) .. + 3 of column
+// l mod 16.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <cstdint>
+#include <cstring>
+
+namespace sitkhip {
+namespace cnn {
+
+typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
+typedef __attribute__((ext_vector_type(4))) float f32x4;
+typedef short i16x4 __attribute__((ext_vector_type(4)));
+
+union Frag {
+    uint4 u;
+    bf16x8 v;
+    uint16_t h[8];
+    i16x4 t[2];
+};
+
+__device__ __forceinline__ bf16x8 zero_frag() {
+    Frag f;
+    f.u = make_uint4(0, 0, 0, 0);
+    return f.v;
+}
+__device__ __forceinline__ bf16x8 load_frag(const void *p) {
+    Frag f;
+    f.u = *reinterpret_cast<const uint4 *>(p);
+    return f.v;
+}
+// Two transposed LDS reads: elements 0..3 from `p`, 4..7 from `p + h`. Lane
+// 16 g + i passes the address of row i / 4, columns 4 (i mod 4) .. + 3 of its
+// group's 4 x 16 block and receives rows 0..3 of column i. All lanes take part.
+__device__ __forceinline__ bf16x8 tr_frag(const char *p, int h) {
+    typedef __attribute__((address_space(3))) i16x4 *lds_ptr;
+    Frag f;
+    f.t[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(p));
+    f.t[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(p + h));
+    return f.v;
+}
+__device__ __forceinline__ f32x4 mfma(bf16x8 a, bf16x8 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ f32x4 zero_acc() { return f32x4{0.0f, 0.0f, 0.0f, 0.0f}; }
+
+// Four floats to four BF16 (round to nearest even), one 8-byte word.
+__device__ __forceinline__ uint2 pack_bf16(const float v[4]) {
+    union {
+        __bf16 h[4];
+        uint2 u;
+    } w;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) w.h[e] = static_cast<__bf16>(v[e]);
+    return w.u;
+}
+__device__ __forceinline__ float bf16_at(const uint2 &w, int e) {
+    const uint32_t p = e < 2 ? w.x : w.y;
+    return __uint_as_float((e & 1) ? (p & 0xffff0000u) : (p << 16));
+}
+
+constexpr int kConvLanes = 256;
+
+// ------------------------------------------------ input tiles, stride 2
+// A chunk of output positions: ZP planes x R rows x all DO columns of one
+// sample. It reads input planes 2 z0 - 1 + .. , rows 2 y0 - 1 .. 2 y0 + 2 R - 1
+// and columns -1 .. DI - 1 (stride 2 never reaches past the high edge).
+// PL planes are staged; plane q's input z is first_z + q * step_z.
+template <int LGDO, int CI, int R, int ZP, int PL>
+struct InTile {
+    static constexpr int DO = 1 << LGDO, DI = 2 * DO;
+    static constexpr int ROWS = 2 * R + 1, COLS = DI + 1, VS = 2 * CI + 16;
+    static constexpr int P = ZP * R * DO;  // output positions
+    static constexpr int ZC = DO / ZP, YC = DO / R;
+    static constexpr int kBytes = PL * ROWS * COLS * VS;
+    static constexpr int kPieces = PL * ROWS * DI * (CI / 8);  // 16 bytes each
+    static constexpr int kPer = (kPieces + kConvLanes - 1) / kConvLanes;
+    static_assert(P % 16 == 0 && (ZP == 1 || R == DO), "whole position tiles");
+
+    __device__ static void chunk(int c, int &n, int &z0, int &y0) {
+        y0 = (c % YC) * R;
+        const int q = c / YC;
+        z0 = (q % ZC) * ZP;
+        n = q / ZC;
+    }
+    static int chunks(int n) { return n * ZC * YC; }
+    // column -1 of every row: zero, never overwritten
+    __device__ static void clear_edge(char *lds) {
+        for (int i = threadIdx.x; i < PL * ROWS * (VS / 16); i += kConvLanes)
+            *reinterpret_cast<uint4 *>(lds + (i / (VS / 16)) * COLS * VS + (i % (VS / 16)) * 16) =
+                make_uint4(0, 0, 0, 0);
+    }
+    __device__ static void load(const uint16_t *__restrict__ x, int n, int first_z, int step_z,
+                                int y0, uint4 (&v)[kPer]) {
+#pragma unroll
+        for (int k = 0; k < kPer; ++k) {
+            const int i = threadIdx.x + k * kConvLanes;
+            const int c8 = i % (CI / 8), xi = i / (CI / 8) % DI, q = i / (CI / 8 * DI);
+            const int zi = first_z + (q / ROWS) * step_z, yi = 2 * y0 - 1 + q % ROWS;
+            v[k] = make_uint4(0, 0, 0, 0);
+            if (i < kPieces && zi >= 0 && yi >= 0)
+                v[k] = *reinterpret_cast<const uint4 *>(
+                    x + (((static_cast<size_t>(n) * DI + zi) * DI + yi) * DI + xi) * CI + c8 * 8);
+        }
+    }
+    __device__ static void store(char *lds, const uint4 (&v)[kPer]) {
+#pragma unroll
+        for (int k = 0; k < kPer; ++k) {
+            const int i = threadIdx.x + k * kConvLanes;
+            const int c8 = i % (CI / 8), xi = i / (CI / 8) % DI, q = i / (CI / 8 * DI);
+            if (i < kPieces)
+                *reinterpret_cast<uint4 *>(lds + (q * COLS + xi + 1) * VS + c8 * 16) = v[k];
+        }
+    }
+    // Byte offset of output position p's first tap (kz = ky = kx = 0); `zs`
+    // staged planes lie between two output planes.
+    __device__ static int at(int p, int zs) {
+        const int xo = p % DO, r = p / DO % R, zp = p / (DO * R);
+        return ((zp * zs * ROWS + 2 * r) * COLS + 2 * xo) * VS;
+    }
+    __host__ __device__ static constexpr int tap(int kz, int ky, int kx) {
+        return ((kz * ROWS + ky) * COLS + kx) * VS;
+    }
+};
+
+// ------------------------------------------------------- forward, stride 2
+// y = bf16(relu(w x + b)). D rows are output channels (A: weights), columns
+// positions, so a lane ends with four consecutive channels of one position.
+// The four waves split the channel tiles first, then the position tiles. HOLD:
+// the wave's weights stay in registers and the workgroup walks many chunks;
+// otherwise they stream from L2 (layers whose weights exceed the registers
+// have few positions).
+// Bound by its traffic in layer 1 (268 MB in, 67 MB out for 32 pairs: 4.6 TB/s)
+// and by latency in layers 3-4 (few positions). Gathering the operands from
+// global memory, with every lane's voxel address worked out per K step, took
+// 203 us for layer 1 and 168 us for layers 2-4 of 32 pairs; this takes 73 and 58.
+template <int LGDO, int CI, int CO, int R, int COW, bool HOLD>
+__global__ __launch_bounds__(kConvLanes) void conv_forward(const uint16_t *__restrict__ x,
+                                                           const uint16_t *__restrict__ wb,
+                                                           const float *__restrict__ bias,
+                                                           uint16_t *__restrict__ y, int nchunks) {
+    using T = InTile<LGDO, CI, R, 1, 3>;
+    constexpr int K = 27 * CI, STEPS = (K + 31) / 32;
+    constexpr int RT = COW / 16, WR = RT < 4 ? RT : 4, NR = RT / WR;  // row tiles per wave
+    constexpr int WP = 4 / WR, PT = T::P / 16 / WP;                   // position tiles per wave
+    static_assert(PT >= 1 && PT * WP * 16 == T::P, "positions split over the waves");
+    extern __shared__ char lds[];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int r16 = lane & 15, g = lane >> 4;
+    const int row0 = blockIdx.y * COW + (w % WR) * NR * 16;
+    const int pt0 = (w / WR) * PT;
+    const uint16_t *wrow = wb + static_cast<size_t>(row0 + r16) * K + 8 * g;
+    auto weights = [&](int nr, int s) {
+        return (STEPS * 32 > K && s == STEPS - 1 && 32 * s + 8 * g >= K)
+                   ? zero_frag()
+                   : load_frag(wrow + static_cast<size_t>(nr) * 16 * K + 32 * s);
+    };
+    bf16x8 held[HOLD ? NR * STEPS : 1];
+    if (HOLD) {
+#pragma unroll
+        for (int i = 0; i < NR * STEPS; ++i) held[i] = weights(i / STEPS, i % STEPS);
+    }
+    int base[PT];
+#pragma unroll
+    for (int p = 0; p < PT; ++p)
+        base[p] = T::at((pt0 + p) * 16 + r16, 2) + (CI == 16 ? 16 * (g & 1) : 16 * g);
+    T::clear_edge(lds);
+    uint4 v[T::kPer];
+    int c = blockIdx.x, n, z0, y0;
+    if (c < nchunks) {
+        T::chunk(c, n, z0, y0);
+        T::load(x, n, 2 * z0 - 1, 1, y0, v);
+    }
+    for (; c < nchunks; c += gridDim.x) {
+        T::chunk(c, n, z0, y0);
+        __syncthreads();
+        T::store(lds, v);
+        __syncthreads();
+        const int cn = c + gridDim.x;
+        if (cn < nchunks) {
+            int n2, z2, y2;
+            T::chunk(cn, n2, z2, y2);
+            T::load(x, n2, 2 * z2 - 1, 1, y2, v);
+        }
+        f32x4 acc[NR][PT];
+#pragma unroll
+        for (int i = 0; i < NR; ++i)
+#pragma unroll
+            for (int p = 0; p < PT; ++p) acc[i][p] = zero_acc();
+#pragma unroll
+        for (int s = 0; s < STEPS; ++s) {
+            int off;
+            if constexpr (CI == 16) {  // two taps per step: this lane group's
+                const int t0 = 2 * s, t1 = 2 * s + 1 < 27 ? 2 * s + 1 : t0;
+                const int o0 = T::tap(t0 / 9, t0 / 3 % 3, t0 % 3), o1 = T::tap(t1 / 9, t1 / 3 % 3, t1 % 3);
+                off = g < 2 ? o0 : o1;
+            } else {
+                const int t = 32 * s / CI;
+                off = T::tap(t / 9, t / 3 % 3, t % 3) + 2 * (32 * s % CI);
+            }
+            bf16x8 b[PT];
+#pragma unroll
+            for (int p = 0; p < PT; ++p) {
+                b[p] = load_frag(lds + base[p] + off);
+                // the padding tap's weights are zero; so is what they meet
+                if (STEPS * 32 > K && s == STEPS - 1 && 32 * s + 8 * g >= K) b[p] = zero_frag();
+            }
+#pragma unroll
+            for (int i = 0; i < NR; ++i) {
+                const bf16x8 a = HOLD ? held[i * STEPS + s] : weights(i, s);
+#pragma unroll
+                for (int p = 0; p < PT; ++p) acc[i][p] = mfma(a, b[p], acc[i][p]);
+            }
+        }
+        const size_t pos0 = ((static_cast<size_t>(n) * T::DO + z0) * T::DO + y0) * T::DO;
+#pragma unroll
+        for (int i = 0; i < NR; ++i) {
+            const int co = row0 + 16 * i + 4 * g;
+#pragma unroll
+            for (int p = 0; p < PT; ++p) {
+                float o[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) o[e] = fmaxf(acc[i][p][e] + bias[co + e], 0.0f);
+                *reinterpret_cast<uint2 *>(y + (pos0 + (pt0 + p) * 16 + r16) * CO + co) = pack_bf16(o);
+            }
+        }
+    }
+}
+
+// ------------------------------------------------ weight gradient, stride 2
+// dW[co][tap][ci] = sum over positions of dy[m][co] x[m's tap][ci], and
+// db[co] = sum of dy[m][co] (one more column, of ones). A workgroup keeps the
+// sums of its KZN kernel planes and COW output channels in the accumulators
+// over its chunks (blockIdx.x, + gridDim.x, ...) and writes one partial row
+// [CO][27 CI], [CO]; reduce_partials adds the rows in a fixed tree.
+// Gathering each operand's eight positions from global memory one scalar at a
+// time, with bias sums and masks in passes of their own, took 5.6 ms for the
+// five layers of 24 pairs and 1.3 ms for those passes; this takes 0.21 ms and
+// the fold of the partial rows 0.025.
+template <int LGDO, int CI, int CO, int R, int ZP, int KZN, int COW>
+__global__ __launch_bounds__(kConvLanes) void conv_wgrad(const uint16_t *__restrict__ x,
+                                                         const uint16_t *__restrict__ dy,
+                                                         float *__restrict__ partial, int nchunks) {
+    using T = InTile<LGDO, CI, R, ZP, KZN * ZP>;
+    constexpr int DS = 2 * COW + 16;                       // bytes per staged dy position
+    constexpr int STEPS = T::P / 32, RT = COW / 16;
+    constexpr int NC = 9 * KZN * CI / 16, NJ = (NC + 3) / 4;  // column tiles, per wave
+    constexpr int DYP = T::P * COW / 8, DYN = (DYP + kConvLanes - 1) / kConvLanes;
+    static_assert(T::P % 32 == 0 && (KZN == 3 ? ZP == 1 : KZN == 1), "chunk shape");
+    extern __shared__ char lds[];
+    char *sdy = lds + T::kBytes;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int i16 = lane & 15, g = lane >> 4;
+    constexpr int KZG = 3 / KZN;  // workgroups along blockIdx.y per channel group
+    const int kz0 = (blockIdx.y % KZG) * KZN, co0 = (blockIdx.y / KZG) * COW;
+    const bool bias_here = kz0 == 0 && w == 3;
+
+    const int p0 = 8 * g + (i16 >> 2);  // this lane's row of the first 4 x 16 block
+    const int xbase = T::at(p0, 1) + 8 * (i16 & 3), dbase = p0 * DS + 8 * (i16 & 3);
+    constexpr int kXHalf = T::DO >= 8 ? 8 * T::VS : 2 * T::COLS * T::VS;     // position + 4
+    constexpr int kXStep = 2 * (32 / T::DO) * T::COLS * T::VS;               // position + 32
+    int toff[NJ];
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+        const int t = w + 4 * j, tap = t / (CI / 16), c = t % (CI / 16);
+        toff[j] = T::tap((tap / 9) * ZP, tap / 3 % 3, tap % 3) + 32 * c;
+    }
+    f32x4 acc[NJ][RT], accb[RT];
+#pragma unroll
+    for (int r = 0; r < RT; ++r) {
+        accb[r] = zero_acc();
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) acc[j][r] = zero_acc();
+    }
+    Frag ones;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) ones.h[e] = 0x3f80;
+
+    T::clear_edge(lds);
+    uint4 v[T::kPer], d[DYN];
+    auto fetch = [&](int c) {
+        int n, z0, y0;
+        T::chunk(c, n, z0, y0);
+        T::load(x, n, 2 * z0 - 1 + kz0, KZN == 3 ? 1 : 2, y0, v);
+        const size_t pos0 = ((static_cast<size_t>(n) * T::DO + z0) * T::DO + y0) * T::DO;
+#pragma unroll
+        for (int k = 0; k < DYN; ++k) {
+            const int i = threadIdx.x + k * kConvLanes;
+            if (i < DYP)
+                d[k] = *reinterpret_cast<const uint4 *>(dy + (pos0 + i / (COW / 8)) * CO + co0 +
+                                                        (i % (COW / 8)) * 8);
+        }
+    };
+    int c = blockIdx.x;
+    if (c < nchunks) fetch(c);
+    for (; c < nchunks; c += gridDim.x) {
+        __syncthreads();
+        T::store(lds, v);
+#pragma unroll
+        for (int k = 0; k < DYN; ++k) {
+            const int i = threadIdx.x + k * kConvLanes;
+            if (i < DYP)
+                *reinterpret_cast<uint4 *>(sdy + (i / (COW / 8)) * DS + (i % (COW / 8)) * 16) = d[k];
+        }
+        __syncthreads();
+        if (c + static_cast<int>(gridDim.x) < nchunks) fetch(c + gridDim.x);
+#pragma unroll
+        for (int s = 0; s < STEPS; ++s) {
+            bf16x8 a[RT];
+#pragma unroll
+            for (int r = 0; r < RT; ++r) a[r] = tr_frag(sdy + dbase + s * 32 * DS + 32 * r, 4 * DS);
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) {
+                if (NC % 4 != 0 && w + 4 * j >= NC) continue;  // the same for the whole wave
+                const bf16x8 b = tr_frag(lds + xbase + toff[j] + s * kXStep, kXHalf);
+#pragma unroll
+                for (int r = 0; r < RT; ++r) acc[j][r] = mfma(a[r], b, acc[j][r]);
+            }
+            if (bias_here)
+#pragma unroll
+                for (int r = 0; r < RT; ++r) accb[r] = mfma(a[r], ones.v, accb[r]);
+        }
+    }
+    float *out = partial + static_cast<size_t>(blockIdx.x) * (CO * 27 * CI + CO);
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+        const int t = w + 4 * j;
+        if (NC % 4 != 0 && t >= NC) continue;
+        const int col = kz0 * 9 * CI + t * 16 + i16;
+#pragma unroll
+        for (int r = 0; r < RT; ++r)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                out[static_cast<size_t>(co0 + 16 * r + 4 * g + e) * (27 * CI) + col] = acc[j][r][e];
+    }
+    if (bias_here && i16 == 0)
+#pragma unroll
+        for (int r = 0; r < RT; ++r)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) out[CO * 27 * CI + co0 + 16 * r + 4 * g + e] = accb[r][e];
+}
+
+// ------------------------------------------------- input gradient, stride 2
+// dx at input position 2 q + p (p a parity triple) sums, along each axis, the
+// taps (k = 1, output q) for p = 0 and (k = 0, output q + 1), (k = 2, output
+// q) for p = 1: eight dense products with 1, 2, 2, 4, 2, 4, 4 and 8 taps over
+// the same staged dy, 27 in all, where one product over every input position
+// would multiply zeros in seven of eight taps. The result is masked by the
+// layer's input (its ReLU) as it is stored.
+// CG > 1: the parity classes are spread over blockIdx.y (layers with few
+// positions). One product over every position took 495 us a layer for layers
+// 1-2 of 24 pairs and 78 for layers 3-4, its masks 0.18 ms more; this takes
+// 157 / 54 and 17 / 17.
+template <int LGDO, int CI, int CO, int QY, int QZ, int CG>
+__global__ __launch_bounds__(kConvLanes) void conv_dgrad(const uint16_t *__restrict__ dy,
+                                                         const uint16_t *__restrict__ wt,
+                                                         const uint16_t *__restrict__ act,
+                                                         uint16_t *__restrict__ dx) {
+    constexpr int DO = 1 << LGDO, DI = 2 * DO, DS = 2 * CO + 16;
+    constexpr int Y1 = QY + 1, Z1 = QZ + 1, X1 = DO + 1;
+    constexpr int P = QZ * QY * DO, WR = CI / 16 < 4 ? CI / 16 : 4, WP = 4 / WR, PT = P / 16 / WP;
+    static_assert(CI / 16 == WR && PT >= 1, "one row tile per wave");
+    extern __shared__ char lds[];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int r16 = lane & 15, g = lane >> 4;
+    const int y0 = (blockIdx.x % (DO / QY)) * QY, z0 = (blockIdx.x / (DO / QY)) % (DO / QZ) * QZ;
+    const size_t n = blockIdx.x / ((DO / QY) * (DO / QZ));
+    constexpr int kPieces = Z1 * Y1 * X1 * (CO / 8);
+#pragma unroll 4
+    for (int i = threadIdx.x; i < kPieces; i += kConvLanes) {
+        const int c8 = i % (CO / 8), xo = i / (CO / 8) % X1, q = i / (CO / 8 * X1);
+        const int yo = y0 + q % Y1, zo = z0 + q / Y1;
+        uint4 v = make_uint4(0, 0, 0, 0);
+        if (xo < DO && yo < DO && zo < DO)
+            v = *reinterpret_cast<const uint4 *>(dy + (((n * DO + zo) * DO + yo) * DO + xo) * CO + c8 * 8);
+        *reinterpret_cast<uint4 *>(lds + (q * X1 + xo) * DS + c8 * 16) = v;
+    }
+    __syncthreads();
+    const int ci0 = (w % WR) * 16;
+    int base[PT], zi[PT], yi[PT], xi[PT];
+#pragma unroll
+    for (int t = 0; t < PT; ++t) {
+        const int p = ((w / WR) * PT + t) * 16 + r16;
+        const int qx = p % DO, qy = p / DO % QY, qz = p / (DO * QY);
+        base[t] = ((qz * Y1 + qy) * X1 + qx) * DS + 16 * g;
+        zi[t] = 2 * (z0 + qz);
+        yi[t] = 2 * (y0 + qy);
+        xi[t] = 2 * qx;
+    }
+    // eight classes with 8, (4 2 1), (4 2), (4 2) taps per group
+    const unsigned group = CG == 1 ? 0xffu : (0x50240b80u >> (8 * blockIdx.y)) & 0xffu;
+    const uint16_t *wrow = wt + static_cast<size_t>(ci0 + r16) * 27 * CO + 8 * g;
+    for (int cls = 0; cls < 8; ++cls) {
+        if (!((group >> cls) & 1u)) continue;
+        const int pz = cls >> 2, py = (cls >> 1) & 1, px = cls & 1;
+        f32x4 acc[PT];
+#pragma unroll
+        for (int t = 0; t < PT; ++t) acc[t] = zero_acc();
+        for (int tz = 0; tz <= pz; ++tz)
+            for (int ty = 0; ty <= py; ++ty)
+                for (int tx = 0; tx <= px; ++tx) {
+                    // parity 1: first k = 0 at q + 1, then k = 2 at q
+                    const int kz = pz ? 2 * tz : 1, ky = py ? 2 * ty : 1, kx = px ? 2 * tx : 1;
+                    const int off = (((pz - tz) * Y1 + (py - ty)) * X1 + (px - tx)) * DS;
+                    const uint16_t *wk = wrow + (kz * 9 + ky * 3 + kx) * CO;
+#pragma unroll
+                    for (int s = 0; s < CO / 32; ++s) {
+                        const bf16x8 a = load_frag(wk + 32 * s);
+#pragma unroll
+                        for (int t = 0; t < PT; ++t)
+                            acc[t] = mfma(a, load_frag(lds + base[t] + off + 64 * s), acc[t]);
+                    }
+                }
+#pragma unroll
+        for (int t = 0; t < PT; ++t) {
+            const size_t at =
+                (((n * DI + zi[t] + pz) * DI + yi[t] + py) * DI + xi[t] + px) * CI + ci0 + 4 * g;
+            const uint2 y = *reinterpret_cast<const uint2 *>(act + at);
+            float o[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[e] = bf16_at(y, e) > 0.0f ? acc[t][e] : 0.0f;
+            *reinterpret_cast<uint2 *>(dx + at) = pack_bf16(o);
+        }
+    }
+}
+
+// ----------------------------------------------------------- first layer
+// 2 -> 16 channels, stride 1, 64^3. A voxel's two channels are one 4-byte
+// word. A chunk is four output rows (one per wave) of one plane; it reads
+// 3 planes x 6 rows x voxels -2 .. 65, zero outside the volume.
+constexpr int kC0Rows = 4, kC0Cols = 68;
+constexpr int kC0Vox = 3 * (kC0Rows + 2) * kC0Cols;
+constexpr int kC0Per = (kC0Vox + kConvLanes - 1) / kConvLanes;
+constexpr int kC0PerPlane = 64 / kC0Rows;
+
+__device__ __forceinline__ void c0_chunk(int c, size_t &n, int &z, int &y0) {
+    y0 = (c % kC0PerPlane) * kC0Rows;
+    z = (c / kC0PerPlane) & 63;
+    n = static_cast<size_t>(c / kC0PerPlane) >> 6;
+}
+__device__ __forceinline__ void c0_load(const uint32_t *__restrict__ x, int c, uint32_t (&v)[kC0Per]) {
+    size_t n;
+    int z, y0;
+    c0_chunk(c, n, z, y0);
+#pragma unroll
+    for (int k = 0; k < kC0Per; ++k) {
+        const int i = threadIdx.x + k * kConvLanes;
+        const int xi = i % kC0Cols - 2, row = i / kC0Cols;
+        const int yi = y0 + row % (kC0Rows + 2) - 1, zi = z + row / (kC0Rows + 2) - 1;
+        v[k] = 0;
+        if (i < kC0Vox && (xi | yi | zi) >= 0 && xi < 64 && yi < 64 && zi < 64)
+            v[k] = x[((n * 64 + zi) * 64 + yi) * 64 + xi];
+    }
+}
+__device__ __forceinline__ void c0_store(char *lds, const uint32_t (&v)[kC0Per]) {
+#pragma unroll
+    for (int k = 0; k < kC0Per; ++k) {
+        const int i = threadIdx.x + k * kConvLanes;
+        if (i < kC0Vox) *reinterpret_cast<uint32_t *>(lds + 4 * i) = v[k];
+    }
+}
+
+// Forward: K = 27 taps x 2 channels = 54, zero-padded to two MFMA steps; an
+// operand's eight K values are four voxel words. Rows are output channels, so
+// a lane stores four consecutive channels of one position. The weights stay
+// in registers over the workgroup's chunks, and the next chunk's voxels load
+// while this one's are multiplied: 163 us for 32 pairs with one chunk per
+// workgroup and voxels of 16 bytes, 96 now (301 MB: 3.1 TB/s).
+__global__ __launch_bounds__(kConvLanes) void conv0_forward(const uint32_t *__restrict__ x,
+                                                            const uint16_t *__restrict__ wb, int ld,
+                                                            const float *__restrict__ bias,
+                                                            uint16_t *__restrict__ y, int nchunks) {
+    __shared__ __attribute__((aligned(16))) char lds[4 * kC0Vox];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int r = lane & 15, g = lane >> 4;
+    bf16x8 a[2];
+    int off[2][4];
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+        Frag f;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int tap = 16 * s + 4 * g + j, t = tap < 27 ? tap : 26;
+            f.h[2 * j] = tap < 27 ? wb[(r * 27 + t) * ld] : static_cast<uint16_t>(0);
+            f.h[2 * j + 1] = tap < 27 ? wb[(r * 27 + t) * ld + 1] : static_cast<uint16_t>(0);
+            off[s][j] = (((t / 9) * (kC0Rows + 2) + w + t / 3 % 3) * kC0Cols + r + t % 3 + 1) * 4;
+        }
+        a[s] = f.v;
+    }
+    float b4[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) b4[e] = bias[4 * g + e];
+    uint32_t v[kC0Per];
+    int c = blockIdx.x;
+    if (c < nchunks) c0_load(x, c, v);
+    for (; c < nchunks; c += gridDim.x) {
+        __syncthreads();
+        c0_store(lds, v);
+        __syncthreads();
+        if (c + static_cast<int>(gridDim.x) < nchunks) c0_load(x, c + gridDim.x, v);
+        size_t n;
+        int z, y0;
+        c0_chunk(c, n, z, y0);
+        uint16_t *row = y + (((n * 64 + z) * 64 + y0 + w) * 64 + r) * 16 + 4 * g;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            f32x4 acc = zero_acc();
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                uint32_t q[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    q[j] = *reinterpret_cast<const uint32_t *>(lds + off[s][j] + 64 * t);
+                    if (16 * s + 4 * g + j >= 27) q[j] = 0;  // padding: zero weights meet zeros
+                }
+                Frag f;
+                f.u = make_uint4(q[0], q[1], q[2], q[3]);
+                acc = mfma(a[s], f.v, acc);
+            }
+            float o[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[e] = fmaxf(acc[e] + b4[e], 0.0f);
+            *reinterpret_cast<uint2 *>(row + 16 * 16 * t) = pack_bf16(o);
+        }
+    }
+}
+
+// Weight gradient: the three kx taps of one (kz, ky) are 12 consecutive bytes
+// of a staged row, so two (kz, ky) pairs fill a 16-column tile with four voxels
+// each (the fourth, past the taps, is computed and dropped). The transposed
+// read takes 8-byte pieces on 8-byte boundaries: odd columns x read voxels
+// x - 1 .. x + 2, even ones x - 2 .. x + 1, in accumulators of their own. Each
+// wave takes one row of 64 positions per chunk.
+constexpr int kW0Dy = 48;  // bytes per staged dy position (16 channels + 16)
+constexpr int kW0Tile = 4 * kC0Vox;
+constexpr int kW0Lds = kW0Tile + kC0Rows * 64 * kW0Dy;
+constexpr int kW0Out = 16 * 54 + 16;      // [16][27][2] and the bias
+
+__global__ __launch_bounds__(kConvLanes) void conv0_wgrad(const uint32_t *__restrict__ x,
+                                                          const uint16_t *__restrict__ dy,
+                                                          float *__restrict__ partial, int nchunks) {
+    __shared__ __attribute__((aligned(16))) char lds[kW0Lds];
+    char *sdy = lds + kW0Tile;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int i16 = lane & 15, g = lane >> 4;
+    f32x4 acc[2][5], accb = zero_acc();
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+#pragma unroll
+        for (int j = 0; j < 5; ++j) acc[q][j] = zero_acc();
+    Frag ones;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) ones.h[e] = 0x3f80;
+    const int kk = 8 * g + (i16 >> 2);  // position 2 kk + parity of the row
+    const int sub = i16 & 3;
+    int xoff[5];
+#pragma unroll
+    for (int j = 0; j < 5; ++j) {
+        const int q = min(2 * j + (sub >> 1), 8);  // (kz, ky)
+        xoff[j] = (((q / 3) * (kC0Rows + 2) + w + q % 3) * kC0Cols + 2 * kk + 2 * (sub & 1)) * 4;
+    }
+    const int dbase = (w * 64 + 2 * kk) * kW0Dy + 8 * sub;
+    constexpr int kDyN = kC0Rows * 64 * 2 / kConvLanes;
+    uint32_t v[kC0Per];
+    uint4 d[kDyN];
+    auto fetch = [&](int c) {
+        c0_load(x, c, v);
+        size_t n;
+        int z, y0;
+        c0_chunk(c, n, z, y0);
+        const size_t pos0 = ((n * 64 + z) * 64 + y0) * 64;
+#pragma unroll
+        for (int k = 0; k < kDyN; ++k)
+            d[k] = *reinterpret_cast<const uint4 *>(dy + pos0 * 16 + (threadIdx.x + k * kConvLanes) * 8);
+    };
+    int c = blockIdx.x;
+    if (c < nchunks) fetch(c);
+    for (; c < nchunks; c += gridDim.x) {
+        __syncthreads();
+        c0_store(lds, v);
+#pragma unroll
+        for (int k = 0; k < kDyN; ++k) {
+            const int i = threadIdx.x + k * kConvLanes;
+            *reinterpret_cast<uint4 *>(sdy + (i >> 1) * kW0Dy + (i & 1) * 16) = d[k];
+        }
+        __syncthreads();
+        if (c + static_cast<int>(gridDim.x) < nchunks) fetch(c + gridDim.x);
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {  // parity of x
+            const bf16x8 a = tr_frag(sdy + dbase + q * kW0Dy, 8 * kW0Dy);
+#pragma unroll
+            for (int j = 0; j < 5; ++j)
+                acc[q][j] = mfma(a, tr_frag(lds + xoff[j] + q * 8, 32), acc[q][j]);
+            accb = mfma(a, ones.v, accb);
+        }
+    }
+    // the four waves' tiles, added in order
+    float *out = partial + static_cast<size_t>(blockIdx.x) * kW0Out;
+    float *red = reinterpret_cast<float *>(lds);  // tile by tile: [wave][co][column]
+    static_assert(kW0Lds >= 4 * 256 * 4, "the waves' tiles fit");
+    const int t = threadIdx.x;
+    const int co = t >> 4, col = t & 15;
+    float sum[2][5];
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+#pragma unroll
+        for (int j = 0; j < 5; ++j) {
+            __syncthreads();
+#pragma unroll
+            for (int e = 0; e < 4; ++e) red[w * 256 + (4 * g + e) * 16 + i16] = acc[q][j][e];
+            __syncthreads();
+            sum[q][j] = ((red[t] + red[256 + t]) + red[512 + t]) + red[768 + t];
+        }
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < 4; ++e) red[w * 256 + (4 * g + e) * 16 + i16] = accb[e];
+    __syncthreads();
+    const float db = ((red[t] + red[256 + t]) + red[512 + t]) + red[768 + t];
+    if (col == 0) out[16 * 54 + co] = db;
+    // even x: column (voxel v, channel c) is tap kx = v - 1; odd x: kx = v.
+    float *even = red, *odd = red + 256;
+#pragma unroll
+    for (int j = 0; j < 5; ++j) {
+        __syncthreads();
+        even[t] = sum[0][j];
+        odd[t] = sum[1][j];
+        __syncthreads();
+        const int q = 2 * j + (col >> 3), kx = (col >> 1) & 3, ch = col & 1;
+        if (q < 9 && kx < 3)
+            out[co * 54 + (q * 3 + kx) * 2 + ch] = even[t + 2] + odd[t];
+    }
+}
+
+// ---------------------------------------------------------- partial rows
+// Layers' partial rows summed into the gradient vector in one launch: a
+// workgroup takes 64 consecutive values of one layer, lane (s, i) adds rows
+// s, s + 4, ... of value i, and the four sums are added in order. Value i of
+// a row goes to out[(i / inner) * ld + i % inner] (the first layer's two used
+// channels lie eight apart in the parameter vector; its bias follows).
+struct PartialRows {
+    const float *p;
+    float *out, *out_bias;  // values from `len` on go to out_bias
+    int rows, len, total, inner, ld;
+    unsigned first_block;
+};
+constexpr int kMaxPartialJobs = 5;
+struct PartialJobs {
+    PartialRows j[kMaxPartialJobs];
+    int n;
+};
+
+__global__ __launch_bounds__(kConvLanes) void reduce_partials(PartialJobs J) {
+    __shared__ float s_sum[4][64];
+    int k = 0;
+    while (k + 1 < J.n && blockIdx.x >= J.j[k + 1].first_block) ++k;
+    const PartialRows &q = J.j[k];
+    const int lane = threadIdx.x & 63, s = threadIdx.x >> 6;
+    const int i = static_cast<int>(blockIdx.x - q.first_block) * 64 + lane;
+    float a = 0.0f;
+    if (i < q.total) {
+        const float *p = q.p + i;
+        int r = s;
+        for (; r + 28 < q.rows; r += 32) {
+            float v[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) v[u] = p[static_cast<size_t>(r + 4 * u) * q.total];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) a += v[u];
+        }
+        for (; r < q.rows; r += 4) a += p[static_cast<size_t>(r) * q.total];
+    }
+    s_sum[s][lane] = a;
+    __syncthreads();
+    if (s == 0 && i < q.total) {
+        const float t = ((s_sum[0][lane] + s_sum[1][lane]) + s_sum[2][lane]) + s_sum[3][lane];
+        if (i < q.len) q.out[(i / q.inner) * q.ld + i % q.inner] = t;
+        else q.out_bias[i - q.len] = t;
+    }
+}
+
+}  // namespace cnn
+}  // namespace sitkhip

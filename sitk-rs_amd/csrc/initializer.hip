@@ -14,15 +14,12 @@
 // Zero 'same' padding. Outputs: the 9 entries of (A - I) and t / 10 mm of the
 // affine x -> A (x - c) + t + c about the fixed image's centre c.
 //
-// Layout: activations channels-last [n][z][y][x][c] in BF16 (input channels
-// padded to 8 with zeros so every 8-wide K group is one 16-byte load); conv
-// weights [co][tap][ci] (tap = kz*9 + ky*3 + kx). Every convolution -- forward,
-// input gradient, weight gradient -- is one implicit GEMM on the gfx950 BF16
-// matrix cores (v_mfma_f32_16x16x32_bf16, FP32 accumulation): a workgroup of 4
-// waves computes a (32 WM) x (32 WN) tile, each wave 2 x 2 MFMA tiles, with the
-// A and B fragments fetched by per-GEMM gather functors. The weight gradient
-// is split over K (the output positions) into fixed partial rows that a second
-// kernel adds in order, so training is deterministic. Master weights, their
+// Layout: activations channels-last [n][z][y][x][c] in BF16 (the input's two
+// channels as one 4-byte word per voxel); conv weights [co][tap][ci] (tap =
+// kz*9 + ky*3 + kx, the first layer's ci padded to 8 in the parameter vector).
+// The convolutions' kernels are in conv3.hpp. The weight gradient is split
+// over the output positions into fixed partial rows that a second kernel adds
+// in a fixed order, so training is deterministic. Master weights, their
 // gradients and Adam's moments are FP32; the MLP head (0.01% of the FLOPs) runs
 // in FP32 on the vector units.
 #include <hip/hip_runtime.h>
@@ -35,18 +32,17 @@
 #include <vector>
 
 #include "common.hpp"
+#include "conv3.hpp"
 #include "image.hpp"
 #include "metric.hpp"
 
 namespace sitkhip {
 namespace cnn {
 
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
-typedef __attribute__((ext_vector_type(4))) float f32x4;
-
 constexpr int kLayers = 5;
 constexpr int kEdge = 64;          // input edge
-constexpr int kCin0 = 8;           // padded input channels (2 used)
+constexpr int kCin0 = 8;           // input channels of the parameter layout (2 used)
+constexpr int kCin0Used = 2;       // input channels held in memory
 constexpr int kFeat = 128;         // GAP features
 constexpr int kHidden = 128;
 constexpr int kOut = 12;
@@ -68,408 +64,7 @@ __host__ __device__ inline float bf2f(uint16_t h) {
     return f;
 }
 
-union Frag {
-    uint4 u;
-    bf16x8 v;
-    uint16_t h[8];
-};
-
-__device__ __forceinline__ bf16x8 zero_frag() {
-    Frag f;
-    f.u = make_uint4(0, 0, 0, 0);
-    return f.v;
-}
-__device__ __forceinline__ bf16x8 load_frag(const uint16_t *p) {
-    Frag f;
-    f.u = *reinterpret_cast<const uint4 *>(p);
-    return f.v;
-}
-
-// One convolution's geometry (all edges and channel counts powers of two).
-struct ConvGeom {
-    int n;                      // batch
-    int lg_di, lg_do;           // log2 input / output edge
-    int lg_ci, lg_co;           // log2 input / output channels
-    int stride;                 // 1 or 2
-    int ci, co;
-    int di, dout;
-};
-
-__device__ __forceinline__ void split_pos(int m, int lg, int &n, int &z, int &y, int &x) {
-    const int mask = (1 << lg) - 1;
-    x = m & mask;
-    y = (m >> lg) & mask;
-    z = (m >> (2 * lg)) & mask;
-    n = m >> (3 * lg);
-}
-
-__device__ __forceinline__ size_t pos_index(int n, int z, int y, int x, int lg) {
-    return (((((static_cast<size_t>(n) << lg) + z) << lg) + y) << lg) + x;
-}
-
-__device__ __forceinline__ void split_tap(int tap, int &kz, int &ky, int &kx) {
-    kz = tap / 9;
-    const int r = tap - 9 * kz;
-    ky = r / 3;
-    kx = r - 3 * ky;
-}
-
-// ------------------------------------------------------- gather functors
-// Forward, A: im2col of the input. Row m = output position, k = tap * ci + c.
-struct FwdA {
-    const uint16_t *x;
-    ConvGeom g;
-    __device__ __forceinline__ bf16x8 operator()(int m, int k) const {
-        const int M = g.n << (3 * g.lg_do);
-        const int K = 27 << g.lg_ci;
-        if (m >= M || k >= K) return zero_frag();
-        const int tap = k >> g.lg_ci, c0 = k & (g.ci - 1);
-        int kz, ky, kx, n, zo, yo, xo;
-        split_tap(tap, kz, ky, kx);
-        split_pos(m, g.lg_do, n, zo, yo, xo);
-        const int zi = zo * g.stride + kz - 1, yi = yo * g.stride + ky - 1, xi = xo * g.stride + kx - 1;
-        if (zi < 0 || yi < 0 || xi < 0 || zi >= g.di || yi >= g.di || xi >= g.di) return zero_frag();
-        const size_t pos = pos_index(n, zi, yi, xi, g.lg_di);
-        return load_frag(x + (pos << g.lg_ci) + c0);
-    }
-};
-
-// A dense row-major BF16 matrix [rows][ld] read as 8-wide K groups.
-struct RowsB {
-    const uint16_t *w;
-    int rows, K, ld;
-    __device__ __forceinline__ bf16x8 operator()(int r, int k) const {
-        if (r >= rows || k >= K) return zero_frag();
-        return load_frag(w + static_cast<size_t>(r) * ld + k);
-    }
-};
-
-// Input gradient, A: row m = input position, k = tap * co + c. The output
-// position that tap reads this input from: zo = (zi + 1 - kz) / stride when
-// that divides and lands inside.
-struct DgradA {
-    const uint16_t *dy;  // masked output gradient, channels-last
-    ConvGeom g;
-    __device__ __forceinline__ bf16x8 operator()(int m, int k) const {
-        const int M = g.n << (3 * g.lg_di);
-        const int K = 27 << g.lg_co;
-        if (m >= M || k >= K) return zero_frag();
-        const int tap = k >> g.lg_co, c0 = k & (g.co - 1);
-        int kz, ky, kx, n, zi, yi, xi;
-        split_tap(tap, kz, ky, kx);
-        split_pos(m, g.lg_di, n, zi, yi, xi);
-        int zo = zi + 1 - kz, yo = yi + 1 - ky, xo = xi + 1 - kx;
-        if (g.stride == 2) {
-            if ((zo | yo | xo) & 1) return zero_frag();
-            zo >>= 1;
-            yo >>= 1;
-            xo >>= 1;
-        }
-        if (zo < 0 || yo < 0 || xo < 0 || zo >= g.dout || yo >= g.dout || xo >= g.dout) return zero_frag();
-        const size_t pos = pos_index(n, zo, yo, xo, g.lg_do);
-        return load_frag(dy + (pos << g.lg_co) + c0);
-    }
-};
-
-// Weight gradient, A: row = output channel co, k = 8 consecutive output
-// positions (gathered with stride co).
-struct WgradA {
-    const uint16_t *dy;
-    ConvGeom g;
-    __device__ __forceinline__ bf16x8 operator()(int co, int k) const {
-        const int M = g.n << (3 * g.lg_do);
-        Frag f;
-#pragma unroll
-        for (int j = 0; j < 8; ++j)
-            f.h[j] = (co < g.co && k + j < M) ? dy[(static_cast<size_t>(k + j) << g.lg_co) + co] : 0;
-        return f.v;
-    }
-};
-
-// Weight gradient, B: row = (tap, ci), k = 8 consecutive output positions:
-// the input value that each position reads through that tap.
-struct WgradB {
-    const uint16_t *x;
-    ConvGeom g;
-    __device__ __forceinline__ bf16x8 operator()(int r, int k) const {
-        const int M = g.n << (3 * g.lg_do);
-        const int R = 27 << g.lg_ci;
-        Frag f;
-        if (r >= R) {
-            f.u = make_uint4(0, 0, 0, 0);
-            return f.v;
-        }
-        const int tap = r >> g.lg_ci, c = r & (g.ci - 1);
-        int kz, ky, kx;
-        split_tap(tap, kz, ky, kx);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            uint16_t v = 0;
-            const int m = k + j;
-            if (m < M) {
-                int n, zo, yo, xo;
-                split_pos(m, g.lg_do, n, zo, yo, xo);
-                const int zi = zo * g.stride + kz - 1, yi = yo * g.stride + ky - 1,
-                          xi = xo * g.stride + kx - 1;
-                if (zi >= 0 && yi >= 0 && xi >= 0 && zi < g.di && yi < g.di && xi < g.di) {
-                    const size_t pos = pos_index(n, zi, yi, xi, g.lg_di);
-                    v = x[(pos << g.lg_ci) + c];
-                }
-            }
-            f.h[j] = v;
-        }
-        return f.v;
-    }
-};
-
-// ------------------------------------------------------------ epilogues
-struct EpiBiasRelu {  // y = bf16(relu(acc + bias))
-    uint16_t *y;
-    const float *bias;
-    int ldc;
-    __device__ __forceinline__ void operator()(int, int m, int n, float acc) const {
-        const float v = fmaxf(acc + bias[n], 0.0f);
-        y[static_cast<size_t>(m) * ldc + n] = f2bf(v);
-    }
-};
-struct EpiStoreBf16 {
-    uint16_t *y;
-    int ldc;
-    __device__ __forceinline__ void operator()(int, int m, int n, float acc) const {
-        y[static_cast<size_t>(m) * ldc + n] = f2bf(acc);
-    }
-};
-struct EpiPartial {  // partial[split][m][n]
-    float *p;
-    int M, N;
-    __device__ __forceinline__ void operator()(int split, int m, int n, float acc) const {
-        p[(static_cast<size_t>(split) * M + m) * N + n] = acc;
-    }
-};
-
-// ------------------------------------------------------------------ GEMM
-// C[m][n] = sum_k A(m, k) B(n, k) over k in this workgroup's split
-// [z * kchunk, min(K, (z + 1) * kchunk)); kchunk is a multiple of 32.
-// MFMA 16x16x32 BF16 lane layout: lane l supplies A row (l mod 16) and B
-// column (l mod 16) with K group 8 * (l / 16) .. + 7, and receives D rows
-// 4 * (l / 16) .. + 3 of column (l mod 16).
-template <int WM, int WN, bool PIPE, class FA, class FB, class EP>
-__global__ __launch_bounds__(256) void mfma_gemm(FA fa, FB fb, EP ep, int M, int N, int K,
-                                                 int kchunk) {
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int wm = w % WM, wn = w / WM;
-    const int m0 = blockIdx.x * (32 * WM) + wm * 32;
-    const int n0 = blockIdx.y * (32 * WN) + wn * 32;
-    const int kb = blockIdx.z * kchunk;
-    const int ke = min(K, kb + kchunk);
-    f32x4 acc[2][2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    const int r = lane & 15, kg = (lane >> 4) * 8;
-    // PIPE: the next K step's four fragments are fetched before the current
-    // step's MFMAs issue, so their gathers overlap the math (measured: the
-    // forward layers 1-4 139 -> 93 us each for 32 pairs; the input-gradient
-    // GEMMs, whose gathers are already spread, 371 -> 418 us, so they do not)
-    bf16x8 a0, a1, b0, b1;
-    if (!PIPE) {
-        for (int k = kb; k < ke; k += 32) {
-            a0 = fa(m0 + r, k + kg);
-            a1 = fa(m0 + 16 + r, k + kg);
-            b0 = fb(n0 + r, k + kg);
-            b1 = fb(n0 + 16 + r, k + kg);
-            acc[0][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, b0, acc[0][0], 0, 0, 0);
-            acc[0][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, b1, acc[0][1], 0, 0, 0);
-            acc[1][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, b0, acc[1][0], 0, 0, 0);
-            acc[1][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, b1, acc[1][1], 0, 0, 0);
-        }
-    }
-    if (PIPE && kb < ke) {
-        a0 = fa(m0 + r, kb + kg);
-        a1 = fa(m0 + 16 + r, kb + kg);
-        b0 = fb(n0 + r, kb + kg);
-        b1 = fb(n0 + 16 + r, kb + kg);
-    }
-    for (int k = kb; PIPE && k < ke; k += 32) {
-        const int kn = k + 32;
-        bf16x8 na0 = zero_frag(), na1 = zero_frag(), nb0 = zero_frag(), nb1 = zero_frag();
-        if (kn < ke) {
-            na0 = fa(m0 + r, kn + kg);
-            na1 = fa(m0 + 16 + r, kn + kg);
-            nb0 = fb(n0 + r, kn + kg);
-            nb1 = fb(n0 + 16 + r, kn + kg);
-        }
-        acc[0][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, b0, acc[0][0], 0, 0, 0);
-        acc[0][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, b1, acc[0][1], 0, 0, 0);
-        acc[1][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, b0, acc[1][0], 0, 0, 0);
-        acc[1][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, b1, acc[1][1], 0, 0, 0);
-        a0 = na0;
-        a1 = na1;
-        b0 = nb0;
-        b1 = nb1;
-    }
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int row = m0 + 16 * i + 4 * (lane >> 4) + e;
-                const int col = n0 + 16 * j + (lane & 15);
-                if (row < M && col < N) ep(blockIdx.z, row, col, acc[i][j][e]);
-            }
-}
-
-template <bool PIPE = false, class FA, class FB, class EP>
-static void gemm(const char *name, FA fa, FB fb, EP ep, int M, int N, int K, int splits = 1) {
-    if (M <= 0 || N <= 0 || K <= 0) return;
-    int kchunk = ((K + splits - 1) / splits + 31) / 32 * 32;
-    splits = (K + kchunk - 1) / kchunk;
-    LaunchScope scope(name);
-    hipStream_t st = backend().stream;
-    if (N <= 32) {
-        dim3 grid((M + 127) / 128, (N + 31) / 32, splits);
-        hipLaunchKernelGGL((mfma_gemm<4, 1, PIPE, FA, FB, EP>), grid, dim3(256), 0, st, fa, fb, ep, M, N, K,
-                           kchunk);
-    } else if (M <= 32) {
-        dim3 grid((M + 31) / 32, (N + 127) / 128, splits);
-        hipLaunchKernelGGL((mfma_gemm<1, 4, PIPE, FA, FB, EP>), grid, dim3(256), 0, st, fa, fb, ep, M, N, K,
-                           kchunk);
-    } else {
-        dim3 grid((M + 63) / 64, (N + 63) / 64, splits);
-        hipLaunchKernelGGL((mfma_gemm<2, 2, PIPE, FA, FB, EP>), grid, dim3(256), 0, st, fa, fb, ep, M, N, K,
-                           kchunk);
-    }
-    check_launch(name);
-}
-
-// ------------------------------------------------- first layer, forward
-// Layer 0 (2 -> 16 channels, 3^3, stride 1, 64^3). As a GEMM over the padded
-// input it has K = 27 taps x 8 channels = 216, three quarters of it zeros;
-// here K = 27 taps x the 2 used channels = 54, zero-padded to 64 (two MFMA K
-// steps). A workgroup takes four output rows (along x) of one (n, z): it
-// stages the 3 x 6 x 66 input voxels they read -- the 4 bytes of each
-// voxel's two channels, zero outside the volume -- in LDS with coalesced
-// loads, and each wave builds its B fragments from there. The product is
-// taken transposed (weights x patches: D[co][position]), so a lane ends with 4
-// consecutive output channels of one position, stored as one 8-byte word.
-constexpr int kC0Rows = 4;  // output rows (waves) per workgroup
-
-__global__ __launch_bounds__(256) void conv0_forward(const uint16_t *__restrict__ x,
-                                                     const uint16_t *__restrict__ wb,
-                                                     const float *__restrict__ bias,
-                                                     uint16_t *__restrict__ y, int n) {
-    constexpr int E = kEdge, LG = 6, CI = kCin0, CO = 16;
-    constexpr int TY = kC0Rows + 2, TX = E + 2;
-    __shared__ uint32_t tile[3][TY][TX];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int groups = E / kC0Rows;
-    const int y0 = (blockIdx.x % groups) * kC0Rows;
-    const int zz = (blockIdx.x / groups) % E;
-    const int nn = blockIdx.x / (groups * E);
-    for (int i = threadIdx.x; i < 3 * TY * TX; i += 256) {
-        const int tx = i % TX, ty = (i / TX) % TY, tz = i / (TX * TY);
-        const int zi = zz + tz - 1, yi = y0 + ty - 1, xi = tx - 1;
-        uint32_t v = 0;
-        if (nn < n && zi >= 0 && yi >= 0 && xi >= 0 && zi < E && yi < E && xi < E)
-            v = *reinterpret_cast<const uint32_t *>(x + pos_index(nn, zi, yi, xi, LG) * CI);
-        tile[tz][ty][tx] = v;
-    }
-    __syncthreads();
-    if (nn >= n) return;
-    const int yy = y0 + w;
-    const int r = lane & 15, kg = (lane >> 4) * 8;
-    bf16x8 a[2];
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {
-        Frag f;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const int k = 32 * s + kg + j, tap = k >> 1, c = k & 1;
-            f.h[j] = tap < 27 ? wb[(r * 27 + tap) * CI + c] : static_cast<uint16_t>(0);
-        }
-        a[s] = f.v;
-    }
-    f32x4 acc[4];
-#pragma unroll
-    for (int b = 0; b < 4; ++b) {
-        acc[b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-        const int xx = 16 * b + r;
-#pragma unroll
-        for (int s = 0; s < 2; ++s) {
-            Frag f;
-#pragma unroll
-            for (int j4 = 0; j4 < 4; ++j4) {
-                const int tap = 16 * s + (kg >> 1) + j4;
-                uint32_t v = 0;
-                if (tap < 27) {
-                    int kz, ky, kx;
-                    split_tap(tap, kz, ky, kx);
-                    v = tile[kz][w + ky][xx + kx];
-                }
-                f.h[2 * j4] = static_cast<uint16_t>(v & 0xffffu);
-                f.h[2 * j4 + 1] = static_cast<uint16_t>(v >> 16);
-            }
-            acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[s], f.v, acc[b], 0, 0, 0);
-        }
-    }
-    const int co0 = 4 * (lane >> 4);
-#pragma unroll
-    for (int b = 0; b < 4; ++b) {
-        const int xx = 16 * b + r;
-        uint16_t h[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) h[e] = f2bf(fmaxf(acc[b][e] + bias[co0 + e], 0.0f));
-        uint2 word;
-        word.x = static_cast<uint32_t>(h[0]) | (static_cast<uint32_t>(h[1]) << 16);
-        word.y = static_cast<uint32_t>(h[2]) | (static_cast<uint32_t>(h[3]) << 16);
-        *reinterpret_cast<uint2 *>(y + pos_index(nn, zz, yy, xx, LG) * CO + co0) = word;
-    }
-}
-
 // ------------------------------------------------------- small kernels
-// out[i] = sum over `splits` rows of partial[s][i], in split order.
-__global__ void sum_partials(const float *__restrict__ p, int splits, size_t len,
-                             float *__restrict__ out) {
-    for (size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < len;
-         i += static_cast<size_t>(gridDim.x) * blockDim.x) {
-        float s = 0.0f;
-        for (int k = 0; k < splits; ++k) s += p[static_cast<size_t>(k) * len + i];
-        out[i] = s;
-    }
-}
-
-// dy_masked = dy * (y > 0), BF16 in place on dy.
-__global__ void relu_mask(uint16_t *__restrict__ dy, const uint16_t *__restrict__ y, size_t n) {
-    for (size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
-         i += static_cast<size_t>(gridDim.x) * blockDim.x)
-        if (!(bf2f(y[i]) > 0.0f)) dy[i] = 0;
-}
-
-// Bias gradient, first stage: partial[s][c] = sum of dy[m][c] over the
-// positions of split s (workgroup (s), lanes over channels then positions,
-// fixed tree). The second stage is sum_partials over the splits.
-constexpr int kBiasSplits = 256;
-__global__ __launch_bounds__(256) void bias_grad_partials(const uint16_t *__restrict__ dy, int M,
-                                                          int C, float *__restrict__ partial) {
-    __shared__ float red[256];
-    const int s = blockIdx.x;
-    const int per = (M + kBiasSplits - 1) / kBiasSplits;
-    const int m0 = s * per, m1 = min(M, m0 + per);
-    const int lanes_per_c = 256 / C;  // C divides 256 (16..128)
-    const int c = threadIdx.x % C, part = threadIdx.x / C;
-    float acc = 0.0f;
-    for (int m = m0 + part; m < m1; m += lanes_per_c) acc += bf2f(dy[static_cast<size_t>(m) * C + c]);
-    red[threadIdx.x] = acc;
-    __syncthreads();
-    if (threadIdx.x < C) {
-        float t = 0.0f;
-        for (int p = 0; p < lanes_per_c; ++p) t += red[p * C + threadIdx.x];
-        partial[static_cast<size_t>(s) * C + threadIdx.x] = t;
-    }
-}
-
 // Global average pool of the last conv output [n][64][128] -> feat [n][128].
 __global__ void gap_forward(const uint16_t *__restrict__ y, int n, float *__restrict__ feat) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -480,11 +75,13 @@ __global__ void gap_forward(const uint16_t *__restrict__ y, int n, float *__rest
     feat[i] = s * (1.0f / 64.0f);
 }
 
-__global__ void gap_backward(const float *__restrict__ dfeat, int n, uint16_t *__restrict__ dy) {
+// The pool's gradient, masked by the last convolution's ReLU.
+__global__ void gap_backward(const float *__restrict__ dfeat, const uint16_t *__restrict__ y, int n,
+                             uint16_t *__restrict__ dy) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n * 64 * kFeat) return;
     const int c = i % kFeat, b = i / (64 * kFeat);
-    dy[i] = f2bf(dfeat[b * kFeat + c] * (1.0f / 64.0f));
+    dy[i] = bf2f(y[i]) > 0.0f ? f2bf(dfeat[b * kFeat + c] * (1.0f / 64.0f)) : 0;
 }
 
 // MLP head forward, one workgroup (128 lanes) per sample.
@@ -619,8 +216,6 @@ __global__ __launch_bounds__(256) void moments_partials(const float *__restrict_
     }
 }
 
-// One input slot: channel `ch` of [64^3][8] = (v - mean) * inv_std as BF16;
-// channels 2..7 are zero.
 // Each volume's normalisation from its 256 partial (sum, sum of squares)
 // pairs, added in order by one lane (lane t: volume t of nvol): norm[2t..] =
 // {mean, 1 / std} as floats.
@@ -643,9 +238,9 @@ __global__ void moments_finish(const double *__restrict__ part, size_t nv, float
 
 // Slots first .. first + gridDim.y - 1 from their two volumes (fixed, moving:
 // volumes 2b and 2b + 1 of `v`, normalisations 4b .. 4b + 3): voxel i of
-// slot b is {(f - mean_f) / std_f, (m - mean_m) / std_m, 0, ..., 0} as BF16.
+// slot b is {(f - mean_f) / std_f, (m - mean_m) / std_m} as BF16, one word.
 __global__ void pack_slots(const float *__restrict__ v, const float *__restrict__ norm,
-                           uint16_t *__restrict__ slots) {
+                           uint32_t *__restrict__ slots) {
     constexpr int nv = kEdge * kEdge * kEdge;
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= nv) return;
@@ -653,11 +248,8 @@ __global__ void pack_slots(const float *__restrict__ v, const float *__restrict_
     const float *f = v + static_cast<size_t>(2 * b) * nv;
     const float *m = f + nv;
     const float *q = norm + 4 * b;
-    uint16_t *o = slots + (static_cast<size_t>(b) * nv + i) * kCin0;
-    o[0] = f2bf((f[i] - q[0]) * q[1]);
-    o[1] = f2bf((m[i] - q[2]) * q[3]);
-#pragma unroll
-    for (int c = 2; c < kCin0; ++c) o[c] = 0;
+    const uint32_t lo = f2bf((f[i] - q[0]) * q[1]), hi = f2bf((m[i] - q[2]) * q[3]);
+    slots[static_cast<size_t>(b) * nv + i] = lo | (hi << 16);
 }
 
 // --------------------------------------------------------------- the net
@@ -668,9 +260,10 @@ struct Net {
     DeviceBuffer<float> params, grads, adam_m, adam_v;
     long long adam_t = 0;
     DeviceBuffer<uint16_t> wb[kLayers], wt[kLayers];
-    DeviceBuffer<uint16_t> act[kLayers + 1];   // act[0] = input slots, act[l+1] = conv l output
-    DeviceBuffer<uint16_t> dact[kLayers + 1];  // gradients w.r.t. act (masked in place)
-    DeviceBuffer<float> partials;
+    DeviceBuffer<uint16_t> act[kLayers + 1];   // act[0] = input slots (2 channels), act[l+1] = conv l output
+    DeviceBuffer<uint16_t> dact[kLayers + 1];  // gradients w.r.t. act (masked); none for the input
+    DeviceBuffer<float> partials;              // weight-gradient rows of every layer
+    size_t off_partial[kLayers];
     DeviceBuffer<float> feat, hid, out, dout, dhid, dfeat;
     bool weights_dirty = true;
 };
@@ -680,32 +273,24 @@ static int out_edge(int layer) {  // edge of conv `layer`'s output (layer 0..4)
     for (int l = 0; l <= layer; ++l) e /= kStride[l];
     return e;
 }
-static int in_edge(int layer) { return layer == 0 ? kEdge : out_edge(layer - 1); }
-static int lg2(int v) {
-    int l = 0;
-    while ((1 << l) < v) ++l;
-    return l;
-}
-
-static ConvGeom geom_of(int layer, int n) {
-    ConvGeom g;
-    g.n = n;
-    g.ci = kCh[layer];
-    g.co = kCh[layer + 1];
-    g.di = in_edge(layer);
-    g.dout = out_edge(layer);
-    g.stride = kStride[layer];
-    g.lg_ci = lg2(g.ci);
-    g.lg_co = lg2(g.co);
-    g.lg_di = lg2(g.di);
-    g.lg_do = lg2(g.dout);
-    return g;
-}
-
 static size_t act_elems(int idx, int n) {  // idx 0 = input, idx l+1 = conv l output
     const int e = idx == 0 ? kEdge : out_edge(idx - 1);
-    const int c = idx == 0 ? kCin0 : kCh[idx];
+    const int c = idx == 0 ? kCin0Used : kCh[idx];
     return static_cast<size_t>(n) * e * e * e * c;
+}
+
+// A layer's weight-gradient partial rows: enough workgroups to fill the chip
+// without the rows' own traffic (55 KB - 0.9 MB each) growing past the
+// activations', never more than the chunks of positions there are.
+static int wgrad_rows(int layer, int n) {
+    static const int most[kLayers] = {1024, 512, 128, 64, 16};
+    const int chunks[kLayers] = {n * kEdge * kC0PerPlane, InTile<5, 16, 2, 1, 3>::chunks(n),
+                                 InTile<4, 32, 2, 1, 3>::chunks(n), InTile<3, 64, 8, 1, 1>::chunks(n),
+                                 InTile<2, 64, 4, 2, 2>::chunks(n)};
+    return std::min(most[layer], chunks[layer]);
+}
+static int wgrad_row_len(int layer) {
+    return kCh[layer + 1] * 27 * (layer == 0 ? kCin0Used : kCh[layer]) + kCh[layer + 1];
 }
 
 static void init_params(Net &net, uint64_t seed) {
@@ -772,18 +357,15 @@ Net *create(int max_batch, uint64_t seed) {
         }
         for (int i = 0; i <= kLayers; ++i) {
             net->act[i].alloc(act_elems(i, max_batch));
-            net->dact[i].alloc(act_elems(i, max_batch));
+            if (i > 0) net->dact[i].alloc(act_elems(i, max_batch));
         }
         HIP_OK(hipMemsetAsync(net->act[0].ptr, 0, net->act[0].bytes(), backend().stream));
-        // weight-gradient partials: the largest (splits x Cout x 27 Cin)
-        size_t most = 0;
+        size_t partials = 0;
         for (int l = 0; l < kLayers; ++l) {
-            const ConvGeom g = geom_of(l, max_batch);
-            const size_t M = static_cast<size_t>(g.n) << (3 * g.lg_do);
-            const int splits = static_cast<int>(std::min<size_t>(256, std::max<size_t>(1, M / 4096)));
-            most = std::max(most, static_cast<size_t>(splits) * g.co * 27 * g.ci);
+            net->off_partial[l] = partials;
+            partials += static_cast<size_t>(wgrad_rows(l, max_batch)) * wgrad_row_len(l);
         }
-        net->partials.alloc(std::max<size_t>(most, static_cast<size_t>(kBiasSplits) * 128));
+        net->partials.alloc(partials);
         net->feat.alloc(static_cast<size_t>(max_batch) * kFeat);
         net->hid.alloc(static_cast<size_t>(max_batch) * kHidden);
         net->out.alloc(static_cast<size_t>(max_batch) * kOut);
@@ -816,22 +398,77 @@ static void check_batch(const Net &net, int n) {
         fail(SITKHIP_ERR_INVALID_ARGUMENT, "batch must be 1.." + std::to_string(net.max_batch));
 }
 
+static const uint32_t *input_words(const Net &net) {
+    return reinterpret_cast<const uint32_t *>(net.act[0].ptr);
+}
+
+// Workgroups of a launch that walks `items`: `per_cu` on every CU, or one each.
+static unsigned resident(int per_cu, int items) {
+    return static_cast<unsigned>(std::max(1, std::min(items, per_cu * backend().cu_count)));
+}
+
+// A kernel with more than 64 KB of dynamic LDS has to be told so.
+template <typename F>
+static void allow_lds(F kernel, size_t bytes) {
+    if (bytes > 64 * 1024)
+        HIP_OK(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bytes)));
+}
+
+template <int LGDO, int CI, int CO, int R, int COW, bool HOLD>
+static void launch_forward(Net &net, int layer, int n, int per_cu) {
+    using T = InTile<LGDO, CI, R, 1, 3>;
+    auto kernel = conv_forward<LGDO, CI, CO, R, COW, HOLD>;
+    const int chunks = T::chunks(n);
+    allow_lds(kernel, T::kBytes);
+    launch_kernel("cnn_conv_fwd", kernel, dim3(resident(per_cu, chunks), CO / COW), dim3(kConvLanes),
+                  T::kBytes, static_cast<const uint16_t *>(net.act[layer].ptr),
+                  static_cast<const uint16_t *>(net.wb[layer].ptr),
+                  static_cast<const float *>(net.params.ptr + net.off_b[layer]), net.act[layer + 1].ptr,
+                  chunks);
+    check_launch("cnn_conv_fwd");
+}
+
+template <int LGDO, int CI, int CO, int QY, int QZ, int CG>
+static void launch_dgrad(Net &net, int layer, int n) {
+    constexpr int DO = 1 << LGDO;
+    constexpr size_t lds = static_cast<size_t>(QZ + 1) * (QY + 1) * (DO + 1) * (2 * CO + 16);
+    static_assert(lds <= 64 * 1024, "the staged dy fits the default limit");
+    launch_kernel("cnn_conv_dgrad", conv_dgrad<LGDO, CI, CO, QY, QZ, CG>,
+                  dim3(n * (DO / QY) * (DO / QZ), CG), dim3(kConvLanes), lds,
+                  static_cast<const uint16_t *>(net.dact[layer + 1].ptr),
+                  static_cast<const uint16_t *>(net.wt[layer].ptr),
+                  static_cast<const uint16_t *>(net.act[layer].ptr), net.dact[layer].ptr);
+    check_launch("cnn_conv_dgrad");
+}
+
+template <int LGDO, int CI, int CO, int R, int ZP, int KZN, int COW>
+static void launch_wgrad(Net &net, int layer, int n) {
+    using T = InTile<LGDO, CI, R, ZP, KZN * ZP>;
+    constexpr size_t lds = T::kBytes + static_cast<size_t>(T::P) * (2 * COW + 16);
+    static_assert(lds <= 64 * 1024, "the staged chunk fits the default limit");
+    launch_kernel("cnn_conv_wgrad", conv_wgrad<LGDO, CI, CO, R, ZP, KZN, COW>,
+                  dim3(wgrad_rows(layer, n), (3 / KZN) * (CO / COW)), dim3(kConvLanes), lds,
+                  static_cast<const uint16_t *>(net.act[layer].ptr),
+                  static_cast<const uint16_t *>(net.dact[layer + 1].ptr),
+                  net.partials.ptr + net.off_partial[layer], T::chunks(n));
+    check_launch("cnn_conv_wgrad");
+}
+
 void forward(Net &net, int n, float *out_host) {
     check_batch(net, n);
     refresh_weights(net);
     {
-        LaunchScope scope("cnn_conv0_fwd");
-        hipLaunchKernelGGL(conv0_forward, dim3(n * kEdge * (kEdge / kC0Rows)), dim3(256), 0,
-                           backend().stream, net.act[0].ptr, net.wb[0].ptr,
-                           net.params.ptr + net.off_b[0], net.act[1].ptr, n);
+        const int chunks = n * kEdge * kC0PerPlane;
+        launch_kernel("cnn_conv0_fwd", conv0_forward, dim3(resident(8, chunks)), dim3(kConvLanes), 0,
+                      input_words(net), static_cast<const uint16_t *>(net.wb[0].ptr), kCin0,
+                      static_cast<const float *>(net.params.ptr + net.off_b[0]), net.act[1].ptr, chunks);
         check_launch("conv0_forward");
     }
-    for (int l = 1; l < kLayers; ++l) {
-        const ConvGeom g = geom_of(l, n);
-        const int M = g.n << (3 * g.lg_do), N = g.co, K = 27 * g.ci;
-        gemm<true>("cnn_conv_fwd", FwdA{net.act[l].ptr, g}, RowsB{net.wb[l].ptr, g.co, K, K},
-             EpiBiasRelu{net.act[l + 1].ptr, net.params.ptr + net.off_b[l], g.co}, M, N, K);
-    }
+    launch_forward<5, 16, 32, 2, 32, true>(net, 1, n, 3);
+    launch_forward<4, 32, 64, 2, 64, true>(net, 2, n, 2);
+    launch_forward<3, 64, 64, 4, 64, false>(net, 3, n, 2);
+    launch_forward<2, 64, 128, 4, 64, false>(net, 4, n, 4);
     {
         LaunchScope scope("cnn_head");
         hipLaunchKernelGGL(gap_forward, dim3((n * kFeat + 255) / 256), dim3(256), 0, backend().stream,
@@ -862,49 +499,39 @@ void backward(Net &net, int n, const float *dout_host) {
                            net.grads.ptr + net.off_w2, net.grads.ptr + net.off_b2, net.dhid.ptr,
                            net.dfeat.ptr);
         hipLaunchKernelGGL(gap_backward, dim3((n * 64 * kFeat + 255) / 256), dim3(256), 0, st,
-                           net.dfeat.ptr, n, net.dact[kLayers].ptr);
+                           net.dfeat.ptr, net.act[kLayers].ptr, n, net.dact[kLayers].ptr);
         check_launch("cnn_head_bwd");
     }
-    for (int l = kLayers - 1; l >= 0; --l) {
-        const ConvGeom g = geom_of(l, n);
-        const size_t ny = act_elems(l + 1, n);
-        const int M = g.n << (3 * g.lg_do);
-        {
-            LaunchScope scope("cnn_relu_mask");
-            hipLaunchKernelGGL(relu_mask, dim3(grid_for(ny, 256, 8192)), dim3(256), 0, st,
-                               net.dact[l + 1].ptr, net.act[l + 1].ptr, ny);
-            check_launch("cnn_relu_mask");
-        }
-        {
-            LaunchScope scope("cnn_bias_grad");
-            hipLaunchKernelGGL(bias_grad_partials, dim3(kBiasSplits), dim3(256), 0, st,
-                               net.dact[l + 1].ptr, M, g.co, net.partials.ptr);
-            hipLaunchKernelGGL(sum_partials, dim3(1), dim3(256), 0, st, net.partials.ptr, kBiasSplits,
-                               static_cast<size_t>(g.co), net.grads.ptr + net.off_b[l]);
-            check_launch("cnn_bias_grad");
-        }
-        // weight gradient: [co] x [27 ci] over K = M output positions, split
-        const int R = 27 * g.ci;
-        const int splits = static_cast<int>(std::min<long long>(256, std::max<long long>(1, M / 4096)));
-        int kchunk = ((M + splits - 1) / splits + 31) / 32 * 32;
-        const int nsplit = (M + kchunk - 1) / kchunk;
-        gemm("cnn_conv_wgrad", WgradA{net.dact[l + 1].ptr, g}, WgradB{net.act[l].ptr, g},
-             EpiPartial{net.partials.ptr, g.co, R}, g.co, R, M, splits);
-        {
-            LaunchScope scope("cnn_sum_partials");
-            const size_t len = static_cast<size_t>(g.co) * R;
-            hipLaunchKernelGGL(sum_partials, dim3(grid_for(len, 256, 1024)), dim3(256), 0, st,
-                               net.partials.ptr, nsplit, len, net.grads.ptr + net.off_w[l]);
-            check_launch("sum_partials");
-        }
-        if (l > 0) {
-            // input gradient: M' = input positions, N' = ci, K' = 27 co
-            const int Mi = g.n << (3 * g.lg_di);
-            const int Kd = 27 * g.co;
-            gemm("cnn_conv_dgrad", DgradA{net.dact[l + 1].ptr, g}, RowsB{net.wt[l].ptr, g.ci, Kd, Kd},
-                 EpiStoreBf16{net.dact[l].ptr, g.ci}, Mi, g.ci, Kd);
-        }
+    launch_wgrad<2, 64, 128, 4, 2, 1, 64>(net, 4, n);
+    launch_dgrad<2, 64, 128, 4, 4, 4>(net, 4, n);
+    launch_wgrad<3, 64, 64, 8, 1, 1, 64>(net, 3, n);
+    launch_dgrad<3, 64, 64, 8, 1, 4>(net, 3, n);
+    launch_wgrad<4, 32, 64, 2, 1, 3, 32>(net, 2, n);
+    launch_dgrad<4, 32, 64, 8, 1, 1>(net, 2, n);
+    launch_wgrad<5, 16, 32, 2, 1, 3, 32>(net, 1, n);
+    launch_dgrad<5, 16, 32, 4, 1, 1>(net, 1, n);
+    launch_kernel("cnn_conv_wgrad", conv0_wgrad, dim3(wgrad_rows(0, n)), dim3(kConvLanes), 0,
+                  input_words(net), static_cast<const uint16_t *>(net.dact[1].ptr),
+                  net.partials.ptr + net.off_partial[0], n * kEdge * kC0PerPlane);
+    check_launch("conv0_wgrad");
+    PartialJobs jobs;
+    jobs.n = kLayers;
+    unsigned blocks = 0;
+    for (int l = 0; l < kLayers; ++l) {
+        PartialRows &q = jobs.j[l];
+        q.p = net.partials.ptr + net.off_partial[l];
+        q.out = net.grads.ptr + net.off_w[l];
+        q.out_bias = net.grads.ptr + net.off_b[l];
+        q.rows = wgrad_rows(l, n);
+        q.total = wgrad_row_len(l);
+        q.len = q.total - kCh[l + 1];
+        q.inner = l == 0 ? kCin0Used : q.len;
+        q.ld = l == 0 ? kCin0 : q.len;
+        q.first_block = blocks;
+        blocks += static_cast<unsigned>((q.total + 63) / 64);
     }
+    launch_kernel("cnn_sum_partials", reduce_partials, dim3(blocks), dim3(kConvLanes), 0, jobs);
+    check_launch("reduce_partials");
     sync();
 }
 
@@ -929,7 +556,7 @@ static void pack(Net &net, int first, int n, const float *vols) {
     if (first < 0 || n < 1 || first + n > net.max_batch)
         fail(SITKHIP_ERR_INVALID_ARGUMENT, "slot out of range");
     const size_t nv = static_cast<size_t>(kEdge) * kEdge * kEdge;
-    uint16_t *dst = net.act[0].ptr + static_cast<size_t>(first) * nv * kCin0;
+    uint32_t *dst = reinterpret_cast<uint32_t *>(net.act[0].ptr) + static_cast<size_t>(first) * nv;
     DeviceBuffer<double> part(static_cast<size_t>(2 * n) * 2 * 256);
     DeviceBuffer<float> norm(static_cast<size_t>(2 * n) * 2);
     hipLaunchKernelGGL(moments_partials, dim3(256, static_cast<unsigned>(2 * n)), dim3(256), 0,
@@ -1123,12 +750,23 @@ int sitkhip_cnn_activation(sitkhip_cnn h, int index, int gradient, int batch, fl
         cnn::Net &net = net_ref(h);
         if (index < 0 || index > cnn::kLayers) fail(SITKHIP_ERR_INVALID_ARGUMENT, "bad index");
         cnn::check_batch(net, batch);
-        const size_t len = cnn::act_elems(index, batch);
+        const size_t held = cnn::act_elems(index, batch);
+        const size_t len = index == 0 ? held / cnn::kCin0Used * cnn::kCin0 : held;
         if (!out || n != len) fail(SITKHIP_ERR_INVALID_ARGUMENT, "length mismatch");
-        std::vector<uint16_t> hb(len);
-        (gradient ? net.dact[index] : net.act[index]).download(hb.data(), len);
-        sync();
-        for (size_t i = 0; i < len; ++i) out[i] = cnn::bf2f(hb[i]);
+        std::vector<uint16_t> hb(held, 0);
+        if (!(index == 0 && gradient)) {  // (the input's gradient is not computed: zeros)
+            (gradient ? net.dact[index] : net.act[index]).download(hb.data(), held);
+            sync();
+        }
+        if (index > 0) {
+            for (size_t i = 0; i < len; ++i) out[i] = cnn::bf2f(hb[i]);
+            return;
+        }
+        for (size_t i = 0; i < len; ++i) {  // the unused channels read zero
+            const size_t v = i / cnn::kCin0, c = i % cnn::kCin0;
+            out[i] = c < static_cast<size_t>(cnn::kCin0Used)
+                         ? cnn::bf2f(hb[v * cnn::kCin0Used + c]) : 0.0f;
+        }
     });
 }
 
