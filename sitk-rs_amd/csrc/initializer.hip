@@ -185,71 +185,80 @@ __global__ void cast_weights(const float *__restrict__ w, int co, int ci, uint16
     }
 }
 
-// Sum and sum of squares of a volume (FP64 partials per workgroup); volume
-// blockIdx.y of consecutive volumes of n voxels, its partials 2 * gridDim.x
-// apart.
-__global__ __launch_bounds__(256) void moments_partials(const float *__restrict__ v, size_t n,
-                                                        double *__restrict__ out) {
-    __shared__ double s1[256], s2[256];
-    v += static_cast<size_t>(blockIdx.y) * n;
-    out += static_cast<size_t>(blockIdx.y) * 2 * gridDim.x;
-    double a = 0.0, b = 0.0;
-    for (size_t i = static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x; i < n;
-         i += static_cast<size_t>(gridDim.x) * 256) {
-        const double x = v[i];
-        a += x;
-        b += x * x;
-    }
-    s1[threadIdx.x] = a;
-    s2[threadIdx.x] = b;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if (threadIdx.x < w) {
-            s1[threadIdx.x] += s1[threadIdx.x + w];
-            s2[threadIdx.x] += s2[threadIdx.x + w];
-        }
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        out[2 * blockIdx.x] = s1[0];
-        out[2 * blockIdx.x + 1] = s2[0];
-    }
+// The 64^3 input volumes are read four voxels per lane.
+constexpr int kVol = kEdge * kEdge * kEdge;
+constexpr int kVolBlocks = kVol / (256 * 4);
+
+// Sums over the 64 lanes of a wave in a fixed order, in every lane.
+__device__ __forceinline__ double wave_sum(double v) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    return v;
 }
 
-// Each volume's normalisation from its 256 partial (sum, sum of squares)
-// pairs, added in order by one lane (lane t: volume t of nvol): norm[2t..] =
-// {mean, 1 / std} as floats.
-__global__ void moments_finish(const double *__restrict__ part, size_t nv, float *__restrict__ norm,
-                               int nvol) {
-    const int t = static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x);
-    if (t >= nvol) return;
-    part += static_cast<size_t>(t) * 512;
-    norm += 2 * t;
+// Sum and sum of squares of 1,024 voxels of volume blockIdx.y (FP64):
+// part[(volume * kVolBlocks + block) * 2 ..].
+__global__ __launch_bounds__(256) void moments_partials(const float *__restrict__ v,
+                                                        double *__restrict__ part) {
+    __shared__ double s[4][2];
+    const float4 q = reinterpret_cast<const float4 *>(
+        v + static_cast<size_t>(blockIdx.y) * kVol)[blockIdx.x * 256 + threadIdx.x];
+    const double x[4] = {q.x, q.y, q.z, q.w};
+    double a = 0.0, b = 0.0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        a += x[k];
+        b += x[k] * x[k];
+    }
+    a = wave_sum(a);
+    b = wave_sum(b);
+    if ((threadIdx.x & 63) == 0) {
+        s[threadIdx.x >> 6][0] = a;
+        s[threadIdx.x >> 6][1] = b;
+    }
+    __syncthreads();
+    if (threadIdx.x < 2)
+        part[(static_cast<size_t>(blockIdx.y) * kVolBlocks + blockIdx.x) * 2 + threadIdx.x] =
+            (s[0][threadIdx.x] + s[1][threadIdx.x]) + (s[2][threadIdx.x] + s[3][threadIdx.x]);
+}
+
+// Volume blockIdx.x's normalisation from its partial sums (one wave, a fixed
+// order): norm[2 b ..] = {mean, 1 / std} as floats.
+__global__ __launch_bounds__(64) void moments_finish(const double *__restrict__ part,
+                                                     float *__restrict__ norm) {
+    part += static_cast<size_t>(blockIdx.x) * kVolBlocks * 2;
     double s1 = 0.0, s2 = 0.0;
-    for (int b = 0; b < 256; ++b) {
+#pragma unroll
+    for (int b = threadIdx.x; b < kVolBlocks; b += 64) {
         s1 += part[2 * b];
         s2 += part[2 * b + 1];
     }
-    const double mean = s1 / static_cast<double>(nv);
-    const double var = fmax(s2 / static_cast<double>(nv) - mean * mean, 1e-12);
-    norm[0] = static_cast<float>(mean);
-    norm[1] = static_cast<float>(1.0 / sqrt(var));
+    s1 = wave_sum(s1);
+    s2 = wave_sum(s2);
+    if (threadIdx.x == 0) {
+        const double mean = s1 / kVol;
+        const double var = fmax(s2 / kVol - mean * mean, 1e-12);
+        norm[2 * blockIdx.x] = static_cast<float>(mean);
+        norm[2 * blockIdx.x + 1] = static_cast<float>(1.0 / sqrt(var));
+    }
 }
 
 // Slots first .. first + gridDim.y - 1 from their two volumes (fixed, moving:
 // volumes 2b and 2b + 1 of `v`, normalisations 4b .. 4b + 3): voxel i of
 // slot b is {(f - mean_f) / std_f, (m - mean_m) / std_m} as BF16, one word.
-__global__ void pack_slots(const float *__restrict__ v, const float *__restrict__ norm,
-                           uint32_t *__restrict__ slots) {
-    constexpr int nv = kEdge * kEdge * kEdge;
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nv) return;
-    const int b = blockIdx.y;
-    const float *f = v + static_cast<size_t>(2 * b) * nv;
-    const float *m = f + nv;
+__global__ __launch_bounds__(256) void pack_slots(const float *__restrict__ v,
+                                                  const float *__restrict__ norm,
+                                                  uint32_t *__restrict__ slots) {
+    const int b = blockIdx.y, i = blockIdx.x * 256 + threadIdx.x;
+    const float4 *src = reinterpret_cast<const float4 *>(v + static_cast<size_t>(2 * b) * kVol);
+    const float4 f = src[i], m = src[i + kVol / 4];
     const float *q = norm + 4 * b;
-    const uint32_t lo = f2bf((f[i] - q[0]) * q[1]), hi = f2bf((m[i] - q[2]) * q[3]);
-    slots[static_cast<size_t>(b) * nv + i] = lo | (hi << 16);
+    auto word = [&](float x, float y) {
+        return static_cast<uint32_t>(f2bf((x - q[0]) * q[1])) |
+               (static_cast<uint32_t>(f2bf((y - q[2]) * q[3])) << 16);
+    };
+    reinterpret_cast<uint4 *>(slots + static_cast<size_t>(b) * kVol)[i] =
+        make_uint4(word(f.x, m.x), word(f.y, m.y), word(f.z, m.z), word(f.w, m.w));
 }
 
 // --------------------------------------------------------------- the net
@@ -555,18 +564,17 @@ void adam(Net &net, float lr, float b1, float b2, float eps) {
 static void pack(Net &net, int first, int n, const float *vols) {
     if (first < 0 || n < 1 || first + n > net.max_batch)
         fail(SITKHIP_ERR_INVALID_ARGUMENT, "slot out of range");
-    const size_t nv = static_cast<size_t>(kEdge) * kEdge * kEdge;
-    uint32_t *dst = reinterpret_cast<uint32_t *>(net.act[0].ptr) + static_cast<size_t>(first) * nv;
-    DeviceBuffer<double> part(static_cast<size_t>(2 * n) * 2 * 256);
-    DeviceBuffer<float> norm(static_cast<size_t>(2 * n) * 2);
-    hipLaunchKernelGGL(moments_partials, dim3(256, static_cast<unsigned>(2 * n)), dim3(256), 0,
-                       backend().stream, vols, nv, part.ptr);
+    uint32_t *dst = reinterpret_cast<uint32_t *>(net.act[0].ptr) + static_cast<size_t>(first) * kVol;
+    const unsigned nv = static_cast<unsigned>(2 * n);
+    DeviceBuffer<double> part(static_cast<size_t>(nv) * kVolBlocks * 2);
+    DeviceBuffer<float> norm(static_cast<size_t>(nv) * 2);
+    launch_kernel("cnn_moments", moments_partials, dim3(kVolBlocks, nv), dim3(256), 0, vols, part.ptr);
     check_launch("moments_partials");
-    hipLaunchKernelGGL(moments_finish, dim3(static_cast<unsigned>((2 * n + 63) / 64)), dim3(64), 0,
-                       backend().stream, part.ptr, nv, norm.ptr, 2 * n);
+    launch_kernel("cnn_moments", moments_finish, dim3(nv), dim3(64), 0,
+                  static_cast<const double *>(part.ptr), norm.ptr);
     check_launch("moments_finish");
-    hipLaunchKernelGGL(pack_slots, dim3(static_cast<unsigned>((nv + 255) / 256), static_cast<unsigned>(n)),
-                       dim3(256), 0, backend().stream, vols, norm.ptr, dst);
+    launch_kernel("cnn_pack", pack_slots, dim3(kVolBlocks, static_cast<unsigned>(n)), dim3(256), 0, vols,
+                  static_cast<const float *>(norm.ptr), dst);
     check_launch("pack_slots");
 }
 
