@@ -29,6 +29,7 @@ namespace cnn {
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 typedef short i16x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));  // a staged 16-byte piece
 
 union Frag {
     uint4 u;
@@ -109,25 +110,25 @@ struct InTile {
                 make_uint4(0, 0, 0, 0);
     }
     __device__ static void load(const uint16_t *__restrict__ x, int n, int first_z, int step_z,
-                                int y0, uint4 (&v)[kPer]) {
+                                int y0, u32x4 (&v)[kPer]) {
 #pragma unroll
         for (int k = 0; k < kPer; ++k) {
             const int i = threadIdx.x + k * kConvLanes;
             const int c8 = i % (CI / 8), xi = i / (CI / 8) % DI, q = i / (CI / 8 * DI);
             const int zi = first_z + (q / ROWS) * step_z, yi = 2 * y0 - 1 + q % ROWS;
-            v[k] = make_uint4(0, 0, 0, 0);
+            v[k] = u32x4{0, 0, 0, 0};
             if (i < kPieces && zi >= 0 && yi >= 0)
-                v[k] = *reinterpret_cast<const uint4 *>(
+                v[k] = *reinterpret_cast<const u32x4 *>(
                     x + (((static_cast<size_t>(n) * DI + zi) * DI + yi) * DI + xi) * CI + c8 * 8);
         }
     }
-    __device__ static void store(char *lds, const uint4 (&v)[kPer]) {
+    __device__ static void store(char *lds, const u32x4 (&v)[kPer]) {
 #pragma unroll
         for (int k = 0; k < kPer; ++k) {
             const int i = threadIdx.x + k * kConvLanes;
             const int c8 = i % (CI / 8), xi = i / (CI / 8) % DI, q = i / (CI / 8 * DI);
             if (i < kPieces)
-                *reinterpret_cast<uint4 *>(lds + (q * COLS + xi + 1) * VS + c8 * 16) = v[k];
+                *reinterpret_cast<u32x4 *>(lds + (q * COLS + xi + 1) * VS + c8 * 16) = v[k];
         }
     }
     // Byte offset of output position p's first tap (kz = ky = kx = 0); `zs`
@@ -151,7 +152,7 @@ struct InTile {
 // Bound by its traffic in layer 1 (268 MB in, 67 MB out for 32 pairs: 4.6 TB/s)
 // and by latency in layers 3-4 (few positions). Gathering the operands from
 // global memory, with every lane's voxel address worked out per K step, took
-// 203 us for layer 1 and 168 us for layers 2-4 of 32 pairs; this takes 73 and 58.
+// 203 us for layer 1 and 168 us for layers 2-4 of 32 pairs; this takes 74 and 61.
 template <int LGDO, int CI, int CO, int R, int COW, bool HOLD>
 __global__ __launch_bounds__(kConvLanes) void conv_forward(const uint16_t *__restrict__ x,
                                                            const uint16_t *__restrict__ wb,
@@ -183,7 +184,7 @@ __global__ __launch_bounds__(kConvLanes) void conv_forward(const uint16_t *__res
     for (int p = 0; p < PT; ++p)
         base[p] = T::at((pt0 + p) * 16 + r16, 2) + (CI == 16 ? 16 * (g & 1) : 16 * g);
     T::clear_edge(lds);
-    uint4 v[T::kPer];
+    u32x4 v[T::kPer];
     int c = blockIdx.x, n, z0, y0;
     if (c < nchunks) {
         T::chunk(c, n, z0, y0);
@@ -195,7 +196,7 @@ __global__ __launch_bounds__(kConvLanes) void conv_forward(const uint16_t *__res
         T::store(lds, v);
         __syncthreads();
         const int cn = c + gridDim.x;
-        if (cn < nchunks) {
+        if (HOLD && cn < nchunks) {
             int n2, z2, y2;
             T::chunk(cn, n2, z2, y2);
             T::load(x, n2, 2 * z2 - 1, 1, y2, v);
@@ -242,6 +243,7 @@ __global__ __launch_bounds__(kConvLanes) void conv_forward(const uint16_t *__res
                 *reinterpret_cast<uint2 *>(y + (pos0 + (pt0 + p) * 16 + r16) * CO + co) = pack_bf16(o);
             }
         }
+        if (!HOLD) break;  // one chunk per workgroup: nothing to carry over
     }
 }
 
@@ -253,10 +255,10 @@ __global__ __launch_bounds__(kConvLanes) void conv_forward(const uint16_t *__res
 // [CO][27 CI], [CO]; reduce_partials adds the rows in a fixed tree.
 // Gathering each operand's eight positions from global memory one scalar at a
 // time, with bias sums and masks in passes of their own, took 5.6 ms for the
-// five layers of 24 pairs and 1.3 ms for those passes; this takes 0.21 ms and
-// the fold of the partial rows 0.025.
+// five layers of 24 pairs and 1.3 ms for those passes; the five layers now take
+// 0.18 ms and the fold of the partial rows 0.025.
 template <int LGDO, int CI, int CO, int R, int ZP, int KZN, int COW>
-__global__ __launch_bounds__(kConvLanes) void conv_wgrad(const uint16_t *__restrict__ x,
+__global__ __launch_bounds__(kConvLanes, CI <= 32 ? 2 : 1) void conv_wgrad(const uint16_t *__restrict__ x,
                                                          const uint16_t *__restrict__ dy,
                                                          float *__restrict__ partial, int nchunks) {
     using T = InTile<LGDO, CI, R, ZP, KZN * ZP>;
@@ -295,7 +297,7 @@ __global__ __launch_bounds__(kConvLanes) void conv_wgrad(const uint16_t *__restr
     for (int e = 0; e < 8; ++e) ones.h[e] = 0x3f80;
 
     T::clear_edge(lds);
-    uint4 v[T::kPer], d[DYN];
+    u32x4 v[T::kPer], d[DYN];
     auto fetch = [&](int c) {
         int n, z0, y0;
         T::chunk(c, n, z0, y0);
@@ -305,7 +307,7 @@ __global__ __launch_bounds__(kConvLanes) void conv_wgrad(const uint16_t *__restr
         for (int k = 0; k < DYN; ++k) {
             const int i = threadIdx.x + k * kConvLanes;
             if (i < DYP)
-                d[k] = *reinterpret_cast<const uint4 *>(dy + (pos0 + i / (COW / 8)) * CO + co0 +
+                d[k] = *reinterpret_cast<const u32x4 *>(dy + (pos0 + i / (COW / 8)) * CO + co0 +
                                                         (i % (COW / 8)) * 8);
         }
     };
@@ -318,7 +320,7 @@ __global__ __launch_bounds__(kConvLanes) void conv_wgrad(const uint16_t *__restr
         for (int k = 0; k < DYN; ++k) {
             const int i = threadIdx.x + k * kConvLanes;
             if (i < DYP)
-                *reinterpret_cast<uint4 *>(sdy + (i / (COW / 8)) * DS + (i % (COW / 8)) * 16) = d[k];
+                *reinterpret_cast<u32x4 *>(sdy + (i / (COW / 8)) * DS + (i % (COW / 8)) * 16) = d[k];
         }
         __syncthreads();
         if (c + static_cast<int>(gridDim.x) < nchunks) fetch(c + gridDim.x);
@@ -368,127 +370,173 @@ __global__ __launch_bounds__(kConvLanes) void conv_wgrad(const uint16_t *__restr
 // CG > 1: the parity classes are spread over blockIdx.y (layers with few
 // positions). One product over every position took 495 us a layer for layers
 // 1-2 of 24 pairs and 78 for layers 3-4, its masks 0.18 ms more; this takes
-// 157 / 54 and 17 / 17.
-template <int LGDO, int CI, int CO, int QY, int QZ, int CG>
-__global__ __launch_bounds__(kConvLanes) void conv_dgrad(const uint16_t *__restrict__ dy,
+// 90 / 53 and 14 / 13.
+// HOLD: the wave's 27 weight operands stay in registers and the workgroup
+// walks many tiles (layer 1: 157 us with a weight load ahead of each product,
+// 91 held: 452 MB, 5.0 TB/s); layers 2-4, whose operands do not fit, read them
+// from L2 (loading a class's together spilled: layer 2 took 79 us).
+template <int LGDO, int CI, int CO, int QY, int QZ, int CG, bool HOLD>
+__global__ __launch_bounds__(kConvLanes, 2) void conv_dgrad(const uint16_t *__restrict__ dy,
                                                          const uint16_t *__restrict__ wt,
                                                          const uint16_t *__restrict__ act,
-                                                         uint16_t *__restrict__ dx) {
-    constexpr int DO = 1 << LGDO, DI = 2 * DO, DS = 2 * CO + 16;
+                                                         uint16_t *__restrict__ dx, int ntiles) {
+    constexpr int DO = 1 << LGDO, DI = 2 * DO, DS = 2 * CO + 16, KS = CO / 32;
     constexpr int Y1 = QY + 1, Z1 = QZ + 1, X1 = DO + 1;
     constexpr int P = QZ * QY * DO, WR = CI / 16 < 4 ? CI / 16 : 4, WP = 4 / WR, PT = P / 16 / WP;
     static_assert(CI / 16 == WR && PT >= 1, "one row tile per wave");
+    constexpr int kPieces = Z1 * Y1 * X1 * (CO / 8), kPer = (kPieces + kConvLanes - 1) / kConvLanes;
     extern __shared__ char lds[];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int r16 = lane & 15, g = lane >> 4;
-    const int y0 = (blockIdx.x % (DO / QY)) * QY, z0 = (blockIdx.x / (DO / QY)) % (DO / QZ) * QZ;
-    const size_t n = blockIdx.x / ((DO / QY) * (DO / QZ));
-    constexpr int kPieces = Z1 * Y1 * X1 * (CO / 8);
-#pragma unroll 4
-    for (int i = threadIdx.x; i < kPieces; i += kConvLanes) {
-        const int c8 = i % (CO / 8), xo = i / (CO / 8) % X1, q = i / (CO / 8 * X1);
-        const int yo = y0 + q % Y1, zo = z0 + q / Y1;
-        uint4 v = make_uint4(0, 0, 0, 0);
-        if (xo < DO && yo < DO && zo < DO)
-            v = *reinterpret_cast<const uint4 *>(dy + (((n * DO + zo) * DO + yo) * DO + xo) * CO + c8 * 8);
-        *reinterpret_cast<uint4 *>(lds + (q * X1 + xo) * DS + c8 * 16) = v;
-    }
-    __syncthreads();
     const int ci0 = (w % WR) * 16;
-    int base[PT], zi[PT], yi[PT], xi[PT];
+    int base[PT], inside[PT];  // LDS bytes of the tile's position q; element offset of 2 q in dx
 #pragma unroll
     for (int t = 0; t < PT; ++t) {
         const int p = ((w / WR) * PT + t) * 16 + r16;
         const int qx = p % DO, qy = p / DO % QY, qz = p / (DO * QY);
         base[t] = ((qz * Y1 + qy) * X1 + qx) * DS + 16 * g;
-        zi[t] = 2 * (z0 + qz);
-        yi[t] = 2 * (y0 + qy);
-        xi[t] = 2 * qx;
+        inside[t] = ((2 * qz * DI + 2 * qy) * DI + 2 * qx) * CI + ci0 + 4 * g;
     }
+    const uint16_t *wrow = wt + static_cast<size_t>(ci0 + r16) * 27 * CO + 8 * g;
+    bf16x8 held[HOLD ? 27 * KS : 1];
+    if (HOLD) {
+#pragma unroll
+        for (int i = 0; i < 27 * KS; ++i) held[i] = load_frag(wrow + 32 * i);
+    }
+    auto origin = [&](int tile, size_t &n, int &z0, int &y0) {
+        y0 = (tile % (DO / QY)) * QY;
+        z0 = tile / (DO / QY) % (DO / QZ) * QZ;
+        n = tile / ((DO / QY) * (DO / QZ));
+    };
+    u32x4 v[kPer];
+    auto fetch = [&](int tile) {
+        size_t n;
+        int z0, y0;
+        origin(tile, n, z0, y0);
+#pragma unroll
+        for (int k = 0; k < kPer; ++k) {
+            const int i = threadIdx.x + k * kConvLanes;
+            const int c8 = i % (CO / 8), xo = i / (CO / 8) % X1, q = i / (CO / 8 * X1);
+            const int yo = y0 + q % Y1, zo = z0 + q / Y1;
+            v[k] = u32x4{0, 0, 0, 0};
+            if (i < kPieces && xo < DO && yo < DO && zo < DO)
+                v[k] = *reinterpret_cast<const u32x4 *>(dy + (((n * DO + zo) * DO + yo) * DO + xo) * CO +
+                                                        c8 * 8);
+        }
+    };
     // eight classes with 8, (4 2 1), (4 2), (4 2) taps per group
     const unsigned group = CG == 1 ? 0xffu : (0x50240b80u >> (8 * blockIdx.y)) & 0xffu;
-    const uint16_t *wrow = wt + static_cast<size_t>(ci0 + r16) * 27 * CO + 8 * g;
-    for (int cls = 0; cls < 8; ++cls) {
-        if (!((group >> cls) & 1u)) continue;
-        const int pz = cls >> 2, py = (cls >> 1) & 1, px = cls & 1;
-        f32x4 acc[PT];
+    int tile = blockIdx.x;
+    if (tile < ntiles) fetch(tile);
+    for (; tile < ntiles; tile += gridDim.x) {
+        __syncthreads();
 #pragma unroll
-        for (int t = 0; t < PT; ++t) acc[t] = zero_acc();
-        for (int tz = 0; tz <= pz; ++tz)
-            for (int ty = 0; ty <= py; ++ty)
-                for (int tx = 0; tx <= px; ++tx) {
-                    // parity 1: first k = 0 at q + 1, then k = 2 at q
-                    const int kz = pz ? 2 * tz : 1, ky = py ? 2 * ty : 1, kx = px ? 2 * tx : 1;
-                    const int off = (((pz - tz) * Y1 + (py - ty)) * X1 + (px - tx)) * DS;
-                    const uint16_t *wk = wrow + (kz * 9 + ky * 3 + kx) * CO;
-#pragma unroll
-                    for (int s = 0; s < CO / 32; ++s) {
-                        const bf16x8 a = load_frag(wk + 32 * s);
-#pragma unroll
-                        for (int t = 0; t < PT; ++t)
-                            acc[t] = mfma(a, load_frag(lds + base[t] + off + 64 * s), acc[t]);
-                    }
-                }
-#pragma unroll
-        for (int t = 0; t < PT; ++t) {
-            const size_t at =
-                (((n * DI + zi[t] + pz) * DI + yi[t] + py) * DI + xi[t] + px) * CI + ci0 + 4 * g;
-            const uint2 y = *reinterpret_cast<const uint2 *>(act + at);
-            float o[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) o[e] = bf16_at(y, e) > 0.0f ? acc[t][e] : 0.0f;
-            *reinterpret_cast<uint2 *>(dx + at) = pack_bf16(o);
+        for (int k = 0; k < kPer; ++k) {
+            const int i = threadIdx.x + k * kConvLanes;
+            if (i < kPieces)
+                *reinterpret_cast<u32x4 *>(lds + i / (CO / 8) * DS + i % (CO / 8) * 16) = v[k];
         }
+        __syncthreads();
+        if (HOLD && tile + static_cast<int>(gridDim.x) < ntiles) fetch(tile + gridDim.x);
+        size_t n;
+        int z0, y0;
+        origin(tile, n, z0, y0);
+        const size_t corner = (((n * DI + 2 * z0) * DI + 2 * y0) * DI) * CI;
+#pragma unroll
+        for (int cls = 0; cls < 8; ++cls) {
+            if (!((group >> cls) & 1u)) continue;
+            const int pz = cls >> 2, py = (cls >> 1) & 1, px = cls & 1;
+            const size_t at = corner + static_cast<size_t>((pz * DI + py) * DI + px) * CI;
+            f32x4 acc[PT];
+            uint2 y[PT];
+#pragma unroll
+            for (int t = 0; t < PT; ++t) {
+                acc[t] = zero_acc();
+                y[t] = *reinterpret_cast<const uint2 *>(act + at + inside[t]);
+            }
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                const int tz = k >> 2, ty = (k >> 1) & 1, tx = k & 1;
+                if (tz > pz || ty > py || tx > px) continue;
+                // parity 1: first k = 0 at q + 1, then k = 2 at q
+                const int tap = (pz ? 2 * tz : 1) * 9 + (py ? 2 * ty : 1) * 3 + (px ? 2 * tx : 1);
+                const int off = (((pz - tz) * Y1 + (py - ty)) * X1 + (px - tx)) * DS;
+#pragma unroll
+                for (int s = 0; s < KS; ++s) {
+                    const bf16x8 a = HOLD ? held[tap * KS + s] : load_frag(wrow + tap * CO + 32 * s);
+#pragma unroll
+                    for (int t = 0; t < PT; ++t)
+                        acc[t] = mfma(a, load_frag(lds + base[t] + off + 64 * s), acc[t]);
+                }
+            }
+#pragma unroll
+            for (int t = 0; t < PT; ++t) {
+                float o[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) o[e] = bf16_at(y[t], e) > 0.0f ? acc[t][e] : 0.0f;
+                *reinterpret_cast<uint2 *>(dx + at + inside[t]) = pack_bf16(o);
+            }
+        }
+        if (!HOLD) break;  // one tile per workgroup: nothing to carry over
     }
 }
 
 // ----------------------------------------------------------- first layer
 // 2 -> 16 channels, stride 1, 64^3. A voxel's two channels are one 4-byte
-// word. A chunk is four output rows (one per wave) of one plane; it reads
-// 3 planes x 6 rows x voxels -2 .. 65, zero outside the volume.
-constexpr int kC0Rows = 4, kC0Cols = 68;
-constexpr int kC0Vox = 3 * (kC0Rows + 2) * kC0Cols;
-constexpr int kC0Per = (kC0Vox + kConvLanes - 1) / kConvLanes;
-constexpr int kC0PerPlane = 64 / kC0Rows;
+// word. A chunk is ROWS output rows (ROWS / 4 per wave) of one plane; it reads
+// 3 planes x (ROWS + 2) rows x voxels -2 .. 65, zero outside the volume.
+template <int ROWS>
+struct C0Tile {
+    static constexpr int COLS = 68, kVox = 3 * (ROWS + 2) * COLS, WAVE_ROWS = ROWS / 4;
+    static constexpr int kPer = (kVox + kConvLanes - 1) / kConvLanes;
 
-__device__ __forceinline__ void c0_chunk(int c, size_t &n, int &z, int &y0) {
-    y0 = (c % kC0PerPlane) * kC0Rows;
-    z = (c / kC0PerPlane) & 63;
-    n = static_cast<size_t>(c / kC0PerPlane) >> 6;
-}
-__device__ __forceinline__ void c0_load(const uint32_t *__restrict__ x, int c, uint32_t (&v)[kC0Per]) {
-    size_t n;
-    int z, y0;
-    c0_chunk(c, n, z, y0);
-#pragma unroll
-    for (int k = 0; k < kC0Per; ++k) {
-        const int i = threadIdx.x + k * kConvLanes;
-        const int xi = i % kC0Cols - 2, row = i / kC0Cols;
-        const int yi = y0 + row % (kC0Rows + 2) - 1, zi = z + row / (kC0Rows + 2) - 1;
-        v[k] = 0;
-        if (i < kC0Vox && (xi | yi | zi) >= 0 && xi < 64 && yi < 64 && zi < 64)
-            v[k] = x[((n * 64 + zi) * 64 + yi) * 64 + xi];
+    static int chunks(int n) { return n * 64 * (64 / ROWS); }
+    __device__ static void chunk(int c, size_t &n, int &z, int &y0) {
+        y0 = (c % (64 / ROWS)) * ROWS;
+        z = (c / (64 / ROWS)) & 63;
+        n = static_cast<size_t>(c / (64 / ROWS)) >> 6;
     }
-}
-__device__ __forceinline__ void c0_store(char *lds, const uint32_t (&v)[kC0Per]) {
+    __device__ static void load(const uint32_t *__restrict__ x, int c, uint32_t (&v)[kPer]) {
+        size_t n;
+        int z, y0;
+        chunk(c, n, z, y0);
 #pragma unroll
-    for (int k = 0; k < kC0Per; ++k) {
-        const int i = threadIdx.x + k * kConvLanes;
-        if (i < kC0Vox) *reinterpret_cast<uint32_t *>(lds + 4 * i) = v[k];
+        for (int k = 0; k < kPer; ++k) {
+            const int i = threadIdx.x + k * kConvLanes;
+            const int xi = i % COLS - 2, row = i / COLS;
+            const int yi = y0 + row % (ROWS + 2) - 1, zi = z + row / (ROWS + 2) - 1;
+            v[k] = 0;
+            if (i < kVox && (xi | yi | zi) >= 0 && xi < 64 && yi < 64 && zi < 64)
+                v[k] = x[((n * 64 + zi) * 64 + yi) * 64 + xi];
+        }
     }
-}
+    __device__ static void store(char *lds, const uint32_t (&v)[kPer]) {
+#pragma unroll
+        for (int k = 0; k < kPer; ++k) {
+            const int i = threadIdx.x + k * kConvLanes;
+            if (i < kVox) *reinterpret_cast<uint32_t *>(lds + 4 * i) = v[k];
+        }
+    }
+    // byte of voxel x - 2 of the row that tap (kz, ky) of this wave's first
+    // output row reads
+    __device__ static int row(int kz, int ky, int wave) {
+        return (kz * (ROWS + 2) + wave * WAVE_ROWS + ky) * COLS * 4;
+    }
+};
 
 // Forward: K = 27 taps x 2 channels = 54, zero-padded to two MFMA steps; an
 // operand's eight K values are four voxel words. Rows are output channels, so
 // a lane stores four consecutive channels of one position. The weights stay
 // in registers over the workgroup's chunks, and the next chunk's voxels load
 // while this one's are multiplied: 163 us for 32 pairs with one chunk per
-// workgroup and voxels of 16 bytes, 96 now (301 MB: 3.1 TB/s).
+// workgroup and voxels of 16 bytes, 79 now (301 MB: 3.8 TB/s).
+constexpr int kF0Rows = 8;  // (chunks of four rows: 96 us)
 __global__ __launch_bounds__(kConvLanes) void conv0_forward(const uint32_t *__restrict__ x,
                                                             const uint16_t *__restrict__ wb, int ld,
                                                             const float *__restrict__ bias,
                                                             uint16_t *__restrict__ y, int nchunks) {
-    __shared__ __attribute__((aligned(16))) char lds[4 * kC0Vox];
+    using T = C0Tile<kF0Rows>;
+    __shared__ __attribute__((aligned(16))) char lds[4 * T::kVox];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int r = lane & 15, g = lane >> 4;
     bf16x8 a[2];
@@ -501,34 +549,35 @@ __global__ __launch_bounds__(kConvLanes) void conv0_forward(const uint32_t *__re
             const int tap = 16 * s + 4 * g + j, t = tap < 27 ? tap : 26;
             f.h[2 * j] = tap < 27 ? wb[(r * 27 + t) * ld] : static_cast<uint16_t>(0);
             f.h[2 * j + 1] = tap < 27 ? wb[(r * 27 + t) * ld + 1] : static_cast<uint16_t>(0);
-            off[s][j] = (((t / 9) * (kC0Rows + 2) + w + t / 3 % 3) * kC0Cols + r + t % 3 + 1) * 4;
+            off[s][j] = T::row(t / 9, t / 3 % 3, w) + (r + t % 3 + 1) * 4;
         }
         a[s] = f.v;
     }
     float b4[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) b4[e] = bias[4 * g + e];
-    uint32_t v[kC0Per];
+    uint32_t v[T::kPer];
     int c = blockIdx.x;
-    if (c < nchunks) c0_load(x, c, v);
+    if (c < nchunks) T::load(x, c, v);
     for (; c < nchunks; c += gridDim.x) {
         __syncthreads();
-        c0_store(lds, v);
+        T::store(lds, v);
         __syncthreads();
-        if (c + static_cast<int>(gridDim.x) < nchunks) c0_load(x, c + gridDim.x, v);
+        if (c + static_cast<int>(gridDim.x) < nchunks) T::load(x, c + gridDim.x, v);
         size_t n;
         int z, y0;
-        c0_chunk(c, n, z, y0);
-        uint16_t *row = y + (((n * 64 + z) * 64 + y0 + w) * 64 + r) * 16 + 4 * g;
+        T::chunk(c, n, z, y0);
+        uint16_t *row = y + (((n * 64 + z) * 64 + y0 + w * T::WAVE_ROWS) * 64 + r) * 16 + 4 * g;
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
+        for (int t = 0; t < 4 * T::WAVE_ROWS; ++t) {  // 16 positions each, four to a row
             f32x4 acc = zero_acc();
 #pragma unroll
             for (int s = 0; s < 2; ++s) {
                 uint32_t q[4];
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
-                    q[j] = *reinterpret_cast<const uint32_t *>(lds + off[s][j] + 64 * t);
+                    q[j] = *reinterpret_cast<const uint32_t *>(lds + off[s][j] + (t / 4) * T::COLS * 4 +
+                                                               64 * (t % 4));
                     if (16 * s + 4 * g + j >= 27) q[j] = 0;  // padding: zero weights meet zeros
                 }
                 Frag f;
@@ -547,16 +596,19 @@ __global__ __launch_bounds__(kConvLanes) void conv0_forward(const uint32_t *__re
 // of a staged row, so two (kz, ky) pairs fill a 16-column tile with four voxels
 // each (the fourth, past the taps, is computed and dropped). The transposed
 // read takes 8-byte pieces on 8-byte boundaries: odd columns x read voxels
-// x - 1 .. x + 2, even ones x - 2 .. x + 1, in accumulators of their own. Each
-// wave takes one row of 64 positions per chunk.
+// x - 1 .. x + 2, even ones x - 2 .. x + 1, in accumulators of their own.
+// (24 pairs, 226 MB: 54 us, 4.2 TB/s, at four waves per SIMD; 85 with three
+// and the staged pieces in scratch; 102 with chunks of eight rows.)
 constexpr int kW0Dy = 48;  // bytes per staged dy position (16 channels + 16)
-constexpr int kW0Tile = 4 * kC0Vox;
-constexpr int kW0Lds = kW0Tile + kC0Rows * 64 * kW0Dy;
+constexpr int kW0Rows = 4;
+constexpr int kW0Tile = 4 * C0Tile<kW0Rows>::kVox;
+constexpr int kW0Lds = kW0Tile + kW0Rows * 64 * kW0Dy;
 constexpr int kW0Out = 16 * 54 + 16;      // [16][27][2] and the bias
 
-__global__ __launch_bounds__(kConvLanes) void conv0_wgrad(const uint32_t *__restrict__ x,
+__global__ __launch_bounds__(kConvLanes, 4) void conv0_wgrad(const uint32_t *__restrict__ x,
                                                           const uint16_t *__restrict__ dy,
                                                           float *__restrict__ partial, int nchunks) {
+    using T = C0Tile<kW0Rows>;
     __shared__ __attribute__((aligned(16))) char lds[kW0Lds];
     char *sdy = lds + kW0Tile;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -575,42 +627,44 @@ __global__ __launch_bounds__(kConvLanes) void conv0_wgrad(const uint32_t *__rest
 #pragma unroll
     for (int j = 0; j < 5; ++j) {
         const int q = min(2 * j + (sub >> 1), 8);  // (kz, ky)
-        xoff[j] = (((q / 3) * (kC0Rows + 2) + w + q % 3) * kC0Cols + 2 * kk + 2 * (sub & 1)) * 4;
+        xoff[j] = T::row(q / 3, q % 3, w) + (2 * kk + 2 * (sub & 1)) * 4;
     }
-    const int dbase = (w * 64 + 2 * kk) * kW0Dy + 8 * sub;
-    constexpr int kDyN = kC0Rows * 64 * 2 / kConvLanes;
-    uint32_t v[kC0Per];
-    uint4 d[kDyN];
+    const int dbase = (w * T::WAVE_ROWS * 64 + 2 * kk) * kW0Dy + 8 * sub;
+    constexpr int kDyN = kW0Rows * 64 * 2 / kConvLanes;
+    uint32_t v[T::kPer];
+    u32x4 d[kDyN];
     auto fetch = [&](int c) {
-        c0_load(x, c, v);
+        T::load(x, c, v);
         size_t n;
         int z, y0;
-        c0_chunk(c, n, z, y0);
+        T::chunk(c, n, z, y0);
         const size_t pos0 = ((n * 64 + z) * 64 + y0) * 64;
 #pragma unroll
         for (int k = 0; k < kDyN; ++k)
-            d[k] = *reinterpret_cast<const uint4 *>(dy + pos0 * 16 + (threadIdx.x + k * kConvLanes) * 8);
+            d[k] = *reinterpret_cast<const u32x4 *>(dy + pos0 * 16 + (threadIdx.x + k * kConvLanes) * 8);
     };
     int c = blockIdx.x;
     if (c < nchunks) fetch(c);
     for (; c < nchunks; c += gridDim.x) {
         __syncthreads();
-        c0_store(lds, v);
+        T::store(lds, v);
 #pragma unroll
         for (int k = 0; k < kDyN; ++k) {
             const int i = threadIdx.x + k * kConvLanes;
-            *reinterpret_cast<uint4 *>(sdy + (i >> 1) * kW0Dy + (i & 1) * 16) = d[k];
+            *reinterpret_cast<u32x4 *>(sdy + (i >> 1) * kW0Dy + (i & 1) * 16) = d[k];
         }
         __syncthreads();
         if (c + static_cast<int>(gridDim.x) < nchunks) fetch(c + gridDim.x);
 #pragma unroll
-        for (int q = 0; q < 2; ++q) {  // parity of x
-            const bf16x8 a = tr_frag(sdy + dbase + q * kW0Dy, 8 * kW0Dy);
+        for (int r = 0; r < T::WAVE_ROWS; ++r)
 #pragma unroll
-            for (int j = 0; j < 5; ++j)
-                acc[q][j] = mfma(a, tr_frag(lds + xoff[j] + q * 8, 32), acc[q][j]);
-            accb = mfma(a, ones.v, accb);
-        }
+            for (int q = 0; q < 2; ++q) {  // parity of x
+                const bf16x8 a = tr_frag(sdy + dbase + (64 * r + q) * kW0Dy, 8 * kW0Dy);
+#pragma unroll
+                for (int j = 0; j < 5; ++j)
+                    acc[q][j] = mfma(a, tr_frag(lds + xoff[j] + r * T::COLS * 4 + q * 8, 32), acc[q][j]);
+                accb = mfma(a, ones.v, accb);
+            }
     }
     // the four waves' tiles, added in order
     float *out = partial + static_cast<size_t>(blockIdx.x) * kW0Out;

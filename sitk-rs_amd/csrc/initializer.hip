@@ -65,97 +65,120 @@ __host__ __device__ inline float bf2f(uint16_t h) {
 }
 
 // ------------------------------------------------------- small kernels
-// Global average pool of the last conv output [n][64][128] -> feat [n][128].
-__global__ void gap_forward(const uint16_t *__restrict__ y, int n, float *__restrict__ feat) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n * kFeat) return;
-    const int b = i / kFeat, c = i - b * kFeat;
-    float s = 0.0f;
-    for (int p = 0; p < 64; ++p) s += bf2f(y[(static_cast<size_t>(b) * 64 + p) * kFeat + c]);
-    feat[i] = s * (1.0f / 64.0f);
-}
-
-// The pool's gradient, masked by the last convolution's ReLU.
-__global__ void gap_backward(const float *__restrict__ dfeat, const uint16_t *__restrict__ y, int n,
-                             uint16_t *__restrict__ dy) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n * 64 * kFeat) return;
-    const int c = i % kFeat, b = i / (64 * kFeat);
-    dy[i] = bf2f(y[i]) > 0.0f ? f2bf(dfeat[b * kFeat + c] * (1.0f / 64.0f)) : 0;
-}
-
-// MLP head forward, one workgroup (128 lanes) per sample.
-__global__ __launch_bounds__(128) void mlp_forward(const float *__restrict__ feat,
-                                                   const float *__restrict__ w1,
-                                                   const float *__restrict__ b1,
-                                                   const float *__restrict__ w2,
-                                                   const float *__restrict__ b2,
-                                                   float *__restrict__ hid, float *__restrict__ out) {
-    __shared__ float f[kFeat], h[kHidden];
-    const int b = blockIdx.x, t = threadIdx.x;
-    f[t] = feat[b * kFeat + t];
-    __syncthreads();
-    float s = b1[t];
-    for (int i = 0; i < kFeat; ++i) s += w1[t * kFeat + i] * f[i];
-    s = fmaxf(s, 0.0f);
-    h[t] = s;
-    hid[b * kHidden + t] = s;
-    __syncthreads();
-    if (t < kOut) {
-        float o = b2[t];
-        for (int j = 0; j < kHidden; ++j) o += w2[t * kHidden + j] * h[j];
-        out[b * kOut + t] = o;
-    }
-}
-
-// MLP head backward over the whole batch (one workgroup, fixed loop orders):
-// gradients of w2, b2, w1, b1 and of the pooled features.
-__global__ __launch_bounds__(128) void mlp_backward(int n, const float *__restrict__ feat,
-                                                    const float *__restrict__ hid,
-                                                    const float *__restrict__ dout,
+// Global average pool of the last conv output [n][64][128] and the MLP head,
+// one workgroup of 256 lanes per sample: lane (h, t) sums half of channel t's
+// positions, then half of row t of W1 (32-byte pieces), and two waves share
+// the output rows.
+__global__ __launch_bounds__(256) void head_forward(const uint16_t *__restrict__ y,
                                                     const float *__restrict__ w1,
+                                                    const float *__restrict__ b1,
                                                     const float *__restrict__ w2,
-                                                    float *__restrict__ gw1, float *__restrict__ gb1,
-                                                    float *__restrict__ gw2, float *__restrict__ gb2,
-                                                    float *__restrict__ dhid,
-                                                    float *__restrict__ dfeat) {
-    const int t = threadIdx.x;
-    // dhid[b][t] = relu'(hid) * sum_o w2[o][t] dout[b][o]
-    for (int b = 0; b < n; ++b) {
-        float s = 0.0f;
-        for (int o = 0; o < kOut; ++o) s += w2[o * kHidden + t] * dout[b * kOut + o];
-        dhid[b * kHidden + t] = hid[b * kHidden + t] > 0.0f ? s : 0.0f;
+                                                    const float *__restrict__ b2,
+                                                    float *__restrict__ feat, float *__restrict__ hid,
+                                                    float *__restrict__ out) {
+    __shared__ float part[2][kFeat], f[kFeat], hh[kHidden];
+    const int b = blockIdx.x, t = threadIdx.x & 127, h = threadIdx.x >> 7;
+    // the lane's half row of W1, on its way while the pool is summed
+    float4 w[kFeat / 8];
+#pragma unroll
+    for (int k = 0; k < kFeat / 8; ++k)
+        w[k] = reinterpret_cast<const float4 *>(w1 + t * kFeat + h * (kFeat / 2))[k];
+    float s = 0.0f;
+#pragma unroll 16
+    for (int p = 32 * h; p < 32 * h + 32; ++p)
+        s += bf2f(y[(static_cast<size_t>(b) * 64 + p) * kFeat + t]);
+    part[h][t] = s;
+    __syncthreads();
+    if (h == 0) {
+        const float v = (part[0][t] + part[1][t]) * (1.0f / 64.0f);
+        f[t] = v;
+        feat[b * kFeat + t] = v;
     }
     __syncthreads();
-    // gw2[o][t] = sum_b dout[b][o] hid[b][t]; gb2[o] = sum_b dout[b][o]
-    for (int o = 0; o < kOut; ++o) {
-        float s = 0.0f;
-        for (int b = 0; b < n; ++b) s += dout[b * kOut + o] * hid[b * kHidden + t];
-        gw2[o * kHidden + t] = s;
+    s = 0.0f;
+#pragma unroll
+    for (int k = 0; k < kFeat / 8; ++k) {
+        const float *q = f + h * (kFeat / 2) + 4 * k;
+        s += w[k].x * q[0];
+        s += w[k].y * q[1];
+        s += w[k].z * q[2];
+        s += w[k].w * q[3];
     }
-    if (t < kOut) {
-        float s = 0.0f;
-        for (int b = 0; b < n; ++b) s += dout[b * kOut + t];
-        gb2[t] = s;
+    part[h][t] = s;
+    __syncthreads();
+    if (h == 0) {
+        const float v = fmaxf(b1[t] + (part[0][t] + part[1][t]), 0.0f);
+        hh[t] = v;
+        hid[b * kHidden + t] = v;
     }
-    // gw1[t][i] = sum_b dhid[b][t] feat[b][i]; gb1[t] = sum_b dhid[b][t]
-    for (int i = 0; i < kFeat; ++i) {
-        float s = 0.0f;
-        for (int b = 0; b < n; ++b) s += dhid[b * kHidden + t] * feat[b * kFeat + i];
-        gw1[t * kFeat + i] = s;
-    }
-    {
-        float s = 0.0f;
-        for (int b = 0; b < n; ++b) s += dhid[b * kHidden + t];
-        gb1[t] = s;
-    }
-    // dfeat[b][t] = sum_j w1[j][t] dhid[b][j]
-    for (int b = 0; b < n; ++b) {
-        float s = 0.0f;
-        for (int j = 0; j < kHidden; ++j) s += w1[j * kFeat + t] * dhid[b * kHidden + j];
-        dfeat[b * kFeat + t] = s;
+    __syncthreads();
+    // output o by wave o mod 4
+    const int lane = threadIdx.x & 63;
+    for (int o = threadIdx.x >> 6; o < kOut; o += 4) {
+        float v = w2[o * kHidden + lane] * hh[lane] + w2[o * kHidden + 64 + lane] * hh[64 + lane];
+#pragma unroll
+        for (int k = 32; k > 0; k >>= 1) v += __shfl_xor(v, k, 64);
+        if (lane == 0) out[b * kOut + o] = b2[o] + v;
     }
 }
+
+// MLP head backward, per sample (one workgroup of 256 lanes): the hidden
+// gradient dhid = relu'(hid) * W2' dout, the pooled features' dfeat = W1' dhid
+// (128 lanes each), and through the pool and the last convolution's ReLU the
+// gradient of its 64 output positions.
+__global__ __launch_bounds__(256) void head_backward_samples(
+    const float *__restrict__ hid, const float *__restrict__ dout, const float *__restrict__ w1,
+    const float *__restrict__ w2, const uint16_t *__restrict__ y, float *__restrict__ dhid,
+    uint16_t *__restrict__ dy) {
+    __shared__ float dh[kHidden], half[2][kFeat];
+    const int b = blockIdx.x, t = threadIdx.x & 127, h = threadIdx.x >> 7;
+    if (h == 0) {
+        float s = 0.0f;
+#pragma unroll
+        for (int o = 0; o < kOut; ++o) s += w2[o * kHidden + t] * dout[b * kOut + o];
+        s = hid[b * kHidden + t] > 0.0f ? s : 0.0f;
+        dh[t] = s;
+        dhid[b * kHidden + t] = s;
+    }
+    __syncthreads();
+    float s = 0.0f;
+#pragma unroll 16
+    for (int j = 64 * h; j < 64 * h + 64; ++j) s += w1[j * kFeat + t] * dh[j];
+    half[h][t] = s;
+    __syncthreads();
+    const uint16_t g = f2bf((half[0][t] + half[1][t]) * (1.0f / 64.0f));
+#pragma unroll 8
+    for (int p = h; p < 64; p += 2) {
+        const size_t i = (static_cast<size_t>(b) * 64 + p) * kFeat + t;
+        dy[i] = bf2f(y[i]) > 0.0f ? g : 0;
+    }
+}
+
+// The head's weight gradients, sums over the batch in order: workgroup r <
+// 128 takes row r of W1 (and b1[r]), workgroup 128 + o row o of W2 (and b2[o]).
+// (One workgroup for the whole head, looping over samples and rows, took
+// 363 us for 24 samples; the two kernels take 8.)
+__global__ __launch_bounds__(128) void head_backward_weights(
+    int n, const float *__restrict__ feat, const float *__restrict__ hid,
+    const float *__restrict__ dout, const float *__restrict__ dhid, float *__restrict__ gw1,
+    float *__restrict__ gb1, float *__restrict__ gw2, float *__restrict__ gb2) {
+    const int t = threadIdx.x;
+    const bool first = blockIdx.x < kHidden;
+    const int r = first ? blockIdx.x : blockIdx.x - kHidden;
+    const float *row = first ? dhid + r : dout + r;
+    const float *col = first ? feat : hid;
+    const int ld = first ? kHidden : kOut;
+    float s = 0.0f, sb = 0.0f;
+#pragma unroll 8
+    for (int b = 0; b < n; ++b) {
+        const float d = row[b * ld];
+        s += d * col[b * kFeat + t];
+        sb += d;
+    }
+    (first ? gw1 : gw2)[r * kFeat + t] = s;
+    if (t == 0) (first ? gb1 : gb2)[r] = sb;
+}
+static_assert(kFeat == kHidden && kFeat == 128, "the head's kernels share their lane layout");
 
 // Adam (Kingma & Ba 2015) on the flat FP32 parameters.
 __global__ void adam_step(float *__restrict__ p, const float *__restrict__ g, float *__restrict__ m,
@@ -172,17 +195,28 @@ __global__ void adam_step(float *__restrict__ p, const float *__restrict__ g, fl
     }
 }
 
-// BF16 copies of one conv layer's weights: w [co][27][ci] and the transposed
-// wt [ci][27][co] the input-gradient GEMM reads.
-__global__ void cast_weights(const float *__restrict__ w, int co, int ci, uint16_t *__restrict__ wb,
-                             uint16_t *__restrict__ wt) {
-    const int n = co * 27 * ci;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        const int c = i % ci, tap = (i / ci) % 27, o = i / (27 * ci);
-        const uint16_t h = f2bf(w[i]);
-        wb[i] = h;
-        wt[(static_cast<size_t>(c) * 27 + tap) * co + o] = h;
-    }
+// BF16 copies of the conv layers' weights, all layers in one launch: w
+// [co][27][ci] and, for the input gradient, transposed [ci][27][co].
+struct CastLayer {
+    const float *w;
+    uint16_t *wb, *wt;
+    int co, ci, begin;  // begin: the layer's first index over all layers
+};
+struct CastLayers {
+    CastLayer l[kLayers];
+    int total;
+};
+__global__ __launch_bounds__(256) void cast_weights(CastLayers L) {
+    const int at = blockIdx.x * 256 + threadIdx.x;
+    if (at >= L.total) return;
+    int k = 0;
+    while (k + 1 < kLayers && at >= L.l[k + 1].begin) ++k;
+    const CastLayer &q = L.l[k];
+    const int i = at - q.begin;
+    const int c = i % q.ci, tap = (i / q.ci) % 27, o = i / (27 * q.ci);
+    const uint16_t h = f2bf(q.w[i]);
+    q.wb[i] = h;
+    q.wt[(static_cast<size_t>(c) * 27 + tap) * q.co + o] = h;
 }
 
 // The 64^3 input volumes are read four voxels per lane.
@@ -273,7 +307,7 @@ struct Net {
     DeviceBuffer<uint16_t> dact[kLayers + 1];  // gradients w.r.t. act (masked); none for the input
     DeviceBuffer<float> partials;              // weight-gradient rows of every layer
     size_t off_partial[kLayers];
-    DeviceBuffer<float> feat, hid, out, dout, dhid, dfeat;
+    DeviceBuffer<float> feat, hid, out, dout, dhid;
     bool weights_dirty = true;
 };
 
@@ -293,7 +327,7 @@ static size_t act_elems(int idx, int n) {  // idx 0 = input, idx l+1 = conv l ou
 // activations', never more than the chunks of positions there are.
 static int wgrad_rows(int layer, int n) {
     static const int most[kLayers] = {1024, 512, 128, 64, 16};
-    const int chunks[kLayers] = {n * kEdge * kC0PerPlane, InTile<5, 16, 2, 1, 3>::chunks(n),
+    const int chunks[kLayers] = {C0Tile<kW0Rows>::chunks(n), InTile<5, 16, 2, 1, 3>::chunks(n),
                                  InTile<4, 32, 2, 1, 3>::chunks(n), InTile<3, 64, 8, 1, 1>::chunks(n),
                                  InTile<2, 64, 4, 2, 2>::chunks(n)};
     return std::min(most[layer], chunks[layer]);
@@ -380,7 +414,6 @@ Net *create(int max_batch, uint64_t seed) {
         net->out.alloc(static_cast<size_t>(max_batch) * kOut);
         net->dout.alloc(static_cast<size_t>(max_batch) * kOut);
         net->dhid.alloc(static_cast<size_t>(max_batch) * kHidden);
-        net->dfeat.alloc(static_cast<size_t>(max_batch) * kFeat);
         init_params(*net, seed);
     } catch (...) {
         delete net;
@@ -391,14 +424,14 @@ Net *create(int max_batch, uint64_t seed) {
 
 static void refresh_weights(Net &net) {
     if (!net.weights_dirty) return;
+    CastLayers L;
+    L.total = 0;
     for (int l = 0; l < kLayers; ++l) {
-        LaunchScope scope("cnn_cast_weights");
-        const int n = kCh[l + 1] * 27 * kCh[l];
-        hipLaunchKernelGGL(cast_weights, dim3((n + 255) / 256), dim3(256), 0, backend().stream,
-                           net.params.ptr + net.off_w[l], kCh[l + 1], kCh[l], net.wb[l].ptr,
-                           net.wt[l].ptr);
-        check_launch("cast_weights");
+        L.l[l] = {net.params.ptr + net.off_w[l], net.wb[l].ptr, net.wt[l].ptr, kCh[l + 1], kCh[l], L.total};
+        L.total += kCh[l + 1] * 27 * kCh[l];
     }
+    launch_kernel("cnn_cast_weights", cast_weights, dim3((L.total + 255) / 256), dim3(256), 0, L);
+    check_launch("cast_weights");
     net.weights_dirty = false;
 }
 
@@ -406,6 +439,8 @@ static void check_batch(const Net &net, int n) {
     if (n < 1 || n > net.max_batch)
         fail(SITKHIP_ERR_INVALID_ARGUMENT, "batch must be 1.." + std::to_string(net.max_batch));
 }
+
+static const float *param(const Net &net, size_t off) { return net.params.ptr + off; }
 
 static const uint32_t *input_words(const Net &net) {
     return reinterpret_cast<const uint32_t *>(net.act[0].ptr);
@@ -425,29 +460,30 @@ static void allow_lds(F kernel, size_t bytes) {
 }
 
 template <int LGDO, int CI, int CO, int R, int COW, bool HOLD>
-static void launch_forward(Net &net, int layer, int n, int per_cu) {
+static void launch_forward(Net &net, int layer, int n, int per_cu = 0) {
     using T = InTile<LGDO, CI, R, 1, 3>;
     auto kernel = conv_forward<LGDO, CI, CO, R, COW, HOLD>;
     const int chunks = T::chunks(n);
     allow_lds(kernel, T::kBytes);
-    launch_kernel("cnn_conv_fwd", kernel, dim3(resident(per_cu, chunks), CO / COW), dim3(kConvLanes),
+    launch_kernel("cnn_conv_fwd", kernel, dim3(HOLD ? resident(per_cu, chunks) : chunks, CO / COW), dim3(kConvLanes),
                   T::kBytes, static_cast<const uint16_t *>(net.act[layer].ptr),
                   static_cast<const uint16_t *>(net.wb[layer].ptr),
-                  static_cast<const float *>(net.params.ptr + net.off_b[layer]), net.act[layer + 1].ptr,
+                  param(net, net.off_b[layer]), net.act[layer + 1].ptr,
                   chunks);
     check_launch("cnn_conv_fwd");
 }
 
-template <int LGDO, int CI, int CO, int QY, int QZ, int CG>
+template <int LGDO, int CI, int CO, int QY, int QZ, int CG, bool HOLD>
 static void launch_dgrad(Net &net, int layer, int n) {
     constexpr int DO = 1 << LGDO;
     constexpr size_t lds = static_cast<size_t>(QZ + 1) * (QY + 1) * (DO + 1) * (2 * CO + 16);
     static_assert(lds <= 64 * 1024, "the staged dy fits the default limit");
-    launch_kernel("cnn_conv_dgrad", conv_dgrad<LGDO, CI, CO, QY, QZ, CG>,
-                  dim3(n * (DO / QY) * (DO / QZ), CG), dim3(kConvLanes), lds,
+    const int tiles = n * (DO / QY) * (DO / QZ);
+    launch_kernel("cnn_conv_dgrad", conv_dgrad<LGDO, CI, CO, QY, QZ, CG, HOLD>,
+                  dim3(HOLD ? resident(2, tiles) : tiles, CG), dim3(kConvLanes), lds,
                   static_cast<const uint16_t *>(net.dact[layer + 1].ptr),
                   static_cast<const uint16_t *>(net.wt[layer].ptr),
-                  static_cast<const uint16_t *>(net.act[layer].ptr), net.dact[layer].ptr);
+                  static_cast<const uint16_t *>(net.act[layer].ptr), net.dact[layer].ptr, tiles);
     check_launch("cnn_conv_dgrad");
 }
 
@@ -468,26 +504,21 @@ void forward(Net &net, int n, float *out_host) {
     check_batch(net, n);
     refresh_weights(net);
     {
-        const int chunks = n * kEdge * kC0PerPlane;
+        const int chunks = C0Tile<kF0Rows>::chunks(n);
         launch_kernel("cnn_conv0_fwd", conv0_forward, dim3(resident(8, chunks)), dim3(kConvLanes), 0,
                       input_words(net), static_cast<const uint16_t *>(net.wb[0].ptr), kCin0,
-                      static_cast<const float *>(net.params.ptr + net.off_b[0]), net.act[1].ptr, chunks);
+                      param(net, net.off_b[0]), net.act[1].ptr, chunks);
         check_launch("conv0_forward");
     }
     launch_forward<5, 16, 32, 2, 32, true>(net, 1, n, 3);
     launch_forward<4, 32, 64, 2, 64, true>(net, 2, n, 2);
-    launch_forward<3, 64, 64, 4, 64, false>(net, 3, n, 2);
-    launch_forward<2, 64, 128, 4, 64, false>(net, 4, n, 4);
-    {
-        LaunchScope scope("cnn_head");
-        hipLaunchKernelGGL(gap_forward, dim3((n * kFeat + 255) / 256), dim3(256), 0, backend().stream,
-                           net.act[kLayers].ptr, n, net.feat.ptr);
-        hipLaunchKernelGGL(mlp_forward, dim3(n), dim3(128), 0, backend().stream, net.feat.ptr,
-                           net.params.ptr + net.off_w1, net.params.ptr + net.off_b1,
-                           net.params.ptr + net.off_w2, net.params.ptr + net.off_b2, net.hid.ptr,
-                           net.out.ptr);
-        check_launch("cnn_head");
-    }
+    launch_forward<3, 64, 64, 4, 64, false>(net, 3, n);
+    launch_forward<2, 64, 128, 4, 64, false>(net, 4, n);
+    launch_kernel("cnn_head", head_forward, dim3(n), dim3(256), 0,
+                  static_cast<const uint16_t *>(net.act[kLayers].ptr), param(net, net.off_w1),
+                  param(net, net.off_b1), param(net, net.off_w2), param(net, net.off_b2), net.feat.ptr,
+                  net.hid.ptr, net.out.ptr);
+    check_launch("cnn_head");
     if (out_host) {
         net.out.download(out_host, static_cast<size_t>(n) * kOut);
     }
@@ -498,30 +529,29 @@ void forward(Net &net, int n, float *out_host) {
 // every parameter gradient into net.grads.
 void backward(Net &net, int n, const float *dout_host) {
     check_batch(net, n);
-    hipStream_t st = backend().stream;
     net.dout.upload(dout_host, static_cast<size_t>(n) * kOut);
-    {
-        LaunchScope scope("cnn_head_bwd");
-        hipLaunchKernelGGL(mlp_backward, dim3(1), dim3(128), 0, st, n, net.feat.ptr, net.hid.ptr,
-                           net.dout.ptr, net.params.ptr + net.off_w1, net.params.ptr + net.off_w2,
-                           net.grads.ptr + net.off_w1, net.grads.ptr + net.off_b1,
-                           net.grads.ptr + net.off_w2, net.grads.ptr + net.off_b2, net.dhid.ptr,
-                           net.dfeat.ptr);
-        hipLaunchKernelGGL(gap_backward, dim3((n * 64 * kFeat + 255) / 256), dim3(256), 0, st,
-                           net.dfeat.ptr, net.act[kLayers].ptr, n, net.dact[kLayers].ptr);
-        check_launch("cnn_head_bwd");
-    }
+    launch_kernel("cnn_head_bwd", head_backward_samples, dim3(n), dim3(256), 0,
+                  static_cast<const float *>(net.hid.ptr), static_cast<const float *>(net.dout.ptr),
+                  param(net, net.off_w1), param(net, net.off_w2),
+                  static_cast<const uint16_t *>(net.act[kLayers].ptr), net.dhid.ptr,
+                  net.dact[kLayers].ptr);
+    launch_kernel("cnn_head_bwd", head_backward_weights, dim3(kHidden + kOut), dim3(128), 0, n,
+                  static_cast<const float *>(net.feat.ptr), static_cast<const float *>(net.hid.ptr),
+                  static_cast<const float *>(net.dout.ptr), static_cast<const float *>(net.dhid.ptr),
+                  net.grads.ptr + net.off_w1, net.grads.ptr + net.off_b1, net.grads.ptr + net.off_w2,
+                  net.grads.ptr + net.off_b2);
+    check_launch("cnn_head_bwd");
     launch_wgrad<2, 64, 128, 4, 2, 1, 64>(net, 4, n);
-    launch_dgrad<2, 64, 128, 4, 4, 4>(net, 4, n);
+    launch_dgrad<2, 64, 128, 4, 4, 4, false>(net, 4, n);
     launch_wgrad<3, 64, 64, 8, 1, 1, 64>(net, 3, n);
-    launch_dgrad<3, 64, 64, 8, 1, 4>(net, 3, n);
+    launch_dgrad<3, 64, 64, 8, 1, 4, false>(net, 3, n);
     launch_wgrad<4, 32, 64, 2, 1, 3, 32>(net, 2, n);
-    launch_dgrad<4, 32, 64, 8, 1, 1>(net, 2, n);
+    launch_dgrad<4, 32, 64, 8, 1, 1, false>(net, 2, n);
     launch_wgrad<5, 16, 32, 2, 1, 3, 32>(net, 1, n);
-    launch_dgrad<5, 16, 32, 4, 1, 1>(net, 1, n);
+    launch_dgrad<5, 16, 32, 4, 1, 1, true>(net, 1, n);
     launch_kernel("cnn_conv_wgrad", conv0_wgrad, dim3(wgrad_rows(0, n)), dim3(kConvLanes), 0,
                   input_words(net), static_cast<const uint16_t *>(net.dact[1].ptr),
-                  net.partials.ptr + net.off_partial[0], n * kEdge * kC0PerPlane);
+                  net.partials.ptr + net.off_partial[0], C0Tile<kW0Rows>::chunks(n));
     check_launch("conv0_wgrad");
     PartialJobs jobs;
     jobs.n = kLayers;
