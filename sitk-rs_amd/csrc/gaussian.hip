@@ -26,6 +26,7 @@
 #include <vector>
 
 #include <cmath>
+#include <cstring>
 #include <mutex>
 
 #include "common.hpp"
@@ -199,26 +200,57 @@ __global__ __launch_bounds__(256) void iir_lines(const SrcT *__restrict__ src, d
 // Two lanes per line, 32 lines per wavefront: lane l < 32 runs the causal
 // recursion of line l forward while lane l + 32 runs the anti-causal recursion
 // of the same line backward, in lock-step. At step i the causal lane produces
-// outs[i] and the anti-causal lane scratch[n-1-i]. Until the middle (i < H =
-// ceil(n/2)) each lane parks its value in LDS; after it, each lane reads its
-// partner's value for the same element (produced n-1-i steps earlier) and
-// writes the finished output outs[k] + scratch[k]. The causal outputs never
-// leave the chip, so a line costs one read of its input per lane and one write
-// of its output. Both recursions have the same shape,
+// outs[i] and the anti-causal lane scratch[n-1-i]. Until the middle each lane
+// parks its values; after it, each lane takes its partner's value for the same
+// element (parked n-1-i steps earlier) and writes the finished output outs[k] +
+// scratch[k] (of an odd line's middle element both lanes hold their term at
+// the same step). The causal outputs never leave the chip, so a line costs one
+// read of its input per lane and one write of its output. Both recursions have
+// the same shape,
 //     v = (((x*c0 + a*c1) + b*c2) + cc*c3) - (((p1*d1 + p2*d2) + p3*d3) + p4*d4),
 // with (c0..c3) = (n0..n3) for the causal lane and (m1..m4) for the anti-causal
 // lane (whose x is data[j+1] for output j), so the loop is lane-uniform.
-// Loads run one to two blocks of kPD steps ahead of their use.
+//
+// The last kRegPairs * 16 values before the middle are parked in registers (a
+// partner's come across the wave by ds_bpermute), the earlier ones in LDS: at
+// 256 voxels a wave of 32 lines takes 24 KB of LDS instead of 64, so every
+// line of a 256 x 256 x 160 volume is resident at once (five waves per CU; with
+// all values in LDS two, and 98 / 72 / 44 us for the three axes; now 47 / 38 /
+// 29: 2.7 / 4.4 / 4.3 TB/s). Four pairs leave 32 KB, which five waves of a CU
+// do not fit, and took 61 / 51 / 30; six spill. The registers then allow two
+// waves per SIMD; fewer pairs for more waves gained nothing on short lines.
+//
+// Steps run in blocks of eight whose inputs load one to two blocks ahead, into
+// two register blocks used in turn (blocks of sixteen measured the same).
+// ALONG0 (axis 0, whose lines are contiguous):
+// a block's inputs are two or four 16-byte loads of the lane's own line, and
+// its outputs 16-byte stores -- one step per instruction touched 64 cache
+// lines for 4 or 8 bytes each and bound that axis.
 constexpr int kPairLines = 32;
-#ifndef SITKHIP_IIR_PD
-#define SITKHIP_IIR_PD 8
-#endif
-constexpr int kPD = SITKHIP_IIR_PD;
+constexpr int kPD = 8;
+constexpr int kRegPairs = 5;
 
-template <typename SrcT, typename DstT>
+// Steps [0, lds_steps) of a line of n voxels (n >= 8) are parked in LDS, the
+// others before the middle in registers.
+__host__ __device__ inline int reg_pairs(int n) {
+    const int k = (n / 2 - 4) / (2 * kPD);
+    return k < kRegPairs ? k : kRegPairs;
+}
+__host__ __device__ inline int lds_steps(int n) { return n / 2 - 2 * kPD * reg_pairs(n); }
+inline size_t pair_lds_bytes(int n) {
+    return static_cast<size_t>(2) * lds_steps(n) * kPairLines * sizeof(double);
+}
+
+// Sixteen bytes of a contiguous line, at the element's alignment.
+template <typename T>
+struct alignas(sizeof(T)) Vec16 {
+    T v[16 / sizeof(T)];
+};
+
+template <typename SrcT, typename DstT, bool ALONG0>
 __device__ __forceinline__ void iir_pair_body(const SrcT *__restrict__ src, DstT *__restrict__ dst,
-                                              const LineSet &L, const IirCoef &k, int H,
-                                              unsigned block, double *lds) {
+                                              const LineSet &L, const IirCoef &k, unsigned block,
+                                              double *lds) {
     const int lane = threadIdx.x;
     const int role = lane >> 5;  // 0 causal, 1 anti-causal
     const int li = lane & 31;
@@ -226,7 +258,7 @@ __device__ __forceinline__ void iir_pair_body(const SrcT *__restrict__ src, DstT
     const bool act = line < L.nlines;
     if (!act) line = L.nlines - 1;  // mirror a valid line; stores are suppressed
     const long long s0 = line_start(L, line);
-    const long long st = L.stride;
+    const long long st = ALONG0 ? 1 : L.stride;
     const int n = L.len;
     const double *c = k.c;
     const double d1 = c[4], d2 = c[5], d3 = c[6], d4 = c[7];
@@ -234,8 +266,9 @@ __device__ __forceinline__ void iir_pair_body(const SrcT *__restrict__ src, DstT
     const double c1 = role ? c[9] : c[1];
     const double c2 = role ? c[10] : c[2];
     const double c3 = role ? c[11] : c[3];
-    double *mine = lds + role * H * kPairLines;
-    const double *partner = lds + (1 - role) * H * kPairLines;
+    const int park = lds_steps(n), pairs = reg_pairs(n), half = n / 2;
+    double *mine = lds + role * park * kPairLines + li;
+    const double *partner = lds + (1 - role) * park * kPairLines + li;
 
     double a, b, cc, p1, p2, p3, p4;
     double v[4];
@@ -277,92 +310,176 @@ __device__ __forceinline__ void iir_pair_body(const SrcT *__restrict__ src, DstT
         p1 = q4; p2 = q3; p3 = q2; p4 = q1;
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i) mine[i * kPairLines + li] = v[i];
+    for (int i = 0; i < 4; ++i) mine[i * kPairLines] = v[i];
 
-    // value read at step i sits at A + i*S; output of step i goes to W + i*S
+    // the value read at step i sits at A + i * S; the output of step i at W + i * S
     const long long S = role ? -st : st;
-    const long long A = role ? s0 + static_cast<long long>(n) * st : s0;
-    const long long W = role ? s0 + static_cast<long long>(n - 1) * st : s0;
+    const SrcT *const A = src + (role ? s0 + static_cast<long long>(n) * st : s0);
+    DstT *const W = dst + (role ? s0 + static_cast<long long>(n - 1) * st : s0);
 
-    // Loads run one block of kPD steps ahead, into two register blocks used
-    // in turn (no copies between them, which would wait for the loads). Every
-    // load is unconditional: a step past the line re-reads step n-1's value,
-    // which is never used.
+    // The inputs of steps base .. base + 7. A block that would pass the line's
+    // end reads inside it instead (its values are not used).
     auto load_block = [&](SrcT (&buf)[kPD], int base) {
+        const bool in = base + kPD <= n;
+        if constexpr (ALONG0) {
+            constexpr int kV = 16 / sizeof(SrcT);
+            // ascending addresses: the anti-causal lane's block is read reversed
+            const SrcT *p = in ? (role ? A - base - (kPD - 1) : A + base) : src + s0;
+            Vec16<SrcT> q[kPD / kV];
 #pragma unroll
-        for (int j = 0; j < kPD; ++j) {
-            const int i = base + j < n ? base + j : n - 1;
-            buf[j] = src[A + i * S];
+            for (int j = 0; j < kPD / kV; ++j) q[j] = *reinterpret_cast<const Vec16<SrcT> *>(p + j * kV);
+#pragma unroll
+            for (int j = 0; j < kPD; ++j) {
+                const int r = kPD - 1 - j;
+                buf[j] = role ? q[r / kV].v[r % kV] : q[j / kV].v[j % kV];
+            }
+        } else {
+            const SrcT *p = A + static_cast<long long>(in ? base : n - 1) * S;
+            const long long step = in ? S : 0;
+#pragma unroll
+            for (int j = 0; j < kPD; ++j) {
+                buf[j] = *p;
+                p += step;
+            }
         }
     };
-    auto recur = [&](SrcT v) {
-        const double x = widen(v);
+    auto store_block = [&](const DstT (&o)[kPD], int base) {
+        if (!act) return;
+        if constexpr (ALONG0) {
+            constexpr int kV = 16 / sizeof(DstT);
+            DstT *p = role ? W - base - (kPD - 1) : W + base;
+#pragma unroll
+            for (int j = 0; j < kPD / kV; ++j) {
+                Vec16<DstT> q;
+#pragma unroll
+                for (int e = 0; e < kV; ++e) q.v[e] = role ? o[kPD - 1 - (j * kV + e)] : o[j * kV + e];
+                *reinterpret_cast<Vec16<DstT> *>(p + j * kV) = q;
+            }
+        } else {
+            DstT *p = W + base * S;
+#pragma unroll
+            for (int j = 0; j < kPD; ++j) {
+                *p = o[j];
+                p += S;
+            }
+        }
+    };
+    auto recur = [&](SrcT in) {
+        const double x = widen(in);
         double o = x * c0 + a * c1 + b * c2 + cc * c3;
         o -= p1 * d1 + p2 * d2 + p3 * d3 + p4 * d4;
         cc = b; b = a; a = x;
         p4 = p3; p3 = p2; p2 = p1; p1 = o;
         return o;
     };
-    // the workgroup is this one wave: before the first read of the partner's
-    // parked values only this wave's LDS writes need to have landed
-    auto lds_sync = [&]() {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-        __builtin_amdgcn_s_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-    };
-    auto run_block = [&](const SrcT (&buf)[kPD], int base) {
-        if (base + kPD <= H) {  // every step parks its value
+    // the input of one step, for what does not fill a block
+    auto input = [&](int i) { return A[static_cast<long long>(i) * S]; };
+
+    // ---- steps 4 .. park - 1 into LDS: first those past whole pairs of blocks
+    const int odd_steps = (park - 4) % (2 * kPD);
+    SrcT bufA[kPD], bufB[kPD];
+    int base = 4 + odd_steps;
+    load_block(bufA, base);
+    {
+        SrcT x[2 * kPD - 1];
 #pragma unroll
-            for (int j = 0; j < kPD; ++j) mine[(base + j) * kPairLines + li] = recur(buf[j]);
-        } else if (base >= H && base + kPD <= n) {  // every step finishes an output
-            if (base == H) lds_sync();
+        for (int j = 0; j < 2 * kPD - 1; ++j) x[j] = input(4 + (j < odd_steps ? j : 0));
+#pragma unroll
+        for (int j = 0; j < 2 * kPD - 1; ++j)
+            if (j < odd_steps) mine[(4 + j) * kPairLines] = recur(x[j]);
+    }
+    for (; base < park; base += 2 * kPD) {
+        load_block(bufB, base + kPD);
+#pragma unroll
+        for (int j = 0; j < kPD; ++j) mine[(base + j) * kPairLines] = recur(bufA[j]);
+        load_block(bufA, base + 2 * kPD);
+#pragma unroll
+        for (int j = 0; j < kPD; ++j) mine[(base + kPD + j) * kPairLines] = recur(bufB[j]);
+    }
+    // ---- steps park .. n / 2 - 1 into registers
+    double held[kRegPairs][2 * kPD];
+#pragma unroll
+    for (int r = 0; r < kRegPairs; ++r) {
+        if (r < pairs) {
+            load_block(bufB, base + kPD);
+#pragma unroll
+            for (int j = 0; j < kPD; ++j) held[r][j] = recur(bufA[j]);
+            load_block(bufA, base + 2 * kPD);
+#pragma unroll
+            for (int j = 0; j < kPD; ++j) held[r][kPD + j] = recur(bufB[j]);
+            base += 2 * kPD;
+        }
+    }
+    // ---- an odd line's middle element: both lanes hold their term now
+    if (n & 1) {
+        const double o = recur(base + kPD <= n ? bufA[0] : input(base));
+        const double q = __shfl_xor(o, 32, 64);
+        if (role == 0 && act) W[static_cast<long long>(half) * S] = narrow<DstT>(o + q);
+        ++base;
+        load_block(bufA, base);
+    }
+    // ---- back through the registers
+    auto run_back = [&](const SrcT (&buf)[kPD], const double (&q)[kPD], int at) {
+        DstT o[kPD];
+#pragma unroll
+        for (int j = 0; j < kPD; ++j) o[j] = narrow<DstT>(recur(buf[j]) + q[j]);
+        store_block(o, at);
+    };
+#pragma unroll
+    for (int r = kRegPairs - 1; r >= 0; --r) {
+        if (r < pairs) {
             double q[kPD];
 #pragma unroll
-            for (int j = 0; j < kPD; ++j) q[j] = partner[(n - 1 - base - j) * kPairLines + li];
+            for (int j = 0; j < kPD; ++j) q[j] = __shfl_xor(held[r][2 * kPD - 1 - j], 32, 64);
+            load_block(bufB, base + kPD);
+            run_back(bufA, q, base);
 #pragma unroll
-            for (int j = 0; j < kPD; ++j) {
-                const double o = recur(buf[j]);
-                if (act) dst[W + (base + j) * S] = narrow<DstT>(o + q[j]);
-            }
-        } else {
+            for (int j = 0; j < kPD; ++j) q[j] = __shfl_xor(held[r][kPD - 1 - j], 32, 64);
+            load_block(bufA, base + 2 * kPD);
+            run_back(bufB, q, base + kPD);
+            base += 2 * kPD;
+        }
+    }
+    // ---- back through LDS. The workgroup is this one wave: before the first
+    // read of the partner's values only this wave's LDS writes need to have landed.
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+    for (; base + 2 * kPD <= n; base += 2 * kPD) {
+        double q[kPD];
 #pragma unroll
-            for (int j = 0; j < kPD; ++j) {
-                const int i = base + j;
-                if (i < n) {
-                    const double o = recur(buf[j]);
-                    if (i < H) {
-                        mine[i * kPairLines + li] = o;
-                    } else {
-                        if (i == H) lds_sync();
-                        const double q = partner[(n - 1 - i) * kPairLines + li];
-                        if (act) dst[W + i * S] = narrow<DstT>(o + q);
-                    }
-                }
+        for (int j = 0; j < kPD; ++j) q[j] = partner[(n - 1 - base - j) * kPairLines];
+        load_block(bufB, base + kPD);
+        run_back(bufA, q, base);
+#pragma unroll
+        for (int j = 0; j < kPD; ++j) q[j] = partner[(n - 1 - base - kPD - j) * kPairLines];
+        load_block(bufA, base + 2 * kPD);
+        run_back(bufB, q, base + kPD);
+    }
+    if (base < n) {  // the last steps, loaded together
+        SrcT x[2 * kPD - 1];
+        double q[2 * kPD - 1];
+#pragma unroll
+        for (int j = 0; j < 2 * kPD - 1; ++j) {
+            const int i = base + j < n ? base + j : n - 1;
+            x[j] = input(i);
+            q[j] = partner[(n - 1 - i) * kPairLines];
+        }
+#pragma unroll
+        for (int j = 0; j < 2 * kPD - 1; ++j) {
+            if (base + j < n) {
+                const double o = recur(x[j]);
+                if (act) W[static_cast<long long>(base + j) * S] = narrow<DstT>(o + q[j]);
             }
         }
-    };
-    SrcT bufA[kPD], bufB[kPD];
-    load_block(bufA, 4);
-    for (int base = 4; base < n; base += 2 * kPD) {
-        load_block(bufB, base + kPD);
-        run_block(bufA, base);
-        load_block(bufA, base + 2 * kPD);
-        run_block(bufB, base + kPD);
-    }
-    // odd n: the middle element was parked by both lanes at step H-1
-    if ((n & 1) && role == 0 && act) {
-        const int mid = (n - 1) >> 1;
-        dst[s0 + static_cast<long long>(mid) * st] =
-            narrow<DstT>(mine[mid * kPairLines + li] + partner[mid * kPairLines + li]);
     }
 }
 
-template <typename SrcT, typename DstT>
-__global__ __launch_bounds__(64) void iir_pair_lines(const SrcT *__restrict__ src,
-                                                     DstT *__restrict__ dst, LineSet L, IirCoef k,
-                                                     int H) {
-    extern __shared__ double lds[];  // [2][H][32]: role, step, line
-    iir_pair_body<SrcT, DstT>(src, dst, L, k, H, blockIdx.x, lds);
+template <typename SrcT, typename DstT, bool ALONG0>
+__global__ __launch_bounds__(64, 2) void iir_pair_lines(const SrcT *__restrict__ src,
+                                                        DstT *__restrict__ dst, LineSet L, IirCoef k) {
+    extern __shared__ double lds[];  // [2][lds_steps][32]: role, step, line
+    iir_pair_body<SrcT, DstT, ALONG0>(src, dst, L, k, blockIdx.x, lds);
 }
 
 // Many volumes' lines along one axis in one launch: workgroup b takes
@@ -374,17 +491,16 @@ struct BatchLines {
     void *dst;
     LineSet L;
     IirCoef k;
-    int H;
     unsigned first_block;
 };
 
-template <typename SrcT, typename DstT>
-__global__ __launch_bounds__(64) void iir_pair_lines_batch(const BatchLines *__restrict__ vols,
-                                                           const int *__restrict__ vol_of) {
+template <typename SrcT, typename DstT, bool ALONG0>
+__global__ __launch_bounds__(64, 2) void iir_pair_lines_batch(const BatchLines *__restrict__ vols,
+                                                              const int *__restrict__ vol_of) {
     extern __shared__ double lds[];
     const BatchLines &v = vols[vol_of[blockIdx.x]];
-    iir_pair_body<SrcT, DstT>(static_cast<const SrcT *>(v.src), static_cast<DstT *>(v.dst), v.L, v.k,
-                              v.H, blockIdx.x - v.first_block, lds);
+    iir_pair_body<SrcT, DstT, ALONG0>(static_cast<const SrcT *>(v.src), static_cast<DstT *>(v.dst), v.L,
+                                      v.k, blockIdx.x - v.first_block, lds);
 }
 
 static LineSet lines_for(const sitkhip_geometry &g, int axis) {
@@ -413,6 +529,17 @@ static size_t max_lds_per_block() {
     return v;
 }
 
+// Whether the two-lane kernel takes lines of n voxels.
+static bool paired(size_t n) {
+    return n >= 8 && n < (1u << 30) && pair_lds_bytes(static_cast<int>(n)) <= max_lds_per_block();
+}
+// A kernel with more than 64 KB of dynamic LDS has to be told so.
+static void allow_lds(const void *kernel, size_t bytes) {
+    if (bytes > 64 * 1024)
+        HIP_OK(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   static_cast<int>(bytes)));
+}
+
 // tmp: an FP64 scratch volume the single-lane kernel needs for its causal
 // outputs (it may alias dst when DstT is double); the two-lane kernel, used
 // whenever its LDS fits, needs none.
@@ -421,15 +548,12 @@ static void launch_axis(const SrcT *src, double *tmp, DstT *dst, const sitkhip_g
                         const IirCoef &k) {
     LineSet L = lines_for(g, axis);
     static const char *names[3] = {"gauss_iir_axis0", "gauss_iir_axis1", "gauss_iir_axis2"};
-    const int H = (L.len + 1) / 2;
-    const size_t lds = static_cast<size_t>(2) * H * kPairLines * sizeof(double);
-    if (L.len >= 8 && lds <= max_lds_per_block()) {
-        unsigned blocks = static_cast<unsigned>((L.nlines + kPairLines - 1) / kPairLines);
-        if (lds > 64 * 1024)
-            HIP_OK(hipFuncSetAttribute(reinterpret_cast<const void *>(&iir_pair_lines<SrcT, DstT>),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize,
-                                       static_cast<int>(lds)));
-        launch_kernel(names[axis], iir_pair_lines<SrcT, DstT>, dim3(blocks), dim3(64), lds, src, dst, L, k, H);
+    if (paired(L.len)) {
+        const size_t lds = pair_lds_bytes(L.len);
+        const dim3 blocks(static_cast<unsigned>((L.nlines + kPairLines - 1) / kPairLines));
+        auto kernel = axis == 0 ? iir_pair_lines<SrcT, DstT, true> : iir_pair_lines<SrcT, DstT, false>;
+        allow_lds(reinterpret_cast<const void *>(kernel), lds);
+        launch_kernel(names[axis], kernel, blocks, dim3(64), lds, src, dst, L, k);
     } else {
         unsigned blocks = static_cast<unsigned>((L.nlines + 255) / 256);
         launch_kernel(names[axis], iir_lines<SrcT, DstT>, dim3(blocks), dim3(256), 0, src, tmp, dst, L, k);
@@ -565,39 +689,33 @@ static void recursive_gaussian_into(const Image &in, const double sigma[3], Imag
 }
 
 // ----------------------------------------------------------- batched volumes
-template <typename SrcT, typename DstT>
-static void launch_axis_batch(const std::vector<const SrcT *> &src, const std::vector<DstT *> &dst,
-                              const std::vector<const sitkhip_geometry *> &g,
-                              const std::vector<IirCoef> &k, int axis) {
-    const size_t n = src.size();
-    std::vector<BatchLines> hv(n);
-    std::vector<int> map;
-    int Hmax = 1;
-    unsigned blocks = 0;
-    for (size_t i = 0; i < n; ++i) {
-        BatchLines &v = hv[i];
-        v.src = src[i];
-        v.dst = dst[i];
-        v.L = lines_for(*g[i], axis);
-        v.k = k[i];
-        v.H = (v.L.len + 1) / 2;
-        v.first_block = blocks;
-        const unsigned nb = static_cast<unsigned>((v.L.nlines + kPairLines - 1) / kPairLines);
-        map.insert(map.end(), nb, static_cast<int>(i));
-        blocks += nb;
-        Hmax = std::max(Hmax, v.H);
+// One axis of a batch's smoothing: every volume's lines, and which volume each
+// workgroup takes.
+struct AxisBatch {
+    std::vector<BatchLines> vols;
+    std::vector<int> vol_of;
+    size_t lds = 0;
+    void add(const void *src, void *dst, const sitkhip_geometry &g, int axis, double sigma) {
+        BatchLines v;
+        v.src = src;
+        v.dst = dst;
+        v.L = lines_for(g, axis);
+        v.k = zero_order_coefficients(sigma / g.spacing[axis]);
+        v.first_block = static_cast<unsigned>(vol_of.size());
+        vol_of.insert(vol_of.end(), static_cast<size_t>((v.L.nlines + kPairLines - 1) / kPairLines),
+                      static_cast<int>(vols.size()));
+        lds = std::max(lds, pair_lds_bytes(v.L.len));
+        vols.push_back(v);
     }
-    const size_t lds = static_cast<size_t>(2) * Hmax * kPairLines * sizeof(double);
-    DeviceBuffer<BatchLines> dv(n);
-    DeviceBuffer<int> dmap(map.size());
-    dv.upload(hv.data(), n);
-    dmap.upload(map.data(), map.size());
+};
+
+template <typename SrcT, typename DstT>
+static void launch_axis_batch(const AxisBatch &b, const BatchLines *vols, const int *vol_of, int axis) {
     static const char *names[3] = {"gauss_iir_axis0", "gauss_iir_axis1", "gauss_iir_axis2"};
-    if (lds > 64 * 1024)
-        HIP_OK(hipFuncSetAttribute(reinterpret_cast<const void *>(&iir_pair_lines_batch<SrcT, DstT>),
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
-    launch_kernel(names[axis], iir_pair_lines_batch<SrcT, DstT>, dim3(blocks), dim3(64), lds,
-                  static_cast<const BatchLines *>(dv.ptr), static_cast<const int *>(dmap.ptr));
+    auto kernel = axis == 0 ? iir_pair_lines_batch<SrcT, DstT, true> : iir_pair_lines_batch<SrcT, DstT, false>;
+    allow_lds(reinterpret_cast<const void *>(kernel), b.lds);
+    launch_kernel(names[axis], kernel, dim3(static_cast<unsigned>(b.vol_of.size())), dim3(64), b.lds, vols,
+                  vol_of);
     check_launch(names[axis]);
 }
 
@@ -617,32 +735,40 @@ std::vector<Image *> recursive_gaussian_batch(const std::vector<const Image *> &
         auto flush = [&]() {
             if (group.empty()) return;
             std::vector<DeviceBuffer<double>> A(group.size()), B(group.size());
-            std::vector<const sitkhip_geometry *> g;
-            std::vector<IirCoef> k0, k1, k2;
-            std::vector<const float *> s0;
-            std::vector<double *> d0, d1;
-            std::vector<const double *> s1, s2;
-            std::vector<float *> d2;
+            AxisBatch axes[3];
             for (size_t j = 0; j < group.size(); ++j) {
                 const size_t i = group[j];
-                const sitkhip_geometry &gi = in[i]->geom;
+                const sitkhip_geometry &g = in[i]->geom;
                 A[j].alloc(in[i]->len());
                 B[j].alloc(in[i]->len());
-                out[i] = image_like(gi);
-                g.push_back(&gi);
-                k0.push_back(zero_order_coefficients(sigma[i][0] / gi.spacing[0]));
-                k1.push_back(zero_order_coefficients(sigma[i][1] / gi.spacing[1]));
-                k2.push_back(zero_order_coefficients(sigma[i][2] / gi.spacing[2]));
-                s0.push_back(in[i]->buf.ptr);
-                d0.push_back(A[j].ptr);
-                s1.push_back(A[j].ptr);
-                d1.push_back(B[j].ptr);
-                s2.push_back(B[j].ptr);
-                d2.push_back(out[i]->buf.ptr);
+                out[i] = image_like(g);
+                axes[0].add(in[i]->buf.ptr, A[j].ptr, g, 0, sigma[i][0]);
+                axes[1].add(A[j].ptr, B[j].ptr, g, 1, sigma[i][1]);
+                axes[2].add(B[j].ptr, out[i]->buf.ptr, g, 2, sigma[i][2]);
             }
-            launch_axis_batch<float, double>(s0, d0, g, k0, 0);
-            launch_axis_batch<double, double>(s1, d1, g, k1, 1);
-            launch_axis_batch<double, float>(s2, d2, g, k2, 2);
+            // the three axes' tables in one copy ahead of the three launches
+            // (volumes first: they hold pointers)
+            size_t at[3][2], bytes = 0;
+            for (int k = 0; k < 2; ++k)
+                for (int d = 0; d < 3; ++d) {
+                    at[d][k] = bytes;
+                    bytes += k == 0 ? axes[d].vols.size() * sizeof(BatchLines)
+                                    : axes[d].vol_of.size() * sizeof(int);
+                }
+            std::vector<unsigned char> host(bytes);
+            for (int d = 0; d < 3; ++d) {
+                std::memcpy(host.data() + at[d][0], axes[d].vols.data(),
+                            axes[d].vols.size() * sizeof(BatchLines));
+                std::memcpy(host.data() + at[d][1], axes[d].vol_of.data(),
+                            axes[d].vol_of.size() * sizeof(int));
+            }
+            DeviceBuffer<unsigned char> dev(bytes);
+            dev.upload(host.data(), bytes);
+            auto vols = [&](int d) { return reinterpret_cast<const BatchLines *>(dev.ptr + at[d][0]); };
+            auto vol_of = [&](int d) { return reinterpret_cast<const int *>(dev.ptr + at[d][1]); };
+            launch_axis_batch<float, double>(axes[0], vols(0), vol_of(0), 0);
+            launch_axis_batch<double, double>(axes[1], vols(1), vol_of(1), 1);
+            launch_axis_batch<double, float>(axes[2], vols(2), vol_of(2), 2);
             group.clear();
             group_bytes = 0;
         };
@@ -650,9 +776,7 @@ std::vector<Image *> recursive_gaussian_batch(const std::vector<const Image *> &
             const sitkhip_geometry &gi = in[i]->geom;
             bool ok = true;
             for (int d = 0; d < 3; ++d) {
-                if (!(sigma[i][d] > 0.0) || gi.size[d] < 8) ok = false;
-                const size_t lds = static_cast<size_t>(2) * ((gi.size[d] + 1) / 2) * kPairLines * sizeof(double);
-                if (lds > max_lds_per_block()) ok = false;
+                if (!(sigma[i][d] > 0.0) || !paired(gi.size[d])) ok = false;
             }
             if (!ok) {
                 out[i] = recursive_gaussian(*in[i], sigma[i].data(), false);
