@@ -56,6 +56,7 @@ struct PairDesc {
     long long tile;
     int kind;
     int ntiles;
+    ColumnTiles columns;  // mean squares walked by columns (blocks > 0): its tiles
 };
 
 struct PairControl {
@@ -135,7 +136,14 @@ __global__ __launch_bounds__(kBlock) SITKHIP_BATCH_OCC void batch_pass1(const Pa
             double acc[14];
 #pragma unroll
             for (int k = 0; k < 14; ++k) acc[k] = 0.0;
-            ms_range<R, true>(d.F, d.M, S, c.X, d.C, d.SS, d.fval, begin, end, acc);
+            if (sizeof(R) == 4 && d.columns.blocks) {
+                const unsigned k = static_cast<unsigned>(tl.index);
+                const int z0 = static_cast<int>(k / d.columns.blocks) * d.columns.zlen;
+                const int z1 = min(z0 + d.columns.zlen, static_cast<int>(d.F.size[2]));
+                ms_columns<true>(d.F, d.M, S, c.X, d.C, d.fval, k % d.columns.blocks, z0, z1, acc);
+            } else {
+                ms_range<R, true>(d.F, d.M, S, c.X, d.C, d.SS, d.fval, begin, end, acc);
+            }
             block_reduce_store<14>(acc, d.partials, static_cast<unsigned>(tl.index));
         }
         __syncthreads();  // the next tile reuses the LDS
@@ -288,7 +296,13 @@ static void build_tiles(BatchEngine &b) {
     std::vector<size_t> row_off(b.n);
     for (size_t i = 0; i < b.n; ++i) {
         const Metric &m = *b.metrics[i];
-        const int nt = static_cast<int>((m.nsamples + T - 1) / T);
+        int nt = static_cast<int>((m.nsamples + T - 1) / T);
+        b.hdesc[i].columns = ColumnTiles{0, 0, 0};
+        if (uses_columns(m)) {
+            b.hdesc[i].columns =
+                column_tiles(m.F, static_cast<int>(std::min<size_t>(T / kBlock, kColumnMax)));
+            nt = static_cast<int>(b.hdesc[i].columns.tiles);
+        }
         b.hdesc[i].tile = static_cast<long long>(T);
         b.hdesc[i].ntiles = nt;
         row_off[i] = rows;
@@ -528,9 +542,9 @@ static void read_outputs(BatchEngine &b, std::vector<BatchOutput> &out) {
             o.value = r.tail.value;
             o.valid = static_cast<size_t>(r.tail.valid);
             o.moments[12] = o.moments[13] = 0.0;
-            if (f32) moments_to_physical(b.metrics[i]->F, o.moments, o.moments + 3);
+            if (f32) moments_to_physical(b.metrics[i]->F, b.metrics[i]->Mv, o.moments, o.moments + 3);
         } else {
-            if (f32) moments_to_physical(b.metrics[i]->F, o.moments + 1, o.moments + 4);
+            if (f32) moments_to_physical(b.metrics[i]->F, b.metrics[i]->Mv, o.moments + 1, o.moments + 4);
             const double count = r.moments[13];
             o.valid = static_cast<size_t>(count);
             o.value = count == 0.0 ? DBL_MAX : r.moments[0] / count;

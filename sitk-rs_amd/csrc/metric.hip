@@ -90,6 +90,24 @@ __global__ __launch_bounds__(kBlock) void ms_pass(FixedGrid F, MovingVol M, Map 
     block_reduce_store<NS>(acc, partials, logical);
 }
 
+// One column tile per workgroup; XCD x (workgroup mod 8) takes the x-th eighth
+// of the tiles, whose workgroups walk neighbouring planes together.
+template <bool MOMENTS, typename Map>
+__global__ __launch_bounds__(kBlock) void ms_columns_pass(FixedGrid F, MovingVol M, Map S, IndexMap X,
+                                                          const ChainConst *__restrict__ C,
+                                                          const float *__restrict__ fval, ColumnTiles T,
+                                                          double *__restrict__ partials) {
+    const unsigned t = (blockIdx.x % 8u) * (gridDim.x / 8u) + blockIdx.x / 8u;
+    if (t >= T.tiles) return;
+    __shared__ double s_stage[kMaxStages * 12];
+    const auto V = stage_to_lds(S, s_stage);
+    const int z0 = static_cast<int>(t / T.blocks) * T.zlen;
+    const int z1 = min(z0 + T.zlen, static_cast<int>(F.size[2]));
+    double acc[MOMENTS ? 14 : 2];
+    ms_columns<MOMENTS>(F, M, V, X, C, fval, t % T.blocks, z0, z1, acc);
+    block_reduce_store<MOMENTS ? 14 : 2>(acc, partials, t);
+}
+
 // Pass 1: joint histogram (fixed point) + fixed-marginal counts; with REC
 // also the per-sample records for the derivative pass that follows.
 template <typename R, bool LDS, bool REC, typename Map, bool BSP = false>
@@ -1393,9 +1411,9 @@ static void launch_hist(Metric &m, const Stages &S, bool tail, bool clear = true
 static std::atomic<unsigned long long> g_eval_seq{0};
 
 template <int NS>
-static void launch_fold(Metric &m) {
+static void launch_fold(Metric &m, unsigned rows = kGrid) {
     m.seq = g_eval_seq.fetch_add(1) + 1;
-    launch_kernel("fold_partials", fold_partials<NS>, dim3(1), dim3(kBlock), 0, m.partials.ptr, kGrid,
+    launch_kernel("fold_partials", fold_partials<NS>, dim3(1), dim3(kBlock), 0, m.partials.ptr, rows,
                   m.res_dev->moments, &m.res_dev->done, m.seq);
     check_launch("fold_partials");
 }
@@ -1524,7 +1542,7 @@ void mattes_derivative_moments(Metric &m, const double *stages, int nstage, cons
     }
     sync();
     std::memcpy(moments, m.res->moments, 12 * sizeof(double));
-    if (m.precision == SITKHIP_PRECISION_F32) moments_to_physical(m.F, moments, moments + 3);
+    if (m.precision == SITKHIP_PRECISION_F32) moments_to_physical(m.F, m.Mv, moments, moments + 3);
 }
 
 static void value_pass(Metric &m, const Stages &S) {
@@ -1561,14 +1579,49 @@ void mattes_value_and_moments(Metric &m, const double *stages, int nstage, doubl
     const TailOut &t = m.res->tail;
     if (moments) {
         std::memcpy(moments, m.res->moments, 12 * sizeof(double));
-        if (m.precision == SITKHIP_PRECISION_F32) moments_to_physical(m.F, moments, moments + 3);
+        if (m.precision == SITKHIP_PRECISION_F32) moments_to_physical(m.F, m.Mv, moments, moments + 3);
     }
     if (value) *value = t.value;
     if (valid) *valid = static_cast<size_t>(t.valid);
 }
 
+// The column walk of a grid metric. Its tiles: as many planes each as make
+// about two kGrid workgroups (256^3: 59 us; one kGrid 61), at least the planes
+// of one step.
+template <bool MOM>
+static void launch_ms_columns(Metric &m, const Stages &S) {
+    constexpr int NS = MOM ? 14 : 2;
+    const ColumnTiles one = column_tiles(m.F, 1);
+    const ColumnTiles T =
+        column_tiles(m.F, std::max(kColumnU, static_cast<int>((one.tiles + 2 * kGrid - 1) / (2 * kGrid))));
+    const size_t need = static_cast<size_t>(T.tiles) * NS;
+    if (m.partials.len < need) m.partials.alloc(need);
+    const IndexMap X = make_index_map(m.F, m.Mv, S.s, S.n);
+    const dim3 grid((T.tiles + 7) / 8 * 8);
+    const char *name = MOM ? "ms_moments" : "ms_value";
+    auto go = [&](const auto &map) {
+        using Map = std::decay_t<decltype(map)>;
+        launch_kernel(name, ms_columns_pass<MOM, Map>, grid, dim3(kBlock), 0, m.F, m.Mv, map, X,
+                      static_cast<const ChainConst *>(m.chain.ptr), static_cast<const float *>(m.fval.ptr), T,
+                      m.partials.ptr);
+    };
+    if (S.n == 1) {
+        OneStage one_stage;
+        std::memcpy(one_stage.m, S.s, sizeof(one_stage.m));
+        go(one_stage);
+    } else {
+        go(S);
+    }
+    check_launch("ms_columns_pass");
+    launch_fold<NS>(m, T.tiles);
+}
+
 template <typename R, bool MOM>
 static void launch_ms(Metric &m, const Stages &S) {
+    if (uses_columns(m)) {
+        launch_ms_columns<MOM>(m, S);
+        return;
+    }
     {
         const char *name = MOM ? "ms_moments" : "ms_value";
         const IndexMap X = make_index_map(m.F, m.Mv, S.s, S.n);
@@ -1594,7 +1647,7 @@ void ms_moments(Metric &m, const double *stages, int nstage, double out[14]) {
     else launch_ms<float, true>(m, S);
     wait_done(m);
     std::memcpy(out, m.res->moments, 14 * sizeof(double));
-    if (m.precision == SITKHIP_PRECISION_F32) moments_to_physical(m.F, out + 1, out + 4);
+    if (m.precision == SITKHIP_PRECISION_F32) moments_to_physical(m.F, m.Mv, out + 1, out + 4);
 }
 
 void ms_value(Metric &m, const double *stages, int nstage, double *sq, size_t *valid) {

@@ -475,16 +475,40 @@ __device__ __forceinline__ void moment_point(const FixedGrid &F, const ChainCons
     }
 }
 
-// Index-space first/second moments -> physical: `a` the 3 first moments, `b`
-// the 3 x 3 second moments [d][c] (rewritten in place as [d][e]).
-inline void moments_to_physical(const FixedGrid &F, const double *a, double *b) {
-    double out[9];
+// The gradient that the moment sums weight by: FP64 path, the physical one
+// per sample as the reference; FP32 path, the index-space gradient itself (the
+// map to physical axes is linear, so the host applies it once to the sums).
+template <typename R>
+__device__ __forceinline__ void moment_gradient(const MovingVol &M, const R gi[3], R g[3]) {
+    if constexpr (sizeof(R) == 4) {
+#pragma unroll
+        for (int d = 0; d < 3; ++d) g[d] = gi[d];
+    } else {
+        physical_gradient<R>(M, gi, g);
+    }
+}
+
+// The FP32 path's moments -> physical: `a` the 3 first moments, `b` the 3 x 3
+// second moments [d][c], d the moving index axes and c the fixed ones, both
+// rewritten in place with d the physical gradient's axes and [d][e] the
+// physical point's.
+inline void moments_to_physical(const FixedGrid &F, const MovingVol &M, double *a, double *b) {
+    double g[3], h[9], out[9];
+    for (int d = 0; d < 3; ++d) {
+        g[d] = 0.0;
+        for (int c = 0; c < 3; ++c) h[d * 3 + c] = 0.0;
+        for (int j = 0; j < 3; ++j) {
+            g[d] += M.p2i[j * 3 + d] * a[j];
+            for (int c = 0; c < 3; ++c) h[d * 3 + c] += M.p2i[j * 3 + d] * b[j * 3 + c];
+        }
+    }
     for (int d = 0; d < 3; ++d)
         for (int e = 0; e < 3; ++e) {
-            double acc = F.origin[e] * a[d];
-            for (int c = 0; c < 3; ++c) acc += F.i2p[e * 3 + c] * b[d * 3 + c];
+            double acc = F.origin[e] * g[d];
+            for (int c = 0; c < 3; ++c) acc += F.i2p[e * 3 + c] * h[d * 3 + c];
             out[d * 3 + e] = acc;
         }
+    for (int i = 0; i < 3; ++i) a[i] = g[i];
     for (int i = 0; i < 9; ++i) b[i] = out[i];
 }
 
@@ -605,7 +629,7 @@ __device__ __forceinline__ void ms_range(const FixedGrid &F, const MovingVol &M,
             if constexpr (MOMENTS) {
                 double x[3];
                 moment_point<R, MapTraits<Map>::points>(F, C, b.flat[u], x);
-                physical_gradient<R>(M, gi, g);
+                moment_gradient<R>(M, gi, g);
 #pragma unroll
                 for (int d = 0; d < 3; ++d) {
                     const double dg = diff * static_cast<double>(g[d]);
@@ -620,6 +644,201 @@ __device__ __forceinline__ void ms_range(const FixedGrid &F, const MovingVol &M,
             }
         }
     }
+}
+
+// Mean squares over every voxel of the fixed grid, FP32, an affine point map:
+// a lane keeps its in-plane voxel (block * kBlock + lane) and walks the planes
+// [z0, z1), at most kColumnMax of them. Against ms_range's walk of the flat
+// grid this needs no index split, 3 FMAs of the composed map instead of 9, and
+// of the second moments only the z one per sample (x and y are the lane's
+// constants; Sum z dg comes from the running sum of S0: with K steps,
+// Sum_k (K - k) dg_k = Sum over steps of S0 after the step).
+// A wave whose samples all lie in interior cells of the moving volume takes no
+// clamps, boundary selects or inside tests; one with a face cell among them
+// takes those too. Samples within kGuard of a decision boundary are marked in a
+// bit mask and run the exact chain after the walk, which keeps its registers
+// out of the loop. The guard is tested on the float fraction f: | |f - 1/2| -
+// 1/4 | <= 1/4 - kGuard keeps f at least kGuard less one float rounding (6e-8)
+// from 0, 1/2 and 1, still 10^5 times the composed map's error.
+constexpr int kColumnMax = 64;
+constexpr int kColumnU = 2;  // planes whose loads are in flight together (one: 68 us, 256^3)
+
+template <bool MOMENTS, typename Map>
+__device__ __forceinline__ void ms_columns(const FixedGrid &F, const MovingVol &M, const Map &S,
+                                           const IndexMap &X, const ChainConst *__restrict__ C,
+                                           const float *__restrict__ fval, unsigned block, int z0,
+                                           int z1, double (&acc)[MOMENTS ? 14 : 2]) {
+    const unsigned nx = F.size[0], plane = nx * F.size[1];
+    const unsigned p = block * kBlock + threadIdx.x;
+    const bool live = p < plane;
+    const unsigned pc = live ? p : 0u;
+    const unsigned iy = fdiv(pc, F.div0), ix = pc - iy * nx;
+    const double dx = static_cast<double>(ix), dy = static_cast<double>(iy);
+    double cxy[3];
+#pragma unroll
+    for (int r = 0; r < 3; ++r)
+        cxy[r] = fma(X.A[r * 3 + 1], dy, fma(X.A[r * 3 + 0], dx, X.b[r]));
+    const unsigned s1 = static_cast<unsigned>(M.stride1), s2 = static_cast<unsigned>(M.stride2);
+    const unsigned n0 = M.size[0], n1 = M.size[1], n2 = M.size[2];
+    double sq = 0.0, s[3] = {0.0, 0.0, 0.0}, run[3] = {0.0, 0.0, 0.0};
+    unsigned count = 0;
+    unsigned long long later = 0;  // steps left to the exact chain
+    double dz = static_cast<double>(z0);
+    int steps = 0;
+    for (int z = z0; z < z1; z += kColumnU, steps += kColumnU) {
+        float f[kColumnU][3], fv[kColumnU];
+        FloatPair q[kColumnU][4];
+        int bx[kColumnU];
+        bool use[kColumnU], faces[kColumnU];  // faces: the same for the whole wave
+#pragma unroll
+        for (int u = 0; u < kColumnU; ++u) {
+            int base[3];
+            bool sure = true;  // (false for a NaN map: the chain drops the sample)
+#pragma unroll
+            for (int r = 0; r < 3; ++r) {
+                const double c = fma(X.A[r * 3 + 2], dz, cxy[r]);
+                const double fl = floor(c);
+                base[r] = static_cast<int>(fl);
+                f[u][r] = static_cast<float>(c - fl);
+                sure = sure && fabsf(fabsf(f[u][r] - 0.5f) - 0.25f) <= 0.25f - static_cast<float>(kGuard);
+            }
+            dz += 1.0;
+            const bool in = live && z + u < z1;
+            const bool inner = static_cast<unsigned>(base[0]) < n0 - 1u &&
+                               static_cast<unsigned>(base[1]) < n1 - 1u &&
+                               static_cast<unsigned>(base[2]) < n2 - 1u;
+            // cells that a sample inside the volume may have: -1 .. n - 1
+            const bool near = static_cast<unsigned>(base[0]) + 1u <= n0 &&
+                              static_cast<unsigned>(base[1]) + 1u <= n1 &&
+                              static_cast<unsigned>(base[2]) + 1u <= n2;
+            if (in && near && !sure) later |= 1ull << (steps + u);
+            use[u] = in && inner && sure;
+            bx[u] = base[0];
+            unsigned t1 = s1, t2 = s2;
+            faces[u] = __any(in && near && sure && !inner);
+            if (faces[u]) {
+                // inside: the nearest voxel exists on every axis
+                bool inside = in && near && sure;
+#pragma unroll
+                for (int r = 0; r < 3; ++r)
+                    inside = inside && static_cast<unsigned>(base[r] + (f[u][r] >= 0.5f ? 1 : 0)) <
+                                           static_cast<unsigned>(M.size[r]);
+                use[u] = inside;
+                // past a face both neighbours are the face's voxel
+                t1 = static_cast<unsigned>(base[1]) < n1 - 1u ? s1 : 0u;
+                t2 = static_cast<unsigned>(base[2]) < n2 - 1u ? s2 : 0u;
+                base[0] = min(max(base[0], 0), static_cast<int>(n0) - 2);
+                base[1] = max(base[1], 0);
+                base[2] = max(base[2], 0);
+            }
+            const unsigned off = use[u] ? static_cast<unsigned>(base[0]) + static_cast<unsigned>(base[1]) * s1 +
+                                              static_cast<unsigned>(base[2]) * s2
+                                        : 0u;
+            const float *v = M.vol + off;
+            q[u][0] = *reinterpret_cast<const FloatPair *>(v);
+            q[u][1] = *reinterpret_cast<const FloatPair *>(v + t1);
+            q[u][2] = *reinterpret_cast<const FloatPair *>(v + t2);
+            q[u][3] = *reinterpret_cast<const FloatPair *>(v + (t1 + t2));
+            const unsigned zc = static_cast<unsigned>(z + u < z1 ? z + u : z);
+            fv[u] = fval[static_cast<size_t>(zc) * plane + pc];
+            if (M.mask && use[u]) {
+                // round half up: the guard keeps the fraction off 1/2 (in a face
+                // cell along x the clamped base is not the cell's)
+                const size_t at =
+                    static_cast<size_t>(bx[u] + (f[u][0] >= 0.5f ? 1 : 0)) +
+                    static_cast<size_t>(base[1] + (t1 && f[u][1] >= 0.5f ? 1 : 0)) * s1 +
+                    static_cast<size_t>(base[2] + (t2 && f[u][2] >= 0.5f ? 1 : 0)) * s2;
+                use[u] = M.mask[at] != 0;
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < kColumnU; ++u) {
+            if (use[u]) {
+                float v[8] = {q[u][0].a, q[u][0].b, q[u][1].a, q[u][1].b,
+                              q[u][2].a, q[u][2].b, q[u][3].a, q[u][3].b};
+                if (faces[u]) {
+                    const bool lo = bx[u] < 0, hi = bx[u] == static_cast<int>(n0) - 1;
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        const float a = v[2 * k], b = v[2 * k + 1];
+                        v[2 * k] = hi ? b : a;
+                        v[2 * k + 1] = lo ? a : b;
+                    }
+                }
+                float mv, gi[3];
+                Trilinear<float>::template eval<MOMENTS>(f[u], v, mv, gi);
+                const double diff = static_cast<double>(mv) - static_cast<double>(fv[u]);
+                sq = fma(diff, diff, sq);
+                ++count;
+                if constexpr (MOMENTS) {
+#pragma unroll
+                    for (int d = 0; d < 3; ++d) s[d] = fma(diff, static_cast<double>(gi[d]), s[d]);
+                }
+            }
+            if constexpr (MOMENTS) {
+#pragma unroll
+                for (int d = 0; d < 3; ++d) run[d] += s[d];
+            }
+        }
+    }
+    // Sum z dg = (z0 + steps) S0 - run
+    double sz[3];
+#pragma unroll
+    for (int d = 0; d < 3; ++d) sz[d] = fma(static_cast<double>(z0 + steps), s[d], -run[d]);
+    while (later) {
+        const int k = __ffsll(static_cast<long long>(later)) - 1;
+        later &= later - 1ull;
+        const unsigned flat = static_cast<unsigned>(z0 + k) * plane + p;
+        double x[3], pt[3];
+        Cell cell;
+        fixed_point(F, *C, flat, x);
+        map_point(S, x, pt);
+        if (!locate(M, *C, pt, cell)) continue;
+        float fr[3], v[8], mv, gi[3];
+#pragma unroll
+        for (int d = 0; d < 3; ++d) fr[d] = static_cast<float>(cell.frac[d]);
+        corners(M, cell, v);
+        Trilinear<float>::template eval<MOMENTS>(fr, v, mv, gi);
+        const double diff = static_cast<double>(mv) - static_cast<double>(fval[flat]);
+        sq = fma(diff, diff, sq);
+        ++count;
+        if constexpr (MOMENTS) {
+#pragma unroll
+            for (int d = 0; d < 3; ++d) {
+                const double dg = diff * static_cast<double>(gi[d]);
+                s[d] += dg;
+                sz[d] = fma(dg, static_cast<double>(z0 + k), sz[d]);
+            }
+        }
+    }
+    acc[0] = sq;
+    if constexpr (MOMENTS) {
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            acc[1 + d] = s[d];
+            acc[4 + d * 3] = dx * s[d];
+            acc[5 + d * 3] = dy * s[d];
+            acc[6 + d * 3] = sz[d];
+        }
+        acc[13] = static_cast<double>(count);
+    } else {
+        acc[1] = static_cast<double>(count);
+    }
+}
+
+// How a grid is cut into column tiles: `blocks` of kBlock in-plane voxels by
+// ceil(nz / zlen) runs of planes, the runs outermost.
+struct ColumnTiles {
+    unsigned blocks, tiles;
+    int zlen;
+};
+inline ColumnTiles column_tiles(const FixedGrid &F, int zlen) {
+    ColumnTiles t;
+    const size_t plane = static_cast<size_t>(F.size[0]) * F.size[1];
+    t.zlen = zlen < 1 ? 1 : (zlen > kColumnMax ? kColumnMax : zlen);
+    t.blocks = static_cast<unsigned>((plane + kBlock - 1) / kBlock);
+    t.tiles = t.blocks * ((F.size[2] + static_cast<unsigned>(t.zlen) - 1) / static_cast<unsigned>(t.zlen));
+    return t;
 }
 
 // What the value pass leaves per sample for a derivative pass that follows it
@@ -780,7 +999,7 @@ __device__ __forceinline__ void deriv_range(const FixedGrid &F, const MovingVol 
             R mv, gi[3], g[3];
             Interp<R, BSP>::template eval<true>(M, L.base[u], L.fr[u], L.v[u], mv, gi);
             if (!Parzen<R>::in_range(P, mv)) continue;
-            physical_gradient<R>(M, gi, g);
+            moment_gradient<R>(M, gi, g);
             R arg[4], dv[4];
             bool mid;
             const int m0 = Parzen<R>::taps(P, mv, arg, mid);
@@ -851,7 +1070,7 @@ __device__ __forceinline__ void deriv_records(const FixedGrid &F, const MovingVo
         for (int u = 0; u < kRecU; ++u) {
             if (q.fb[u] == kNoBin || isnan(q.r[u].mv)) continue;
             R g[3];
-            physical_gradient<R>(M, q.r[u].gi, g);
+            moment_gradient<R>(M, q.r[u].gi, g);
             R arg[4], dv[4];
             bool mid;
             const int m0 = Parzen<R>::taps(P, q.r[u].mv, arg, mid);
@@ -1250,6 +1469,14 @@ struct Metric {
     size_t nsamples = 0;
     size_t voxels_fixed = 0;
 };
+
+// Whether the mean-squares evaluation walks columns (ms_columns): every voxel
+// of a grid, FP32, linear interpolation, a moving volume whose cells have an
+// interior on every axis.
+inline bool uses_columns(const Metric &m) {
+    return m.kind == SITKHIP_METRIC_MEAN_SQUARES && m.precision == SITKHIP_PRECISION_F32 && !m.SS.idx &&
+           !m.F.pts && !m.bspline && m.Mv.size[0] >= 2 && m.Mv.size[1] >= 2 && m.Mv.size[2] >= 2;
+}
 
 // The Mattes tail of metric m into `out` (one workgroup; metric.hip).
 void launch_tail(Metric &m, TailOut *out, bool clear = true);
