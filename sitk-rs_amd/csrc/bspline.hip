@@ -187,11 +187,11 @@ __device__ __forceinline__ void stage_cell_coefs(const BSplineMap &B, int cell, 
 }
 
 // map_point for a sample of a cell: the stored support weights ws (w0, w1,
-// w2; 12 doubles) and the cell's coefficients from LDS, the same sums in the
+// w2; 12 doubles, `n` apart) and the cell's coefficients from LDS, the same sums in the
 // same order as the general map; a sample of the outside bucket maps to
 // itself. Then the stage, if any.
 __device__ __forceinline__ void map_point_cell(const BSplineMap &B, const double x[3], bool in_cell,
-                                               const double *__restrict__ ws, const double *sc,
+                                               const double *__restrict__ ws, size_t n, const double *sc,
                                                double p[3]) {
     if (!in_cell) {
         p[0] = x[0]; p[1] = x[1]; p[2] = x[2];
@@ -200,14 +200,14 @@ __device__ __forceinline__ void map_point_cell(const BSplineMap &B, const double
     }
     double w2[4];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) w2[k] = ws[8 + k];
+    for (int k = 0; k < 4; ++k) w2[k] = ws[(8 + k) * n];
     // (w0[i] w1[j]) once per sample, then one k-slab (48 LDS reads) unrolled
     // so the reads are issued ahead of the dependent sums
     double w01[16];
 #pragma unroll
     for (int j = 0; j < 4; ++j)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) w01[j * 4 + i] = ws[i] * ws[4 + j];
+        for (int i = 0; i < 4; ++i) w01[j * 4 + i] = ws[i * n] * ws[(4 + j) * n];
     double d0 = 0.0, d1 = 0.0, d2 = 0.0;
 #pragma unroll 1
     for (int k = 0; k < 4; ++k)
@@ -228,12 +228,14 @@ __device__ __forceinline__ void map_point_cell(const BSplineMap &B, const double
 }
 
 // The support weights of every sample of a cell (they depend only on the
-// fixed point): w[12] per sample in the cell-grouped order, computed once.
+// fixed point), computed once: w[k][s], twelve planes of the n samples in the
+// cell-grouped order, so that a wave reads each as one run (twelve together per
+// sample spread a wave's load over 48 cache lines).
 // A sample whose support on the device is not its cell's (the grouping was
 // made on the host) raises *mismatch.
 __global__ void bs_weights(FixedGrid F, BSplineMap B, const ChainConst *__restrict__ C,
                            const uint32_t *__restrict__ idx, const int *__restrict__ cell_begin,
-                           int ncells, double *__restrict__ wts, int *__restrict__ mismatch) {
+                           int ncells, size_t n, double *__restrict__ wts, int *__restrict__ mismatch) {
     const int cell = blockIdx.y;
     const int m0 = B.gs[0] - 3, m1 = B.gs[1] - 3;
     const int sx = cell % m0, sy = (cell / m0) % m1, sz = cell / (m0 * m1);
@@ -248,7 +250,7 @@ __global__ void bs_weights(FixedGrid F, BSplineMap B, const ChainConst *__restri
 #pragma unroll
         for (int d = 0; d < 3; ++d)
 #pragma unroll
-            for (int k = 0; k < 4; ++k) wts[static_cast<size_t>(s) * 12 + d * 4 + k] = w[d][k];
+            for (int k = 0; k < 4; ++k) wts[(d * 4 + k) * n + s] = w[d][k];
     }
 }
 
@@ -293,7 +295,7 @@ __global__ __launch_bounds__(kBlock) void bs_value(FixedGrid F, MovingVol M, BSp
             if (fb != kNoBin) {
                 double x[3], p[3];
                 fixed_point(F, *C, idx[s], x);
-                map_point_cell(B, x, cell < ncells, wts + static_cast<size_t>(s) * 12, s_coef, p);
+                map_point_cell(B, x, cell < ncells, wts + s, static_cast<size_t>(n), s_coef, p);
                 ok = locate(M, *C, p, cl);
             }
             if (!ok) {
@@ -306,6 +308,192 @@ __global__ __launch_bounds__(kBlock) void bs_value(FixedGrid F, MovingVol M, BSp
             float v[8];
             corners(M, cl, v);
             hist_sample<R, true>(P, h_joint, h_marg, r, s, ok, fb, fr, v);
+        }
+    }
+    __syncthreads();
+    const unsigned copy = (blockIdx.y * gridDim.x + blockIdx.x) % kHistCopies;
+    g_joint += (static_cast<size_t>(st) * kHistCopies + copy) * P.bins * P.bins;
+    g_marg += (static_cast<size_t>(st) * kHistCopies + copy) * P.bins;
+    for (int i = threadIdx.x; i < nb; i += kBlock) {
+        const unsigned long long v = s_hist[i];
+        if (v) atomicAdd(i < P.bins * P.bins ? g_joint + i : g_marg + (i - P.bins * P.bins), v);
+    }
+}
+
+// What an FP32 evaluation composes on the host for one start: the affine part of
+// the map from the fixed index to the moving continuous index (the moving-
+// initial stage included) and Q = P M, which takes a B-spline displacement to
+// index space (P the moving physical-to-index matrix, M the stage's): the
+// moving index of fixed voxel i with displacement u is X.A i + X.b + Q u.
+struct CellMap {
+    IndexMap X;
+    double Q[9];
+};
+
+// The FP32 path's value pass: the same cells, histogram and records, the
+// displacement and the index composed with fused multiply-adds, two samples per
+// lane. The displacement is summed along x, then y, then z (252 FMAs instead of
+// 64 weight products and 192 rounded multiply-adds), and a cell's coefficients
+// come as scalar loads -- a multiply-add takes one operand from a scalar
+// register -- where LDS broadcasts took 192 reads per sample. A sample whose
+// composed index lies within kGuard of a decision boundary runs the reference's
+// chain on the coefficients in LDS (every sample does where the map puts voxels
+// on voxels, as zero coefficients on equal grids do). With few starts a cell's
+// samples are shared by `parts` workgroups (an integer histogram does not depend
+// on it). 64 starts of 707,788 samples on 7^3 cells: 1,363 us before, 1,240 now;
+// one start 53, now 47. The vector pipes issue 54 % of that time and the texture
+// path is busy 65 % (the eight corners of 64 scattered samples); 230 registers
+// leave two waves per SIMD. One sample per lane: 1,290 us at three waves (and 41
+// for one start); a bound of three waves on two samples spills: 2,076.
+constexpr int kCellU = 2;
+// Displacement in moving voxels below which the composed sum's rounding (some
+// 20 FP64 roundings of terms up to 3 kFar: 1e-7) stays under kGuard.
+constexpr double kFar = 16777216.0;
+
+__global__ __launch_bounds__(kBlock) void bs_value_f32(
+    FixedGrid F, MovingVol M, BSplineMap B0, const double *__restrict__ coef,
+    const double *__restrict__ stage, const CellMap *__restrict__ maps, CellMap own,
+    const int *__restrict__ active, const ChainConst *__restrict__ C, const uint32_t *__restrict__ idx,
+    const uint8_t *__restrict__ fbin, const int *__restrict__ cell_begin, const double *__restrict__ wts,
+    int ncells, int cpb, int parts, MattesParams P, unsigned long long *__restrict__ g_joint,
+    unsigned long long *__restrict__ g_marg, SampleRec<float> *__restrict__ rec, long long n) {
+    extern __shared__ unsigned long long s_hist[];
+    __shared__ double s_coef[192];
+    const int st = active[blockIdx.x];
+    const BSplineMap B = start_map(B0, coef, stage, st);
+    const CellMap cm = maps ? maps[st] : own;
+    const int nb = P.bins * P.bins + P.bins;
+    unsigned long long *h_joint = s_hist, *h_marg = s_hist + P.bins * P.bins;
+    SampleRec<float> *r = rec + static_cast<size_t>(st) * n;
+    for (int i = threadIdx.x; i < nb; i += kBlock) s_hist[i] = 0ull;
+    const int group = blockIdx.y / parts, part = blockIdx.y % parts;
+    const int g0 = B0.gs[0], g01 = B0.gs[0] * B0.gs[1], m0 = B0.gs[0] - 3, m1 = B0.gs[1] - 3;
+    double qmax = 0.0;
+    for (int k = 0; k < 9; ++k) qmax = fmax(qmax, fabs(cm.Q[k]));
+    for (int q = 0; q < cpb; ++q) {
+        const int cell = group * cpb + q;
+        if (cell > ncells) break;  // the same for every lane
+        __syncthreads();           // the previous cell's coefficients are no longer read
+        // displacements so large that the composed sum's rounding could pass
+        // kGuard (or not numbers): every sample of the cell takes the chain
+        bool far = false;
+        if (cell < ncells) {
+            stage_cell_coefs(B, cell, s_coef);
+            if (threadIdx.x < 192) far = !(fabs(s_coef[threadIdx.x]) * qmax < kFar);
+        }
+        const double unsure = __syncthreads_or(far) ? static_cast<double>(NAN) : 0.0;
+        const int cb = cell_begin[cell], ce = cell_begin[cell + 1];
+        const int len = (ce - cb + parts - 1) / parts;
+        const int b = cb + part * len, e = min(b + len, ce);
+        // read-only for the whole launch: constant address space, scalar loads
+        typedef const __attribute__((address_space(4))) double *ConstPtr;
+        const ConstPtr cf = (ConstPtr)(coef + static_cast<size_t>(st) * 3 * B0.ncp + cell % m0 +
+                                       g0 * ((cell / m0) % m1) + static_cast<size_t>(g01) * (cell / (m0 * m1)));
+        for (int s0 = b + threadIdx.x; s0 < e; s0 += kBlock * kCellU) {
+            // (opaque, so that the coefficients are read again each round as
+            // scalar loads: hoisted out of the loop they fill the registers)
+            int again = 0;
+            asm volatile("" : "+s"(again));
+            uint32_t flat[kCellU];
+            int fb[kCellU];
+            double c[kCellU][3];
+#pragma unroll
+            for (int u = 0; u < kCellU; ++u) {
+                const int s = s0 + u * kBlock < e ? s0 + u * kBlock : s0;
+                flat[u] = idx[s];
+                fb[u] = fbin[s];
+                uint32_t i0, i1, i2;
+                split_index(F, flat[u], i0, i1, i2);
+                const double d0 = i0, d1 = i1, d2 = i2;
+#pragma unroll
+                for (int k = 0; k < 3; ++k)
+                    c[u][k] = fma(cm.X.A[k * 3 + 2], d2,
+                                  fma(cm.X.A[k * 3 + 1], d1, fma(cm.X.A[k * 3 + 0], d0, cm.X.b[k])));
+            }
+            if (cell < ncells) {
+                double w[kCellU][12], D[kCellU][3];
+#pragma unroll
+                for (int u = 0; u < kCellU; ++u) {
+                    const int s = s0 + u * kBlock < e ? s0 + u * kBlock : s0;
+#pragma unroll
+                    for (int k = 0; k < 12; ++k) w[u][k] = wts[static_cast<size_t>(k) * n + s];
+#pragma unroll
+                    for (int d = 0; d < 3; ++d) D[u][d] = unsure;
+                }
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    double t[kCellU][3];
+#pragma unroll
+                    for (int u = 0; u < kCellU; ++u)
+#pragma unroll
+                        for (int d = 0; d < 3; ++d) t[u][d] = 0.0;
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+#pragma unroll
+                        for (int d = 0; d < 3; ++d) {
+                            const ConstPtr row = cf + again + d * B0.ncp + (j * g0 + k * g01);
+                            const double x0 = row[0], x1 = row[1], x2 = row[2], x3 = row[3];
+#pragma unroll
+                            for (int u = 0; u < kCellU; ++u) {
+                                const double rx =
+                                    fma(w[u][3], x3, fma(w[u][2], x2, fma(w[u][1], x1, w[u][0] * x0)));
+                                t[u][d] = fma(w[u][4 + j], rx, t[u][d]);
+                            }
+                        }
+#pragma unroll
+                    for (int u = 0; u < kCellU; ++u)
+#pragma unroll
+                        for (int d = 0; d < 3; ++d) D[u][d] = fma(w[u][8 + k], t[u][d], D[u][d]);
+                }
+#pragma unroll
+                for (int u = 0; u < kCellU; ++u)
+#pragma unroll
+                    for (int k = 0; k < 3; ++k)
+                        c[u][k] = fma(cm.Q[k * 3 + 2], D[u][2],
+                                      fma(cm.Q[k * 3 + 1], D[u][1], fma(cm.Q[k * 3 + 0], D[u][0], c[u][k])));
+            }
+#pragma unroll
+            for (int u = 0; u < kCellU; ++u) {
+                const int s = s0 + u * kBlock;
+                if (s >= e) continue;
+                Cell cl;
+                bool sure = true, ok = true;
+#pragma unroll
+                for (int k = 0; k < 3; ++k) {
+                    const double fl = floor(c[u][k]);
+                    cl.base[k] = static_cast<int>(fl);
+                    cl.frac[k] = c[u][k] - fl;
+                    // kGuard from every integer and half-integer, on the float
+                    // fraction (ms_columns); false for NaN
+                    const float f = static_cast<float>(cl.frac[k]);
+                    sure = sure && fabsf(fabsf(f - 0.5f) - 0.25f) <= 0.25f - static_cast<float>(kGuard);
+                    ok = ok && c[u][k] >= -0.5 && c[u][k] < static_cast<double>(M.size[k]) - 0.5;
+                }
+                if (!sure) {
+                    double x[3], p[3];
+                    fixed_point(F, *C, flat[u], x);
+                    map_point_cell(B, x, cell < ncells, wts + s, static_cast<size_t>(n), s_coef, p);
+                    ok = locate(M, *C, p, cl);
+                } else if (ok && M.mask) {
+                    // round half up of an inside point is a voxel
+                    size_t at = 0;
+#pragma unroll
+                    for (int k = 0; k < 3; ++k)
+                        at += static_cast<size_t>(cl.base[k] + (cl.frac[k] >= 0.5 ? 1 : 0)) *
+                              static_cast<size_t>(k == 0 ? 1 : (k == 1 ? M.stride1 : M.stride2));
+                    ok = M.mask[at] != 0;
+                }
+                ok = ok && fb[u] != kNoBin;
+                if (!ok) {
+                    cl.base[0] = cl.base[1] = cl.base[2] = 0;
+                    cl.frac[0] = cl.frac[1] = cl.frac[2] = 0.0;
+                }
+                float fr[3], v[8];
+#pragma unroll
+                for (int d = 0; d < 3; ++d) fr[d] = static_cast<float>(cl.frac[d]);
+                corners(M, cl, v);
+                hist_sample<float, true>(P, h_joint, h_marg, r, s, ok, fb[u], fr, v);
+            }
         }
     }
     __syncthreads();
@@ -334,8 +522,8 @@ __global__ __launch_bounds__(kTail) void bs_tail(const int *__restrict__ active,
                       pratio + st * nb, pratio_f + st * nb, tail + st, s_fold);
 }
 
-// Derivative pass, one workgroup per (cell, start), from the value pass's
-// records: per valid sample the pRatio-weighted B3' sum a times the moving
+// Derivative pass, one workgroup per (part of a cell, start), from the value
+// pass's records: per valid sample the pRatio-weighted B3' sum a times the moving
 // gradient (through the stage's transposed matrix when there is one), g_d;
 // then out[cell][16 n + m] = sum over the cell's samples of u_m t_n with
 // u_m = w0[m % 4] w1[m / 4] and t_n = g_{n / 4} w2[n % 4] (n < 12), i.e.
@@ -343,125 +531,174 @@ __global__ __launch_bounds__(kTail) void bs_tail(const int *__restrict__ active,
 // is a 16 x 4 by 4 x 16 FP64 matrix product per four samples
 // (v_mfma_f64_16x16x4f64): each lane stages its sample's weights and g in
 // LDS, then lane l feeds A[l % 16][l / 16] = u and B[l / 16][l % 16] = t of
-// sample 4 r + l / 16. The four waves' tiles are added in a fixed order.
+// sample 4 r + l / 16. The four waves' tiles are added in a fixed order. A
+// cell's samples are cut into `parts` (fixed for the metric, so a start's sums do
+// not depend on its batch). FP32: g is Q' times the record's index gradient.
+// A lane's sixteen LDS values lie 17 apart (16 apart, every lane's store of one
+// value hit the same two banks), a wave reads only its own rows, so that waves
+// go on without a barrier, and the next samples' record and weights are loaded
+// before the products of these. 64 starts of 707,788 samples on 7^3 cells: 1,196
+// us before, 903 with the padding and Q', 863 with pRatio in LDS, 805 without
+// barriers and branches in the products, 767 with the loads ahead: LDS is active
+// 72 % of the time and the matrix cores 44 %. One start: 41, now 24 (the parts).
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 static_assert(kBlock == 256, "the derivative pass adds four waves' tiles");
+// pRatio up to this size goes to LDS: the samples' tables of 34 KB leave it that
+// much with four workgroups on a compute unit.
+constexpr size_t kRatioLds = 6144;
+// A wave's own LDS rows, written and then read by its lanes: the wave's LDS
+// operations are carried out in order, so the compiler's order is all that it takes.
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+}
 
 template <typename R>
 __global__ __launch_bounds__(kBlock) void bs_deriv(FixedGrid F, MovingVol M, BSplineMap B0,
                                                    const double *__restrict__ stage,
+                                                   const CellMap *__restrict__ maps, CellMap own,
                                                    const int *__restrict__ active,
-                                                   const uint32_t *__restrict__ idx,
                                                    const int *__restrict__ cell_begin,
                                                    const double *__restrict__ wts,
                                                    const uint8_t *__restrict__ fbin,
                                                    MattesParams P, const R *__restrict__ pratio,
                                                    const SampleRec<R> *__restrict__ rec, long long n,
-                                                   int ncells, double *__restrict__ out) {
-    __shared__ double s_x[kBlock / 64][64][16];  // per lane: w[3][4], g[3], pad
+                                                   int parts, bool together, bool ratio_in_lds,
+                                                   double *__restrict__ out) {
+    __shared__ double s_x[kBlock / 64][64][17];  // per lane: w[3][4], g[3], pad
+    extern __shared__ double s_ratio[];          // pRatio, when the launch has room for it
     const int st = active[blockIdx.x];
     const BSplineMap B = start_map(B0, nullptr, stage, st);
     const SampleRec<R> *r = rec + static_cast<size_t>(st) * n;
     pratio += static_cast<size_t>(st) * P.bins * P.bins;
-    const int cell = blockIdx.y;
-    const int b = cell_begin[cell], e = cell_begin[cell + 1];
+    // one part per workgroup, or all parts of a cell in turn (`together`), added
+    // in the same order
+    const int cell = together ? blockIdx.y : blockIdx.y / parts;
+    const int p0 = together ? 0 : blockIdx.y % parts, p1 = together ? parts : p0 + 1;
+    const int cb = cell_begin[cell], ce = cell_begin[cell + 1];
+    const int len = (ce - cb + parts - 1) / parts;
+    const CellMap cm = maps ? maps[st] : own;
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int c = lane & 15, g4 = lane >> 4;
-    f64x4 acc = {0.0, 0.0, 0.0, 0.0};
-    for (int s0 = b; s0 < e; s0 += kBlock) {
-        const int s = s0 + threadIdx.x;
-        double g[3] = {0.0, 0.0, 0.0};
-        double w[3][4] = {{0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}};
-        if (s < e) {
-            const SampleRec<R> rr = r[s];
-            if (rr.mv == rr.mv) {  // a sample the value pass kept
+    R *lratio = reinterpret_cast<R *>(s_ratio);
+    if (ratio_in_lds) {
+        for (int i = threadIdx.x; i < P.bins * P.bins; i += kBlock) lratio[i] = pratio[i];
+        __syncthreads();
+    }
+    double total = 0.0;
+    for (int part = p0; part < p1; ++part) {
+        const int b = cb + part * len, e = min(b + len, ce);
+        f64x4 acc = {0.0, 0.0, 0.0, 0.0};
+        // (a lane without a sample holds the last one's, with g = 0)
+        SampleRec<R> rr;
+        double w[12];
+        int fb;
+        auto fetch = [&](int s) {
+            s = min(s, e - 1);
+            rr = r[s];
+            fb = fbin[s];
 #pragma unroll
-                for (int d = 0; d < 3; ++d)
-#pragma unroll
-                    for (int k = 0; k < 4; ++k) w[d][k] = wts[static_cast<size_t>(s) * 12 + d * 4 + k];
-                R gp[3];
-                physical_gradient<R>(M, rr.gi, gp);
+            for (int k = 0; k < 12; ++k) w[k] = wts[static_cast<size_t>(k) * n + s];
+        };
+        if (b < e) fetch(b + threadIdx.x);
+        for (int s0 = b; s0 < e; s0 += kBlock) {
+            double g[3] = {0.0, 0.0, 0.0};
+            if (s0 + static_cast<int>(threadIdx.x) < e && rr.mv == rr.mv) {  // a sample the value pass kept
                 R arg[4], dv[4];
                 bool mid;
                 const int m0 = Parzen<R>::taps(P, rr.mv, arg, mid);
                 parzen_derivs<R>(arg, mid, dv);
-                const R *row = pratio + fbin[s] * P.bins + m0;
-                R a = R(0);
+                const int at = fb * P.bins + m0;
+                const R a = ratio_in_lds ? tap_sum<R>(lratio + at, dv) : tap_sum<R>(pratio + at, dv);
+                double gq[3];
+                if constexpr (sizeof(R) == 4) {
 #pragma unroll
-                for (int k = 0; k < 4; ++k) a += row[k] * dv[k];
-                double gq[3] = {static_cast<double>(gp[0]), static_cast<double>(gp[1]),
-                                static_cast<double>(gp[2])};
-                if (B.post) {
-                    // the sparse Jacobian's columns left-multiplied by the
-                    // stage's matrix: the gradient enters as M' grad
+                    for (int d = 0; d < 3; ++d)
+                        gq[d] = fma(cm.Q[6 + d], static_cast<double>(rr.gi[2]),
+                                    fma(cm.Q[3 + d], static_cast<double>(rr.gi[1]),
+                                        cm.Q[d] * static_cast<double>(rr.gi[0])));
+                } else {
+                    R gp[3];
+                    physical_gradient<R>(M, rr.gi, gp);
 #pragma unroll
-                    for (int d = 0; d < 3; ++d) {
-                        double acc2 = 0.0;
+                    for (int d = 0; d < 3; ++d) gq[d] = gp[d];
+                    if (B.post) {
+                        // the sparse Jacobian's columns left-multiplied by the
+                        // stage's matrix: the gradient enters as M' grad
 #pragma unroll
-                        for (int q = 0; q < 3; ++q)
-                            acc2 += B.stage[q * 3 + d] * static_cast<double>(gp[q]);
-                        gq[d] = acc2;
+                        for (int d = 0; d < 3; ++d) {
+                            double acc2 = 0.0;
+#pragma unroll
+                            for (int q = 0; q < 3; ++q) acc2 += B.stage[q * 3 + d] * gp[q];
+                            gq[d] = acc2;
+                        }
                     }
                 }
 #pragma unroll
                 for (int d = 0; d < 3; ++d) g[d] = static_cast<double>(a) * gq[d];
             }
-        }
-        double *x = s_x[wv][lane];
+            double *x = s_x[wv][lane];
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            x[k] = w[0][k];
-            x[4 + k] = w[1][k];
-            x[8 + k] = w[2][k];
-        }
-        x[12] = g[0];
-        x[13] = g[1];
-        x[14] = g[2];
-        __syncthreads();
-#pragma unroll 4
-        for (int q = 0; q < 16; ++q) {
-            const double *y = s_x[wv][4 * q + g4];
-            const double ua = y[c & 3] * y[4 + (c >> 2)];
-            const double tb = c < 12 ? y[12 + (c >> 2)] * y[8 + (c & 3)] : 0.0;
-            acc = __builtin_amdgcn_mfma_f64_16x16x4f64(ua, tb, acc, 0, 0, 0);
+            for (int k = 0; k < 12; ++k) x[k] = w[k];
+#pragma unroll
+            for (int d = 0; d < 3; ++d) x[12 + d] = g[d];
+            x[15] = 0.0;  // columns 12 to 15
+            wave_lds_sync();
+            fetch(s0 + kBlock + threadIdx.x);  // in flight during the products
+#pragma unroll
+            for (int q = 0; q < 16; ++q) {
+                const double *y = s_x[wv][4 * q + g4];
+                const double ua = y[c & 3] * y[4 + (c >> 2)];
+                const double tb = y[12 + (c >> 2)] * y[8 + (c & 3)];
+                acc = __builtin_amdgcn_mfma_f64_16x16x4f64(ua, tb, acc, 0, 0, 0);
+            }
+            wave_lds_sync();
         }
         __syncthreads();
-    }
-    // accumulator i of lane l is tile element (row l / 16 + 4 i, column l % 16);
-    // wave w's tile goes to red[w][row][column]
-    double *red = &s_x[0][0][0];
+        // accumulator i of lane l is tile element (row l / 16 + 4 i, column l % 16);
+        // wave w's tile goes to red[w][row][column]
+        double *red = &s_x[0][0][0];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) red[wv * 256 + (g4 + 4 * i) * 16 + c] = acc[i];
-    __syncthreads();
-    if (threadIdx.x < 192) {
-        const int t = threadIdx.x;
-        const int o = (t & 15) * 16 + (t >> 4);
-        out[(static_cast<size_t>(st) * ncells + cell) * 192 + t] =
-            (red[o] + red[256 + o]) + (red[512 + o] + red[768 + o]);
+        for (int i = 0; i < 4; ++i) red[wv * 256 + (g4 + 4 * i) * 16 + c] = acc[i];
+        __syncthreads();
+        if (threadIdx.x < 192) {
+            const int o = (threadIdx.x & 15) * 16 + (threadIdx.x >> 4);
+            total += (red[o] + red[256 + o]) + (red[512 + o] + red[768 + o]);
+        }
+        __syncthreads();  // the next part's samples go where the tiles were
     }
+    if (threadIdx.x < 192)
+        out[(static_cast<size_t>(st) * gridDim.y + blockIdx.y) * 192 + threadIdx.x] = total;
 }
 
-// deriv[d][cp] = sum over the cells whose support holds cp (cell order).
-__global__ void bs_gather(BSplineMap B, const int *__restrict__ active, int ncells,
-                          const double *__restrict__ cellT, double *__restrict__ deriv) {
+// deriv[d][cp] = sum over the (up to 64) cells whose support holds cp and their
+// parts: one wave per control point, lane (x, y, z offset of cp in the cell's
+// support) one cell, added across the wave in a fixed order. (One lane per
+// control point walked 64 cells one after another: 17 us for one start of 1,000
+// control points, 4 now; 64 starts, which filled the chip, 22 and now 28.)
+__global__ __launch_bounds__(256) void bs_gather(BSplineMap B, const int *__restrict__ active, int ncells,
+                                                 int parts, const double *__restrict__ cellT,
+                                                 double *__restrict__ deriv) {
     const int st = active[blockIdx.y];
-    cellT += static_cast<size_t>(st) * ncells * 192;
+    cellT += static_cast<size_t>(st) * ncells * parts * 192;
     deriv += static_cast<size_t>(st) * 3 * B.ncp;
-    const int cp = blockIdx.x * blockDim.x + threadIdx.x;
+    const int cp = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (cp >= B.ncp) return;
     const int m0 = B.gs[0] - 3, m1 = B.gs[1] - 3, m2 = B.gs[2] - 3;
-    const int px = cp % B.gs[0], py = (cp / B.gs[0]) % B.gs[1], pz = cp / (B.gs[0] * B.gs[1]);
+    const int sx = cp % B.gs[0] - (lane & 3), sy = (cp / B.gs[0]) % B.gs[1] - ((lane >> 2) & 3),
+              sz = cp / (B.gs[0] * B.gs[1]) - (lane >> 4);
     double sum[3] = {0.0, 0.0, 0.0};
-    for (int sz = max(0, pz - 3); sz <= min(m2 - 1, pz); ++sz)
-        for (int sy = max(0, py - 3); sy <= min(m1 - 1, py); ++sy)
-            for (int sx = max(0, px - 3); sx <= min(m0 - 1, px); ++sx) {
-                const int cell = sx + m0 * (sy + m1 * sz);
-                const int o = (px - sx) + 4 * (py - sy) + 16 * (pz - sz);
+    if (sx >= 0 && sx < m0 && sy >= 0 && sy < m1 && sz >= 0 && sz < m2) {
+        const double *t = cellT + static_cast<size_t>(sx + m0 * (sy + m1 * sz)) * parts * 192 + lane;
+        for (int p = 0; p < parts; ++p)
 #pragma unroll
-                for (int d = 0; d < 3; ++d) sum[d] += cellT[static_cast<size_t>(cell) * 192 + d * 64 + o];
-            }
+            for (int d = 0; d < 3; ++d) sum[d] += t[p * 192 + d * 64];
+    }
 #pragma unroll
-    for (int d = 0; d < 3; ++d) deriv[static_cast<size_t>(d) * B.ncp + cp] = sum[d];
+    for (int d = 0; d < 3; ++d) {
+        const double v = wave_total_f64(sum[d]);
+        if (lane == 63) deriv[static_cast<size_t>(d) * B.ncp + cp] = v;
+    }
 }
 
 // ------------------------------------------------------------------ host side
@@ -472,6 +709,7 @@ struct BSplineMetric {
     Metric *m = nullptr;        // the Mattes metric (bins set); not owned
     BSplineMap B{};             // coef unused: every evaluation brings its coefficients
     int ncells = 0;
+    int parts = 1;              // parts of a cell in the derivative pass
     SampleSet SS{};             // cell-grouped samples
     DeviceBuffer<uint32_t> idx;
     DeviceBuffer<uint8_t> fbin;
@@ -540,6 +778,9 @@ BSplineMetric *bspline_create(Metric &m, const size_t gs[3], const double origin
             cell[s] = c;
             ++count[c];
         }
+        // about four rounds of a workgroup's lanes per part
+        b->parts = std::max(1, std::min(8, (*std::max_element(count.begin(), count.end()) + 4 * kBlock - 1) /
+                                               (4 * kBlock)));
         std::vector<int> begin(b->ncells + 2, 0);
         for (int c = 0; c <= b->ncells; ++c) begin[c + 1] = begin[c] + count[c];
         std::vector<uint32_t> sflat(n);
@@ -566,7 +807,7 @@ BSplineMetric *bspline_create(Metric &m, const size_t gs[3], const double origin
             DeviceBuffer<int> bad(1);
             HIP_OK(hipMemsetAsync(bad.ptr, 0, sizeof(int), backend().stream));
             hipLaunchKernelGGL(bs_weights, dim3(8, b->ncells), dim3(256), 0, backend().stream, m.F,
-                               b->B, m.chain.ptr, b->idx.ptr, b->cell_begin.ptr, b->ncells,
+                               b->B, m.chain.ptr, b->idx.ptr, b->cell_begin.ptr, b->ncells, n,
                                b->wts.ptr, bad.ptr);
             check_launch("bs_weights");
             int flag = 0;
@@ -655,6 +896,7 @@ struct BSplineMulti {
     size_t np = 0;               // parameters per start (3 ncp)
     bool staged = false;         // per-start stages (else the metric's own)
     DeviceBuffer<double> coef, stage, pratio, cellT, deriv;
+    DeviceBuffer<CellMap> maps;  // staged: each start's composed map (FP32)
     DeviceBuffer<float> pratio_f;
     DeviceBuffer<unsigned long long> joint, marg;
     DeviceBuffer<TailOut> tail;
@@ -672,6 +914,20 @@ struct BSplineMulti {
 };
 
 void bspline_multi_free(BSplineMulti *u) { delete u; }
+
+static CellMap make_cell_map(const Metric &m, const double *stage) {
+    static const double identity[12] = {1, 0, 0, 0, 1, 0, 0, 0, 1, 0, 0, 0};
+    const double *s = stage ? stage : identity;
+    CellMap c;
+    c.X = make_index_map(m.F, m.Mv, s, 1);
+    for (int j = 0; j < 3; ++j)
+        for (int d = 0; d < 3; ++d) {
+            double q = 0.0;
+            for (int k = 0; k < 3; ++k) q += m.Mv.p2i[j * 3 + k] * s[k * 3 + d];
+            c.Q[j * 3 + d] = q;
+        }
+    return c;
+}
 
 // stages: S x 12, or null for the metric's own moving-initial stage.
 BSplineMulti *bspline_multi_create(BSplineMetric &b, int S, const double *stages) {
@@ -691,7 +947,7 @@ BSplineMulti *bspline_multi_create(BSplineMetric &b, int S, const double *stages
         u->stage.alloc(static_cast<size_t>(S) * 12);
         u->pratio.alloc(S * nb);
         u->pratio_f.alloc(S * nb);
-        u->cellT.alloc(static_cast<size_t>(S) * std::max(1, b.ncells) * 192);
+        u->cellT.alloc(static_cast<size_t>(S) * std::max(1, b.ncells) * b.parts * 192);
         u->deriv.alloc(S * u->np);
         u->joint.alloc(static_cast<size_t>(S) * kHistCopies * nb);
         u->marg.alloc(static_cast<size_t>(S) * kHistCopies * B);
@@ -704,7 +960,13 @@ BSplineMulti *bspline_multi_create(BSplineMetric &b, int S, const double *stages
         HIP_OK(hipHostMalloc(reinterpret_cast<void **>(&u->h_deriv), S * u->np * sizeof(double), hipHostMallocDefault));
         HIP_OK(hipHostMalloc(reinterpret_cast<void **>(&u->h_tail), S * sizeof(TailOut), hipHostMallocDefault));
         HIP_OK(hipHostMalloc(reinterpret_cast<void **>(&u->h_active), S * sizeof(int), hipHostMallocDefault));
-        if (stages) u->stage.upload(stages, static_cast<size_t>(S) * 12);
+        std::vector<CellMap> maps;
+        if (stages) {
+            u->stage.upload(stages, static_cast<size_t>(S) * 12);
+            for (int s = 0; s < S; ++s) maps.push_back(make_cell_map(*b.m, stages + 12 * s));
+            u->maps.alloc(maps.size());
+            u->maps.upload(maps.data(), maps.size());
+        }
         std::memset(u->h_coef, 0, S * u->np * sizeof(double));
         sync();
     } catch (...) {
@@ -723,16 +985,29 @@ static void multi_passes(BSplineMulti &u, const int *active, int nact, bool deri
     const size_t shm = static_cast<size_t>(B * B + B) * sizeof(unsigned long long);
     const double *stage = u.staged ? u.stage.ptr : nullptr;
     auto *rec = reinterpret_cast<SampleRec<R> *>(u.rec.ptr);
+    const CellMap *maps = u.staged ? u.maps.ptr : nullptr;
+    const CellMap own = make_cell_map(m, b.B.post ? b.B.stage : nullptr);
+    // many starts: several cells per workgroup; few: a cell shared by several,
+    // so that one start's cells fill the chip
     const int cpb = nact >= 16 ? kCellsPerBlockMany : 1;
     const unsigned groups = static_cast<unsigned>((b.ncells + 1 + cpb - 1) / cpb);
-    {
-        LaunchScope scope("bs_value");
-        hipLaunchKernelGGL(bs_value<R>, dim3(nact, groups), dim3(kBlock), shm, st, m.F, m.Mv, b.B,
-                           u.coef.ptr, stage, active, m.chain.ptr, b.idx.ptr, b.fbin.ptr,
-                           b.cell_begin.ptr, b.wts.ptr, b.ncells, cpb, m.P, u.joint.ptr, u.marg.ptr,
-                           rec, b.SS.n);
-        check_launch("bs_value");
+    if constexpr (sizeof(R) == 4) {
+        const int vparts = nact >= 4 ? 1 : b.parts;
+        launch_kernel("bs_value", bs_value_f32, dim3(nact, groups * vparts), dim3(kBlock), shm, m.F, m.Mv, b.B,
+                      static_cast<const double *>(u.coef.ptr), stage, maps, own, active,
+                      static_cast<const ChainConst *>(m.chain.ptr), static_cast<const uint32_t *>(b.idx.ptr),
+                      static_cast<const uint8_t *>(b.fbin.ptr), static_cast<const int *>(b.cell_begin.ptr),
+                      static_cast<const double *>(b.wts.ptr), b.ncells, cpb, vparts, m.P, u.joint.ptr,
+                      u.marg.ptr, rec, b.SS.n);
+    } else {
+        launch_kernel("bs_value", bs_value<R>, dim3(nact, groups), dim3(kBlock), shm, m.F, m.Mv, b.B,
+                      static_cast<const double *>(u.coef.ptr), stage, active,
+                      static_cast<const ChainConst *>(m.chain.ptr), static_cast<const uint32_t *>(b.idx.ptr),
+                      static_cast<const uint8_t *>(b.fbin.ptr), static_cast<const int *>(b.cell_begin.ptr),
+                      static_cast<const double *>(b.wts.ptr), b.ncells, cpb, m.P, u.joint.ptr, u.marg.ptr, rec,
+                      b.SS.n);
     }
+    check_launch("bs_value");
     {
         LaunchScope scope("bs_tail");
         hipLaunchKernelGGL(bs_tail, dim3(nact), dim3(kTail), shm, st, active, B, m.P.mbs,
@@ -742,17 +1017,21 @@ static void multi_passes(BSplineMulti &u, const int *active, int nact, bool deri
     if (!derivative) return;
     const R *pr = sizeof(R) == 4 ? reinterpret_cast<const R *>(u.pratio_f.ptr)
                                  : reinterpret_cast<const R *>(u.pratio.ptr);
+    // one start's parts fill the chip as workgroups of their own; many starts do
+    // without, and leave the gather a third of the rows to read
+    const int rows = nact >= 4 ? 1 : b.parts;
+    const size_t ratio_all = static_cast<size_t>(B) * B * sizeof(R);
+    const size_t ratio_bytes = ratio_all <= kRatioLds ? ratio_all : 0;
     if (b.ncells > 0) {
-        LaunchScope scope("bs_deriv");
-        hipLaunchKernelGGL(bs_deriv<R>, dim3(nact, b.ncells), dim3(kBlock), 0, st, m.F, m.Mv, b.B,
-                           stage, active, b.idx.ptr, b.cell_begin.ptr, b.wts.ptr, b.fbin.ptr, m.P,
-                           pr, rec,
-                           b.SS.n, b.ncells, u.cellT.ptr);
+        launch_kernel("bs_deriv", bs_deriv<R>, dim3(nact, b.ncells * rows), dim3(kBlock), ratio_bytes, m.F, m.Mv, b.B,
+                      stage, maps, own, active, static_cast<const int *>(b.cell_begin.ptr),
+                      static_cast<const double *>(b.wts.ptr), static_cast<const uint8_t *>(b.fbin.ptr), m.P, pr,
+                      static_cast<const SampleRec<R> *>(rec), b.SS.n, b.parts, rows < b.parts, ratio_bytes > 0,
+                      u.cellT.ptr);
         check_launch("bs_deriv");
     }
-    LaunchScope scope("bs_gather");
-    hipLaunchKernelGGL(bs_gather, dim3((b.B.ncp + 255) / 256, nact), dim3(256), 0, st, b.B,
-                       active, b.ncells, u.cellT.ptr, u.deriv.ptr);
+    launch_kernel("bs_gather", bs_gather, dim3((b.B.ncp + 3) / 4, nact), dim3(256), 0, b.B, active, b.ncells,
+                  rows, static_cast<const double *>(u.cellT.ptr), u.deriv.ptr);
     check_launch("bs_gather");
 }
 

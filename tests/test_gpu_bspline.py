@@ -255,3 +255,51 @@ def test_deformable_pair_at_scale_against_the_oracle(hip, precision):
         assert valid[s] == want_n, s
         assert abs(vals[s] - want_v) <= tv * abs(want_v), (s, vals[s], want_v)
         assert rel_vec(ders[s], want_d) < td, (s, rel_vec(ders[s], want_d))
+
+
+@pytest.mark.parametrize("bins", [24, 44])
+@pytest.mark.parametrize("shape,mesh,kind", [((37, 33, 35), (2, 2, 2), "zero"),
+                                             ((37, 33, 35), (2, 2, 2), "large"),
+                                             ((37, 33, 35), (2, 1, 2), "part"),
+                                             ((9, 7, 8), (3, 2, 4), "part")])
+def test_cells_cut_into_parts_against_the_oracle(hip, bins, shape, mesh, kind):
+    """FP32 at the edges of the cell passes: cells cut into parts (2,600 to
+    9,400 samples) and cells of a few samples; every sample on a decision
+    boundary (zero coefficients on equal grids); displacements of 1e9 that the
+    stage takes back, beyond the composed index's bound; a grid over part of the
+    image, with a moving mask; pRatio in LDS (24 bins) and not (44). The oracle's
+    value, derivative and valid count at the FP32 tolerances above, and the same
+    bits for one start alone as among 3, 4 and 16."""
+    nx, ny, nz = shape
+    f = blob_volume((nz, ny, nx), 5, spacing=SP)
+    m = blob_volume((nz, ny, nx), 6, spacing=SP) * 0.4 + f * 0.6
+    rng = np.random.default_rng(15)
+    mask = None
+    if kind == "part":
+        mask = (rng.random((nz, ny, nx)) < 0.8).astype(np.uint8)
+    df = hip.DeviceImage.upload(f, spacing=SP, origin=ORG)
+    dm = hip.DeviceImage.upload(m, spacing=SP, origin=ORG)
+    met = hip.ResidentMattes(df, dm, bins=bins, moving_mask=None if mask is None else
+                             hip.DeviceMask.upload(mask, spacing=SP, origin=ORG))
+    size = [n - 2 if kind == "part" else n for n in shape]
+    ncp = int(np.prod([k + 3 for k in mesh]))
+    c0 = {"zero": 0.0, "large": 1e9, "part": 0.0}[kind]
+    coeffs = c0 + (0.0 if kind == "zero" else rng.normal(0.0, 0.5, 3 * ncp))
+    coeffs = np.broadcast_to(coeffs, 3 * ncp).copy()
+    t = O.make_bspline(size, SP, ORG, np.eye(3), mesh, coeffs)
+    bs = hip.BSplineMattes(met, list(t.grid_size), list(t.grid_origin), list(t.grid_spacing),
+                           np.array(list(t.grid_direction)).reshape(3, 3))
+    back = O.make_transform(O.TRANSLATION, [-c0] * 3)
+    pb = O.MetricProblem(f, SP, ORG, m, SP, ORG, moving_mask=mask)
+    want_v, want_d, want_n = pb.mattes_evaluate_composed(pb.mattes_geometry(bins), t, back)
+    stage = O.transform_stage(back)
+    bs.set_moving_initial(stage)
+    v, d, n = bs.value_and_derivative(coeffs)
+    assert n == want_n
+    assert abs(v - want_v) <= 1e-6 * abs(want_v), (v, want_v)
+    assert rel_vec(d, want_d) < 1e-4, rel_vec(d, want_d)
+    for starts in (3, 4, 16):
+        multi = hip.BSplineMulti(bs, starts, np.stack([stage] * starts))
+        vals, ders, valid = multi.value_and_derivative(np.stack([coeffs] * starts))
+        for s in (0, starts - 1):
+            assert vals[s] == v and valid[s] == n and np.array_equal(ders[s], d), (starts, s)
