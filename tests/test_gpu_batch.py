@@ -315,3 +315,35 @@ def test_probe_values_are_the_zero_iteration_values(hip):
             assert pv[i] == res0[i].value, (i, pv[i], res0[i].value)
         else:
             assert abs(pv[i] - res0[i].value) <= 1e-12 * abs(res0[i].value)
+
+
+@pytest.mark.parametrize("n", [1, 10, 11, 700])
+@pytest.mark.parametrize("graph", [True, False])
+def test_replays_wait_for_their_own_results(hip, n, graph):
+    """Evaluations in turn on one batch, with other work and its
+    synchronization between them: each returns the results of its own stages and flags, the same
+    bits as a fresh batch's (controls of 1 pair, of the last words of one
+    workgroup of the control copy and the first of the next, and of many; no
+    pair active; all; some)."""
+    rng = np.random.default_rng(3)
+    f = blob_volume((6, 7, 9), 1)
+    m = blob_volume((6, 7, 9), 2) * 0.5 + f * 0.5
+    df, dm = hip.DeviceImage.upload(f), hip.DeviceImage.upload(m)
+    mets = [hip.ResidentMattes(df, dm, bins=12) if i % 3 == 0 else hip.ResidentMetric(df, dm)
+            for i in range(n)]
+    sets = [np.stack([_euler_stage(rng, (4.0, 3.0, 2.5), mm=0.5)[1] for _ in range(n)]) for _ in range(3)]
+    want = []
+    for s in sets:
+        fresh = hip.Batch(mets)
+        want.append(fresh.evaluate(s))
+        fresh.free()
+    batch = hip.Batch(mets)
+    batch.set_tiling(use_graph=graph)
+    masks = [None, np.zeros(n, np.uint8), (np.arange(n) % 2 == 0).astype(np.uint8)]
+    for k in range(9):
+        v, mom, valid = batch.evaluate(sets[k % 3], masks[(k // 3 + k) % 3])
+        on = slice(None) if masks[(k // 3 + k) % 3] is None else masks[(k // 3 + k) % 3] != 0
+        for got, ref in zip((v, mom, valid), want[k % 3]):
+            assert np.array_equal(got[on], ref[on]), k
+        if k % 2:
+            hip.recursive_gaussian(df, [1.0] * 3).to_host()
