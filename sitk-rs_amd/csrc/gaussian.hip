@@ -17,8 +17,8 @@
 // Layout: volumes are dimension-0 fastest. A smoothed axis is one launch. Lines
 // along axes 1 and 2 are assigned to lanes by their dimension-0 coordinate, so
 // every step of the recursion is one coalesced access across a wavefront; axis 0
-// lines are contiguous, so there a step touches one cache line per lane and the
-// following steps hit it in cache.
+// lines are contiguous, so there a lane reads and writes 16 bytes of its line at
+// a time.
 #include <hip/hip_runtime.h>
 
 #include <array>
