@@ -331,8 +331,8 @@ struct CellMap {
 };
 
 // The FP32 path's value pass: the same cells, histogram and records, the
-// displacement and the index composed with fused multiply-adds, two samples per
-// lane. The displacement is summed along x, then y, then z (252 FMAs instead of
+// displacement and the index composed with fused multiply-adds, kCellU samples
+// per lane. The displacement is summed along x, then y, then z (252 FMAs instead of
 // 64 weight products and 192 rounded multiply-adds), and a cell's coefficients
 // come as scalar loads -- a multiply-add takes one operand from a scalar
 // register -- where LDS broadcasts took 192 reads per sample. A sample whose
@@ -341,16 +341,18 @@ struct CellMap {
 // on voxels, as zero coefficients on equal grids do). With few starts a cell's
 // samples are shared by `parts` workgroups (an integer histogram does not depend
 // on it). 64 starts of 707,788 samples on 7^3 cells: 1,363 us before, 1,240 now;
-// one start 53, now 47. The vector pipes issue 54 % of that time and the texture
-// path is busy 65 % (the eight corners of 64 scattered samples); 230 registers
-// leave two waves per SIMD. One sample per lane: 1,290 us at three waves (and 41
-// for one start); a bound of three waves on two samples spills: 2,076.
-constexpr int kCellU = 2;
+// one start 53, now 42. The vector pipes issue 54 % of the many starts' time and
+// the texture path is busy 65 % (the eight corners of 64 scattered samples).
+// Two samples per lane share a coefficient load and take 230 registers, two waves
+// per SIMD; few starts, whose workgroups are short of samples, take one at three
+// waves: one start 42 us against 47, 64 starts 1,290 against 1,240. (A bound of
+// three waves on two samples spills: 2,076; one of two waves costs 1,320.)
 // Displacement in moving voxels below which the composed sum's rounding (some
 // 20 FP64 roundings of terms up to 3 kFar: 1e-7) stays under kGuard.
 constexpr double kFar = 16777216.0;
 
-__global__ __launch_bounds__(kBlock) void bs_value_f32(
+template <int kCellU>
+__global__ __launch_bounds__(kBlock, kCellU == 1 ? 3 : 1) void bs_value_f32(
     FixedGrid F, MovingVol M, BSplineMap B0, const double *__restrict__ coef,
     const double *__restrict__ stage, const CellMap *__restrict__ maps, CellMap own,
     const int *__restrict__ active, const ChainConst *__restrict__ C, const uint32_t *__restrict__ idx,
@@ -993,7 +995,8 @@ static void multi_passes(BSplineMulti &u, const int *active, int nact, bool deri
     const unsigned groups = static_cast<unsigned>((b.ncells + 1 + cpb - 1) / cpb);
     if constexpr (sizeof(R) == 4) {
         const int vparts = nact >= 4 ? 1 : b.parts;
-        launch_kernel("bs_value", bs_value_f32, dim3(nact, groups * vparts), dim3(kBlock), shm, m.F, m.Mv, b.B,
+        auto kernel = nact >= 4 ? bs_value_f32<2> : bs_value_f32<1>;
+        launch_kernel("bs_value", kernel, dim3(nact, groups * vparts), dim3(kBlock), shm, m.F, m.Mv, b.B,
                       static_cast<const double *>(u.coef.ptr), stage, maps, own, active,
                       static_cast<const ChainConst *>(m.chain.ptr), static_cast<const uint32_t *>(b.idx.ptr),
                       static_cast<const uint8_t *>(b.fbin.ptr), static_cast<const int *>(b.cell_begin.ptr),
