@@ -133,7 +133,7 @@ struct InTile {
     }
     // Byte offset of output position p's first tap (kz = ky = kx = 0); `zs`
     // staged planes lie between two output planes.
-    __device__ static int at(int p, int zs) {
+    __device__ static constexpr int at(int p, int zs) {
         const int xo = p % DO, r = p / DO % R, zp = p / (DO * R);
         return ((zp * zs * ROWS + 2 * r) * COLS + 2 * xo) * VS;
     }
@@ -248,53 +248,54 @@ __global__ __launch_bounds__(kConvLanes) void conv_forward(const uint16_t *__res
 }
 
 // ------------------------------------------------ weight gradient, stride 2
-// dW[co][tap][ci] = sum over positions of dy[m][co] x[m's tap][ci], and
-// db[co] = sum of dy[m][co] (one more column, of ones). A workgroup keeps the
-// sums of its KZN kernel planes and COW output channels in the accumulators
-// over its chunks (blockIdx.x, + gridDim.x, ...) and writes one partial row
-// [CO][27 CI], [CO]; reduce_partials adds the rows in a fixed tree.
-// Gathering each operand's eight positions from global memory one scalar at a
-// time, with bias sums and masks in passes of their own, took 5.6 ms for the
-// five layers of 24 pairs and 1.3 ms for those passes; the five layers now take
-// 0.18 ms and the fold of the partial rows 0.025.
-template <int LGDO, int CI, int CO, int R, int ZP, int KZN, int COW>
+// dW[co][tap][ci] = sum over positions of dy[m][co] x[m's tap][ci]. The
+// positions are cut into splits of `per` (a multiple of 32, wgrad_split), one
+// per blockIdx.x; a split's products are added 32 positions at a time in the
+// positions' order into one partial row [CO][27 CI], and reduce_partials adds
+// the rows in order. The order of a gradient's sums is kept for good: a
+// training run amplifies the rounding of a sum (Adam divides each gradient by
+// its own size) until two orders differ by several percent after four steps.
+// So the chip is filled by splitting the outputs, kernel planes (KZN), channels
+// (COW) and column tiles (CG groups) over blockIdx.y, and the staged chunk (P
+// positions) is large, since a split's chunks come one after another. 24 pairs,
+// layers 1 to 4: 70, 56, 49 and 24 us (without column groups 70, 65, 73 and 27;
+// a second chunk on its way changed nothing), bound by the LDS reads and stores
+// between two barriers. Rows of any positions, added in a tree, took 60, 37, 14
+// and 9. The first kernels, which gathered each operand's positions from global
+// memory one scalar at a time, took 5.6 ms for the five layers.
+template <int LGDO, int CI, int CO, int R, int ZP, int KZN, int COW, int CG>
 __global__ __launch_bounds__(kConvLanes, CI <= 32 ? 2 : 1) void conv_wgrad(const uint16_t *__restrict__ x,
                                                          const uint16_t *__restrict__ dy,
-                                                         float *__restrict__ partial, int nchunks) {
+                                                         float *__restrict__ partial, int per, int total) {
     using T = InTile<LGDO, CI, R, ZP, KZN * ZP>;
     constexpr int DS = 2 * COW + 16;                       // bytes per staged dy position
     constexpr int STEPS = T::P / 32, RT = COW / 16;
-    constexpr int NC = 9 * KZN * CI / 16, NJ = (NC + 3) / 4;  // column tiles, per wave
+    constexpr int NC = 9 * KZN * CI / 16 / CG, NJ = (NC + 3) / 4;  // column tiles, per wave
     constexpr int DYP = T::P * COW / 8, DYN = (DYP + kConvLanes - 1) / kConvLanes;
     static_assert(T::P % 32 == 0 && (KZN == 3 ? ZP == 1 : KZN == 1), "chunk shape");
+    static_assert(9 * KZN * CI / 16 % CG == 0, "column groups of whole tiles");
     extern __shared__ char lds[];
     char *sdy = lds + T::kBytes;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int i16 = lane & 15, g = lane >> 4;
-    constexpr int KZG = 3 / KZN;  // workgroups along blockIdx.y per channel group
-    const int kz0 = (blockIdx.y % KZG) * KZN, co0 = (blockIdx.y / KZG) * COW;
-    const bool bias_here = kz0 == 0 && w == 3;
+    constexpr int KZG = 3 / KZN;  // workgroups along blockIdx.y: column groups, planes, channels
+    const int t0 = (blockIdx.y % CG) * NC;
+    const int kz0 = (blockIdx.y / CG % KZG) * KZN, co0 = (blockIdx.y / (CG * KZG)) * COW;
 
     const int p0 = 8 * g + (i16 >> 2);  // this lane's row of the first 4 x 16 block
     const int xbase = T::at(p0, 1) + 8 * (i16 & 3), dbase = p0 * DS + 8 * (i16 & 3);
     constexpr int kXHalf = T::DO >= 8 ? 8 * T::VS : 2 * T::COLS * T::VS;     // position + 4
-    constexpr int kXStep = 2 * (32 / T::DO) * T::COLS * T::VS;               // position + 32
     int toff[NJ];
 #pragma unroll
     for (int j = 0; j < NJ; ++j) {
-        const int t = w + 4 * j, tap = t / (CI / 16), c = t % (CI / 16);
+        const int t = t0 + w + 4 * j, tap = t / (CI / 16), c = t % (CI / 16);
         toff[j] = T::tap((tap / 9) * ZP, tap / 3 % 3, tap % 3) + 32 * c;
     }
-    f32x4 acc[NJ][RT], accb[RT];
+    f32x4 acc[NJ][RT];
 #pragma unroll
-    for (int r = 0; r < RT; ++r) {
-        accb[r] = zero_acc();
+    for (int r = 0; r < RT; ++r)
 #pragma unroll
         for (int j = 0; j < NJ; ++j) acc[j][r] = zero_acc();
-    }
-    Frag ones;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) ones.h[e] = 0x3f80;
 
     T::clear_edge(lds);
     u32x4 v[T::kPer], d[DYN];
@@ -302,7 +303,7 @@ __global__ __launch_bounds__(kConvLanes, CI <= 32 ? 2 : 1) void conv_wgrad(const
         int n, z0, y0;
         T::chunk(c, n, z0, y0);
         T::load(x, n, 2 * z0 - 1 + kz0, KZN == 3 ? 1 : 2, y0, v);
-        const size_t pos0 = ((static_cast<size_t>(n) * T::DO + z0) * T::DO + y0) * T::DO;
+        const size_t pos0 = static_cast<size_t>(c) * T::P;
 #pragma unroll
         for (int k = 0; k < DYN; ++k) {
             const int i = threadIdx.x + k * kConvLanes;
@@ -311,9 +312,24 @@ __global__ __launch_bounds__(kConvLanes, CI <= 32 ? 2 : 1) void conv_wgrad(const
                                                         (i % (COW / 8)) * 8);
         }
     };
-    int c = blockIdx.x;
-    if (c < nchunks) fetch(c);
-    for (; c < nchunks; c += gridDim.x) {
+    auto step = [&](int s) {
+        bf16x8 a[RT];
+#pragma unroll
+        for (int r = 0; r < RT; ++r) a[r] = tr_frag(sdy + dbase + s * 32 * DS + 32 * r, 4 * DS);
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            if (NC % 4 != 0 && w + 4 * j >= NC) continue;  // the same for the whole wave
+            const bf16x8 b = tr_frag(lds + xbase + toff[j] + T::at(32 * s, 1), kXHalf);
+#pragma unroll
+            for (int r = 0; r < RT; ++r) acc[j][r] = mfma(a[r], b, acc[j][r]);
+        }
+    };
+    // the split's positions; its first and last chunk may be a neighbour's too
+    const int begin = blockIdx.x * per, end = min(begin + per, total);
+    const int c_end = (end + T::P - 1) / T::P;
+    int c = begin / T::P;
+    if (c < c_end) fetch(c);
+    for (; c < c_end; ++c) {
         __syncthreads();
         T::store(lds, v);
 #pragma unroll
@@ -323,41 +339,74 @@ __global__ __launch_bounds__(kConvLanes, CI <= 32 ? 2 : 1) void conv_wgrad(const
                 *reinterpret_cast<u32x4 *>(sdy + (i / (COW / 8)) * DS + (i % (COW / 8)) * 16) = d[k];
         }
         __syncthreads();
-        if (c + static_cast<int>(gridDim.x) < nchunks) fetch(c + gridDim.x);
+        if (c + 1 < c_end) fetch(c + 1);
+        const int at = c * T::P;
+        if (at >= begin && at + T::P <= end) {
 #pragma unroll
-        for (int s = 0; s < STEPS; ++s) {
-            bf16x8 a[RT];
+            for (int s = 0; s < STEPS; ++s) step(s);
+        } else {
 #pragma unroll
-            for (int r = 0; r < RT; ++r) a[r] = tr_frag(sdy + dbase + s * 32 * DS + 32 * r, 4 * DS);
-#pragma unroll
-            for (int j = 0; j < NJ; ++j) {
-                if (NC % 4 != 0 && w + 4 * j >= NC) continue;  // the same for the whole wave
-                const bf16x8 b = tr_frag(lds + xbase + toff[j] + s * kXStep, kXHalf);
-#pragma unroll
-                for (int r = 0; r < RT; ++r) acc[j][r] = mfma(a[r], b, acc[j][r]);
-            }
-            if (bias_here)
-#pragma unroll
-                for (int r = 0; r < RT; ++r) accb[r] = mfma(a[r], ones.v, accb[r]);
+            for (int s = 0; s < STEPS; ++s)
+                if (at + 32 * s >= begin && at + 32 * s < end) step(s);
         }
     }
-    float *out = partial + static_cast<size_t>(blockIdx.x) * (CO * 27 * CI + CO);
+    float *out = partial + static_cast<size_t>(blockIdx.x) * (CO * 27 * CI);
 #pragma unroll
     for (int j = 0; j < NJ; ++j) {
         const int t = w + 4 * j;
         if (NC % 4 != 0 && t >= NC) continue;
-        const int col = kz0 * 9 * CI + t * 16 + i16;
+        const int col = kz0 * 9 * CI + (t0 + t) * 16 + i16;
 #pragma unroll
         for (int r = 0; r < RT; ++r)
 #pragma unroll
             for (int e = 0; e < 4; ++e)
                 out[static_cast<size_t>(co0 + 16 * r + 4 * g + e) * (27 * CI) + col] = acc[j][r][e];
     }
-    if (bias_here && i16 == 0)
+}
+
+// ------------------------------------------------------------ bias gradient
+// db[co] = sum of dy[m][co], every layer in one launch: a workgroup takes one
+// of kBiasSplits runs of a layer's positions, lane (c, part) adds channel c of
+// positions part, part + 256 / C, ..., the parts are added in order, and
+// reduce_partials adds the runs in order (see conv_wgrad on the order). 24
+// pairs, 265 MB: 52 us (5.1 TB/s; the first kernels 709).
+struct BiasLayer {
+    const uint16_t *dy;
+    float *partial;  // [kBiasSplits][channels]
+    int positions, channels;
+};
+struct BiasLayers {
+    BiasLayer l[5];
+};
+constexpr int kBiasSplits = 256;
+constexpr int kBiasLoads = 64;  // in flight per lane: the first layer has 1,024 waves for 201 MB
+
+__global__ __launch_bounds__(kConvLanes) void bias_grad(BiasLayers L) {
+    __shared__ float red[kConvLanes];
+    const BiasLayer &q = L.l[blockIdx.y];
+    const int C = q.channels, parts = kConvLanes / C;
+    const int per = (q.positions + kBiasSplits - 1) / kBiasSplits;
+    const int m0 = blockIdx.x * per, m1 = min(q.positions, m0 + per);
+    const int c = threadIdx.x % C, part = threadIdx.x / C;
+    const uint16_t *p = q.dy + c;
+    float acc = 0.0f;
+    int m = m0 + part;
+    for (; m + (kBiasLoads - 1) * parts < m1; m += kBiasLoads * parts) {
+        uint16_t v[kBiasLoads];
 #pragma unroll
-        for (int r = 0; r < RT; ++r)
+        for (int u = 0; u < kBiasLoads; ++u) v[u] = p[static_cast<size_t>(m + u * parts) * C];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) out[CO * 27 * CI + co0 + 16 * r + 4 * g + e] = accb[r][e];
+        for (int u = 0; u < kBiasLoads; ++u) acc += __uint_as_float(static_cast<uint32_t>(v[u]) << 16);
+    }
+#pragma unroll 8
+    for (; m < m1; m += parts) acc += __uint_as_float(static_cast<uint32_t>(p[static_cast<size_t>(m) * C]) << 16);
+    red[threadIdx.x] = acc;
+    __syncthreads();
+    if (static_cast<int>(threadIdx.x) < C) {
+        float t = 0.0f;
+        for (int k = 0; k < parts; ++k) t += red[k * C + threadIdx.x];
+        q.partial[static_cast<size_t>(blockIdx.x) * C + threadIdx.x] = t;
+    }
 }
 
 // ------------------------------------------------- input gradient, stride 2
@@ -485,10 +534,10 @@ __global__ __launch_bounds__(kConvLanes, 2) void conv_dgrad(const uint16_t *__re
 // 2 -> 16 channels, stride 1, 64^3. A voxel's two channels are one 4-byte
 // word. A chunk is ROWS output rows (ROWS / 4 per wave) of one plane; it reads
 // 3 planes x (ROWS + 2) rows x voxels -2 .. 65, zero outside the volume.
-template <int ROWS>
+template <int ROWS, int LANES = kConvLanes>
 struct C0Tile {
     static constexpr int COLS = 68, kVox = 3 * (ROWS + 2) * COLS, WAVE_ROWS = ROWS / 4;
-    static constexpr int kPer = (kVox + kConvLanes - 1) / kConvLanes;
+    static constexpr int kPer = (kVox + LANES - 1) / LANES;
 
     static int chunks(int n) { return n * 64 * (64 / ROWS); }
     __device__ static void chunk(int c, size_t &n, int &z, int &y0) {
@@ -502,7 +551,7 @@ struct C0Tile {
         chunk(c, n, z, y0);
 #pragma unroll
         for (int k = 0; k < kPer; ++k) {
-            const int i = threadIdx.x + k * kConvLanes;
+            const int i = threadIdx.x + k * LANES;
             const int xi = i % COLS - 2, row = i / COLS;
             const int yi = y0 + row % (ROWS + 2) - 1, zi = z + row / (ROWS + 2) - 1;
             v[k] = 0;
@@ -513,7 +562,7 @@ struct C0Tile {
     __device__ static void store(char *lds, const uint32_t (&v)[kPer]) {
 #pragma unroll
         for (int k = 0; k < kPer; ++k) {
-            const int i = threadIdx.x + k * kConvLanes;
+            const int i = threadIdx.x + k * LANES;
             if (i < kVox) *reinterpret_cast<uint32_t *>(lds + 4 * i) = v[k];
         }
     }
@@ -592,162 +641,129 @@ __global__ __launch_bounds__(kConvLanes) void conv0_forward(const uint32_t *__re
     }
 }
 
-// Weight gradient: the three kx taps of one (kz, ky) are 12 consecutive bytes
-// of a staged row, so two (kz, ky) pairs fill a 16-column tile with four voxels
-// each (the fourth, past the taps, is computed and dropped). The transposed
-// read takes 8-byte pieces on 8-byte boundaries: odd columns x read voxels
-// x - 1 .. x + 2, even ones x - 2 .. x + 1, in accumulators of their own.
-// (24 pairs, 226 MB: 54 us, 4.2 TB/s, at four waves per SIMD; 85 with three
-// and the staged pieces in scratch; 102 with chunks of eight rows.)
+// Weight gradient, the positions 32 at a time in their order (see conv_wgrad):
+// one split of `per` positions per workgroup, one 16-column tile per wave of the
+// first kW0Tiles. The three kx taps of one (kz, ky) are 12 consecutive bytes of
+// a staged row, read as two 8-byte pieces (voxels x - 1, x and x + 1, x + 2;
+// the last voxel's products are dropped), four pieces to a tile. A transposed
+// read takes 8-byte pieces on 8-byte boundaries, so the rows are staged twice,
+// the second time one voxel earlier, and an even x reads there. At most 256
+// splits, a workgroup per CU: eight waves stage, two chunks ahead. 24 pairs, 226
+// MB: 70 us (3.2 TB/s; 1,024 rows of any positions took 52).
+constexpr int kW0Lanes = 512;
 constexpr int kW0Dy = 48;  // bytes per staged dy position (16 channels + 16)
-constexpr int kW0Rows = 4;
-constexpr int kW0Tile = 4 * C0Tile<kW0Rows>::kVox;
-constexpr int kW0Lds = kW0Tile + kW0Rows * 64 * kW0Dy;
-constexpr int kW0Out = 16 * 54 + 16;      // [16][27][2] and the bias
+constexpr int kW0Rows = 8;
+constexpr int kW0Tiles = 5;
+constexpr int kW0Copy = 4 * C0Tile<kW0Rows, kW0Lanes>::kVox;  // one staged copy of the rows
+constexpr int kW0Lds = 2 * kW0Copy + kW0Rows * 64 * kW0Dy;
+constexpr int kW0Out = 16 * 54;  // [16][27][2]
 
-__global__ __launch_bounds__(kConvLanes, 4) void conv0_wgrad(const uint32_t *__restrict__ x,
-                                                          const uint16_t *__restrict__ dy,
-                                                          float *__restrict__ partial, int nchunks) {
-    using T = C0Tile<kW0Rows>;
+__global__ __launch_bounds__(kW0Lanes) void conv0_wgrad(const uint32_t *__restrict__ x,
+                                                        const uint16_t *__restrict__ dy,
+                                                        float *__restrict__ partial, int per, int total) {
+    using T = C0Tile<kW0Rows, kW0Lanes>;
+    constexpr int P = kW0Rows * 64;  // positions of a chunk; splits are whole chunks
     __shared__ __attribute__((aligned(16))) char lds[kW0Lds];
-    char *sdy = lds + kW0Tile;
+    char *sdy = lds + 2 * kW0Copy;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int i16 = lane & 15, g = lane >> 4;
-    f32x4 acc[2][5], accb = zero_acc();
-#pragma unroll
-    for (int q = 0; q < 2; ++q)
-#pragma unroll
-        for (int j = 0; j < 5; ++j) acc[q][j] = zero_acc();
-    Frag ones;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) ones.h[e] = 0x3f80;
-    const int kk = 8 * g + (i16 >> 2);  // position 2 kk + parity of the row
-    const int sub = i16 & 3;
-    int xoff[5];
-#pragma unroll
-    for (int j = 0; j < 5; ++j) {
-        const int q = min(2 * j + (sub >> 1), 8);  // (kz, ky)
-        xoff[j] = T::row(q / 3, q % 3, w) + (2 * kk + 2 * (sub & 1)) * 4;
-    }
-    const int dbase = (w * T::WAVE_ROWS * 64 + 2 * kk) * kW0Dy + 8 * sub;
-    constexpr int kDyN = kW0Rows * 64 * 2 / kConvLanes;
-    uint32_t v[T::kPer];
-    u32x4 d[kDyN];
-    auto fetch = [&](int c) {
-        T::load(x, c, v);
-        size_t n;
-        int z, y0;
-        T::chunk(c, n, z, y0);
-        const size_t pos0 = ((n * 64 + z) * 64 + y0) * 64;
+    const int i16 = lane & 15, g = lane >> 4, sub = i16 & 3;
+    const int p0 = 8 * g + (i16 >> 2);  // this lane's row of the first 4 x 16 block
+    const int piece = min(4 * w + sub, 17);
+    // voxel x - 1 lies at word x + 1 of its row, in the second copy at word x
+    const int xoff = T::row(piece / 6, piece / 2 % 3, 0) + (p0 & 1 ? 4 * (p0 + 1) : kW0Copy + 4 * p0) +
+                     8 * (piece & 1);
+    const int dbase = p0 * kW0Dy + 8 * sub;
+    f32x4 acc = zero_acc();
+    constexpr int kDyN = P * 2 / kW0Lanes;
+    struct Chunk {
+        uint32_t v[T::kPer];
+        u32x4 d[kDyN];
+    } even, odd;
+    auto fetch = [&](Chunk &q, int c) {
+        T::load(x, c, q.v);
 #pragma unroll
         for (int k = 0; k < kDyN; ++k)
-            d[k] = *reinterpret_cast<const u32x4 *>(dy + pos0 * 16 + (threadIdx.x + k * kConvLanes) * 8);
+            q.d[k] = *reinterpret_cast<const u32x4 *>(dy + static_cast<size_t>(c) * P * 16 +
+                                                      (threadIdx.x + k * kW0Lanes) * 8);
     };
-    int c = blockIdx.x;
-    if (c < nchunks) fetch(c);
-    for (; c < nchunks; c += gridDim.x) {
+    const int c_end = min(static_cast<int>(blockIdx.x + 1) * per, total) / P;
+    auto run = [&](Chunk &q, int c) {
+        if (c >= c_end) return;
         __syncthreads();
-        T::store(lds, v);
+#pragma unroll
+        for (int k = 0; k < T::kPer; ++k) {
+            const int i = threadIdx.x + k * kW0Lanes;
+            if (i < T::kVox) {
+                *reinterpret_cast<uint32_t *>(lds + 4 * i) = q.v[k];
+                if (i > 0) *reinterpret_cast<uint32_t *>(lds + kW0Copy + 4 * (i - 1)) = q.v[k];
+            }
+        }
 #pragma unroll
         for (int k = 0; k < kDyN; ++k) {
-            const int i = threadIdx.x + k * kConvLanes;
-            *reinterpret_cast<u32x4 *>(sdy + (i >> 1) * kW0Dy + (i & 1) * 16) = d[k];
+            const int i = threadIdx.x + k * kW0Lanes;
+            *reinterpret_cast<u32x4 *>(sdy + (i >> 1) * kW0Dy + (i & 1) * 16) = q.d[k];
         }
         __syncthreads();
-        if (c + static_cast<int>(gridDim.x) < nchunks) fetch(c + gridDim.x);
+        if (c + 2 < c_end) fetch(q, c + 2);
+        if (w >= kW0Tiles) return;  // these waves stage only
 #pragma unroll
-        for (int r = 0; r < T::WAVE_ROWS; ++r)
-#pragma unroll
-            for (int q = 0; q < 2; ++q) {  // parity of x
-                const bf16x8 a = tr_frag(sdy + dbase + (64 * r + q) * kW0Dy, 8 * kW0Dy);
-#pragma unroll
-                for (int j = 0; j < 5; ++j)
-                    acc[q][j] = mfma(a, tr_frag(lds + xoff[j] + r * T::COLS * 4 + q * 8, 32), acc[q][j]);
-                accb = mfma(a, ones.v, accb);
-            }
+        for (int s = 0; s < P / 32; ++s) {
+            const bf16x8 a = tr_frag(sdy + dbase + 32 * s * kW0Dy, 4 * kW0Dy);
+            acc = mfma(a, tr_frag(lds + xoff + (s >> 1) * T::COLS * 4 + (s & 1) * 128, 16), acc);
+        }
+    };
+    int c = blockIdx.x * per / P;
+    if (c < c_end) fetch(even, c);
+    if (c + 1 < c_end) fetch(odd, c + 1);
+    for (; c < c_end; c += 2) {
+        run(even, c);
+        run(odd, c + 1);
     }
-    // the four waves' tiles, added in order
+    if (w >= kW0Tiles) return;
     float *out = partial + static_cast<size_t>(blockIdx.x) * kW0Out;
-    float *red = reinterpret_cast<float *>(lds);  // tile by tile: [wave][co][column]
-    static_assert(kW0Lds >= 4 * 256 * 4, "the waves' tiles fit");
-    const int t = threadIdx.x;
-    const int co = t >> 4, col = t & 15;
-    float sum[2][5];
+    const int pi = 4 * w + (i16 >> 2), kx = 2 * (pi & 1) + ((i16 >> 1) & 1);  // this lane's column
+    if (pi < 18 && kx < 3)
 #pragma unroll
-    for (int q = 0; q < 2; ++q)
-#pragma unroll
-        for (int j = 0; j < 5; ++j) {
-            __syncthreads();
-#pragma unroll
-            for (int e = 0; e < 4; ++e) red[w * 256 + (4 * g + e) * 16 + i16] = acc[q][j][e];
-            __syncthreads();
-            sum[q][j] = ((red[t] + red[256 + t]) + red[512 + t]) + red[768 + t];
-        }
-    __syncthreads();
-#pragma unroll
-    for (int e = 0; e < 4; ++e) red[w * 256 + (4 * g + e) * 16 + i16] = accb[e];
-    __syncthreads();
-    const float db = ((red[t] + red[256 + t]) + red[512 + t]) + red[768 + t];
-    if (col == 0) out[16 * 54 + co] = db;
-    // even x: column (voxel v, channel c) is tap kx = v - 1; odd x: kx = v.
-    float *even = red, *odd = red + 256;
-#pragma unroll
-    for (int j = 0; j < 5; ++j) {
-        __syncthreads();
-        even[t] = sum[0][j];
-        odd[t] = sum[1][j];
-        __syncthreads();
-        const int q = 2 * j + (col >> 3), kx = (col >> 1) & 3, ch = col & 1;
-        if (q < 9 && kx < 3)
-            out[co * 54 + (q * 3 + kx) * 2 + ch] = even[t + 2] + odd[t];
-    }
+        for (int e = 0; e < 4; ++e)
+            out[(4 * g + e) * 54 + ((pi >> 1) * 3 + kx) * 2 + (i16 & 1)] = acc[e];
 }
 
 // ---------------------------------------------------------- partial rows
-// Layers' partial rows summed into the gradient vector in one launch: a
-// workgroup takes 64 consecutive values of one layer, lane (s, i) adds rows
-// s, s + 4, ... of value i, and the four sums are added in order. Value i of
-// a row goes to out[(i / inner) * ld + i % inner] (the first layer's two used
-// channels lie eight apart in the parameter vector; its bias follows).
+// Partial rows summed into the gradient vector in one launch, each value's rows
+// in their order (see conv_wgrad), sixteen loads ahead (24 pairs: 12 us). Value i goes to
+// out[(i / inner) * ld + i % inner] (the first layer's two used channels lie
+// eight apart in the parameter vector).
 struct PartialRows {
     const float *p;
-    float *out, *out_bias;  // values from `len` on go to out_bias
-    int rows, len, total, inner, ld;
+    float *out;
+    int rows, len, inner, ld;
     unsigned first_block;
 };
-constexpr int kMaxPartialJobs = 5;
+constexpr int kMaxPartialJobs = 10;
 struct PartialJobs {
     PartialRows j[kMaxPartialJobs];
     int n;
 };
+constexpr int kPartialLanes = 64;
 
-__global__ __launch_bounds__(kConvLanes) void reduce_partials(PartialJobs J) {
-    __shared__ float s_sum[4][64];
+__global__ __launch_bounds__(kPartialLanes) void reduce_partials(PartialJobs J) {
     int k = 0;
     while (k + 1 < J.n && blockIdx.x >= J.j[k + 1].first_block) ++k;
     const PartialRows &q = J.j[k];
-    const int lane = threadIdx.x & 63, s = threadIdx.x >> 6;
-    const int i = static_cast<int>(blockIdx.x - q.first_block) * 64 + lane;
-    float a = 0.0f;
-    if (i < q.total) {
-        const float *p = q.p + i;
-        int r = s;
-        for (; r + 28 < q.rows; r += 32) {
-            float v[8];
+    const int i = static_cast<int>(blockIdx.x - q.first_block) * kPartialLanes + threadIdx.x;
+    if (i >= q.len) return;
+    const float *p = q.p + i;
+    float s = 0.0f;
+    int r = 0;
+    for (; r + 16 <= q.rows; r += 16) {
+        float v[16];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) v[u] = p[static_cast<size_t>(r + 4 * u) * q.total];
+        for (int u = 0; u < 16; ++u) v[u] = p[static_cast<size_t>(r + u) * q.len];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) a += v[u];
-        }
-        for (; r < q.rows; r += 4) a += p[static_cast<size_t>(r) * q.total];
+        for (int u = 0; u < 16; ++u) s += v[u];
     }
-    s_sum[s][lane] = a;
-    __syncthreads();
-    if (s == 0 && i < q.total) {
-        const float t = ((s_sum[0][lane] + s_sum[1][lane]) + s_sum[2][lane]) + s_sum[3][lane];
-        if (i < q.len) q.out[(i / q.inner) * q.ld + i % q.inner] = t;
-        else q.out_bias[i - q.len] = t;
-    }
+    for (; r < q.rows; ++r) s += p[static_cast<size_t>(r) * q.len];
+    q.out[(i / q.inner) * q.ld + i % q.inner] = s;
 }
 
 }  // namespace cnn

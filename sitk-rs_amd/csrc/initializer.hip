@@ -66,9 +66,11 @@ __host__ __device__ inline float bf2f(uint16_t h) {
 
 // ------------------------------------------------------- small kernels
 // Global average pool of the last conv output [n][64][128] and the MLP head,
-// one workgroup of 256 lanes per sample: lane (h, t) sums half of channel t's
-// positions, then half of row t of W1 (32-byte pieces), and two waves share
-// the output rows.
+// one workgroup per sample: lane t of 128 sums channel t's positions, then row t
+// of W1, then (t < 12) row t of W2, each in order: the sums decide the rounding
+// of the gradients' BF16 values, see conv_wgrad. All 256 lanes load W1, in whole
+// rows, and half of its columns at a time goes to LDS.
+constexpr int kHeadCols = kFeat / 2;
 __global__ __launch_bounds__(256) void head_forward(const uint16_t *__restrict__ y,
                                                     const float *__restrict__ w1,
                                                     const float *__restrict__ b1,
@@ -76,61 +78,70 @@ __global__ __launch_bounds__(256) void head_forward(const uint16_t *__restrict__
                                                     const float *__restrict__ b2,
                                                     float *__restrict__ feat, float *__restrict__ hid,
                                                     float *__restrict__ out) {
-    __shared__ float part[2][kFeat], f[kFeat], hh[kHidden];
-    const int b = blockIdx.x, t = threadIdx.x & 127, h = threadIdx.x >> 7;
-    // the lane's half row of W1, on its way while the pool is summed
-    float4 w[kFeat / 8];
-#pragma unroll
-    for (int k = 0; k < kFeat / 8; ++k)
-        w[k] = reinterpret_cast<const float4 *>(w1 + t * kFeat + h * (kFeat / 2))[k];
+    __shared__ float f[kFeat], hh[kHidden], sw1[kHidden][kHeadCols + 1], sw2[kOut][kHidden + 1];
+    const int b = blockIdx.x, t = threadIdx.x;
     float s = 0.0f;
-#pragma unroll 16
-    for (int p = 32 * h; p < 32 * h + 32; ++p)
-        s += bf2f(y[(static_cast<size_t>(b) * 64 + p) * kFeat + t]);
-    part[h][t] = s;
-    __syncthreads();
-    if (h == 0) {
-        const float v = (part[0][t] + part[1][t]) * (1.0f / 64.0f);
-        f[t] = v;
-        feat[b * kFeat + t] = v;
-    }
-    __syncthreads();
-    s = 0.0f;
+    if (t < kFeat) {
+        uint16_t v[64];
 #pragma unroll
-    for (int k = 0; k < kFeat / 8; ++k) {
-        const float *q = f + h * (kFeat / 2) + 4 * k;
-        s += w[k].x * q[0];
-        s += w[k].y * q[1];
-        s += w[k].z * q[2];
-        s += w[k].w * q[3];
-    }
-    part[h][t] = s;
-    __syncthreads();
-    if (h == 0) {
-        const float v = fmaxf(b1[t] + (part[0][t] + part[1][t]), 0.0f);
-        hh[t] = v;
-        hid[b * kHidden + t] = v;
-    }
-    __syncthreads();
-    // output o by wave o mod 4
-    const int lane = threadIdx.x & 63;
-    for (int o = threadIdx.x >> 6; o < kOut; o += 4) {
-        float v = w2[o * kHidden + lane] * hh[lane] + w2[o * kHidden + 64 + lane] * hh[64 + lane];
+        for (int p = 0; p < 64; ++p) v[p] = y[(static_cast<size_t>(b) * 64 + p) * kFeat + t];
 #pragma unroll
-        for (int k = 32; k > 0; k >>= 1) v += __shfl_xor(v, k, 64);
-        if (lane == 0) out[b * kOut + o] = b2[o] + v;
+        for (int p = 0; p < 64; ++p) s += bf2f(v[p]);
+        s *= 1.0f / 64.0f;
+        f[t] = s;
+        feat[b * kFeat + t] = s;
+        s = b1[t];
+    }
+    for (int i = t; i < kOut * kHidden; i += 256) sw2[i / kHidden][i % kHidden] = w2[i];
+    constexpr int kQuads = kHidden * kHeadCols / 4 / 256;  // per lane and half
+    float4 w[2][kQuads];
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int k = 0; k < kQuads; ++k) {
+            const int i = t + 256 * k, row = i / (kHeadCols / 4), col = i % (kHeadCols / 4);
+            w[h][k] = reinterpret_cast<const float4 *>(w1 + row * kFeat + h * kHeadCols)[col];
+        }
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < kQuads; ++k) {
+            const int i = t + 256 * k, row = i / (kHeadCols / 4), col = i % (kHeadCols / 4) * 4;
+            sw1[row][col] = w[h][k].x;
+            sw1[row][col + 1] = w[h][k].y;
+            sw1[row][col + 2] = w[h][k].z;
+            sw1[row][col + 3] = w[h][k].w;
+        }
+        __syncthreads();
+        if (t < kHidden)
+#pragma unroll 32
+            for (int i = 0; i < kHeadCols; ++i) s += sw1[t][i] * f[h * kHeadCols + i];
+    }
+    if (t < kHidden) {
+        s = fmaxf(s, 0.0f);
+        hh[t] = s;
+        hid[b * kHidden + t] = s;
+    }
+    __syncthreads();
+    if (t < kOut) {
+        float o = b2[t];
+#pragma unroll 32
+        for (int j = 0; j < kHidden; ++j) o += sw2[t][j] * hh[j];
+        out[b * kOut + t] = o;
     }
 }
 
 // MLP head backward, per sample (one workgroup of 256 lanes): the hidden
 // gradient dhid = relu'(hid) * W2' dout, the pooled features' dfeat = W1' dhid
-// (128 lanes each), and through the pool and the last convolution's ReLU the
-// gradient of its 64 output positions.
+// (128 lanes each, in order), and through the pool and the last convolution's
+// ReLU the gradient of its 64 output positions.
 __global__ __launch_bounds__(256) void head_backward_samples(
     const float *__restrict__ hid, const float *__restrict__ dout, const float *__restrict__ w1,
     const float *__restrict__ w2, const uint16_t *__restrict__ y, float *__restrict__ dhid,
     uint16_t *__restrict__ dy) {
-    __shared__ float dh[kHidden], half[2][kFeat];
+    __shared__ float dh[kHidden];
+    __shared__ uint16_t grad[kFeat];
     const int b = blockIdx.x, t = threadIdx.x & 127, h = threadIdx.x >> 7;
     if (h == 0) {
         float s = 0.0f;
@@ -141,12 +152,14 @@ __global__ __launch_bounds__(256) void head_backward_samples(
         dhid[b * kHidden + t] = s;
     }
     __syncthreads();
-    float s = 0.0f;
-#pragma unroll 16
-    for (int j = 64 * h; j < 64 * h + 64; ++j) s += w1[j * kFeat + t] * dh[j];
-    half[h][t] = s;
+    if (h == 0) {
+        float s = 0.0f;
+#pragma unroll 32
+        for (int j = 0; j < kHidden; ++j) s += w1[j * kFeat + t] * dh[j];
+        grad[t] = f2bf(s * (1.0f / 64.0f));
+    }
     __syncthreads();
-    const uint16_t g = f2bf((half[0][t] + half[1][t]) * (1.0f / 64.0f));
+    const uint16_t g = grad[t];
 #pragma unroll 8
     for (int p = h; p < 64; p += 2) {
         const size_t i = (static_cast<size_t>(b) * 64 + p) * kFeat + t;
@@ -157,7 +170,7 @@ __global__ __launch_bounds__(256) void head_backward_samples(
 // The head's weight gradients, sums over the batch in order: workgroup r <
 // 128 takes row r of W1 (and b1[r]), workgroup 128 + o row o of W2 (and b2[o]).
 // (One workgroup for the whole head, looping over samples and rows, took
-// 363 us for 24 samples; the two kernels take 8.)
+// 363 us for 24 samples; the two kernels take 10.)
 __global__ __launch_bounds__(128) void head_backward_weights(
     int n, const float *__restrict__ feat, const float *__restrict__ hid,
     const float *__restrict__ dout, const float *__restrict__ dhid, float *__restrict__ gw1,
@@ -306,7 +319,8 @@ struct Net {
     DeviceBuffer<uint16_t> act[kLayers + 1];   // act[0] = input slots (2 channels), act[l+1] = conv l output
     DeviceBuffer<uint16_t> dact[kLayers + 1];  // gradients w.r.t. act (masked); none for the input
     DeviceBuffer<float> partials;              // weight-gradient rows of every layer
-    size_t off_partial[kLayers];
+    DeviceBuffer<float> bias_partials;         // [kBiasSplits][channels] of every layer
+    size_t off_partial[kLayers], off_bias_partial[kLayers];
     DeviceBuffer<float> feat, hid, out, dout, dhid;
     bool weights_dirty = true;
 };
@@ -322,18 +336,28 @@ static size_t act_elems(int idx, int n) {  // idx 0 = input, idx l+1 = conv l ou
     return static_cast<size_t>(n) * e * e * e * c;
 }
 
-// A layer's weight-gradient partial rows: enough workgroups to fill the chip
-// without the rows' own traffic (55 KB - 0.9 MB each) growing past the
-// activations', never more than the chunks of positions there are.
-static int wgrad_rows(int layer, int n) {
-    static const int most[kLayers] = {1024, 512, 128, 64, 16};
-    const int chunks[kLayers] = {C0Tile<kW0Rows>::chunks(n), InTile<5, 16, 2, 1, 3>::chunks(n),
-                                 InTile<4, 32, 2, 1, 3>::chunks(n), InTile<3, 64, 8, 1, 1>::chunks(n),
-                                 InTile<2, 64, 4, 2, 2>::chunks(n)};
-    return std::min(most[layer], chunks[layer]);
+// How a layer's output positions are split for the weight gradient: one part per
+// 4,096 of them, at most 256, each a whole number of 32-position steps. Part of
+// the order of a gradient's sums (conv_wgrad), so nothing else decides it.
+struct WgradSplit {
+    int positions, per, rows;
+};
+static WgradSplit wgrad_split(int layer, int n) {
+    WgradSplit s;
+    const int e = out_edge(layer);
+    s.positions = n * e * e * e;
+    const int want = std::min(256, std::max(1, s.positions / 4096));
+    s.per = ((s.positions + want - 1) / want + 31) / 32 * 32;
+    s.rows = (s.positions + s.per - 1) / s.per;
+    return s;
+}
+// The most rows that batches up to n have.
+static int wgrad_max_rows(int layer, int n) {
+    const int e = out_edge(layer);
+    return std::min(256, std::max(1, n * e * e * e / 4096));
 }
 static int wgrad_row_len(int layer) {
-    return kCh[layer + 1] * 27 * (layer == 0 ? kCin0Used : kCh[layer]) + kCh[layer + 1];
+    return kCh[layer + 1] * 27 * (layer == 0 ? kCin0Used : kCh[layer]);
 }
 
 static void init_params(Net &net, uint64_t seed) {
@@ -403,12 +427,15 @@ Net *create(int max_batch, uint64_t seed) {
             if (i > 0) net->dact[i].alloc(act_elems(i, max_batch));
         }
         HIP_OK(hipMemsetAsync(net->act[0].ptr, 0, net->act[0].bytes(), backend().stream));
-        size_t partials = 0;
+        size_t partials = 0, bias_partials = 0;
         for (int l = 0; l < kLayers; ++l) {
             net->off_partial[l] = partials;
-            partials += static_cast<size_t>(wgrad_rows(l, max_batch)) * wgrad_row_len(l);
+            partials += static_cast<size_t>(wgrad_max_rows(l, max_batch)) * wgrad_row_len(l);
+            net->off_bias_partial[l] = bias_partials;
+            bias_partials += static_cast<size_t>(kBiasSplits) * kCh[l + 1];
         }
         net->partials.alloc(partials);
+        net->bias_partials.alloc(bias_partials);
         net->feat.alloc(static_cast<size_t>(max_batch) * kFeat);
         net->hid.alloc(static_cast<size_t>(max_batch) * kHidden);
         net->out.alloc(static_cast<size_t>(max_batch) * kOut);
@@ -487,16 +514,17 @@ static void launch_dgrad(Net &net, int layer, int n) {
     check_launch("cnn_conv_dgrad");
 }
 
-template <int LGDO, int CI, int CO, int R, int ZP, int KZN, int COW>
+template <int LGDO, int CI, int CO, int R, int ZP, int KZN, int COW, int CG>
 static void launch_wgrad(Net &net, int layer, int n) {
     using T = InTile<LGDO, CI, R, ZP, KZN * ZP>;
     constexpr size_t lds = T::kBytes + static_cast<size_t>(T::P) * (2 * COW + 16);
-    static_assert(lds <= 64 * 1024, "the staged chunk fits the default limit");
-    launch_kernel("cnn_conv_wgrad", conv_wgrad<LGDO, CI, CO, R, ZP, KZN, COW>,
-                  dim3(wgrad_rows(layer, n), (3 / KZN) * (CO / COW)), dim3(kConvLanes), lds,
+    const WgradSplit s = wgrad_split(layer, n);
+    auto kernel = conv_wgrad<LGDO, CI, CO, R, ZP, KZN, COW, CG>;
+    allow_lds(kernel, lds);
+    launch_kernel("cnn_conv_wgrad", kernel, dim3(s.rows, CG * (3 / KZN) * (CO / COW)), dim3(kConvLanes), lds,
                   static_cast<const uint16_t *>(net.act[layer].ptr),
                   static_cast<const uint16_t *>(net.dact[layer + 1].ptr),
-                  net.partials.ptr + net.off_partial[layer], T::chunks(n));
+                  net.partials.ptr + net.off_partial[layer], s.per, s.positions);
     check_launch("cnn_conv_wgrad");
 }
 
@@ -541,35 +569,41 @@ void backward(Net &net, int n, const float *dout_host) {
                   net.grads.ptr + net.off_w1, net.grads.ptr + net.off_b1, net.grads.ptr + net.off_w2,
                   net.grads.ptr + net.off_b2);
     check_launch("cnn_head_bwd");
-    launch_wgrad<2, 64, 128, 4, 2, 1, 64>(net, 4, n);
+    launch_wgrad<2, 64, 128, 4, 4, 1, 16, 3>(net, 4, n);
     launch_dgrad<2, 64, 128, 4, 4, 4, false>(net, 4, n);
-    launch_wgrad<3, 64, 64, 8, 1, 1, 64>(net, 3, n);
+    launch_wgrad<3, 64, 64, 8, 2, 1, 16, 3>(net, 3, n);
     launch_dgrad<3, 64, 64, 8, 1, 4, false>(net, 3, n);
-    launch_wgrad<4, 32, 64, 2, 1, 3, 32>(net, 2, n);
+    launch_wgrad<4, 32, 64, 8, 1, 1, 32, 3>(net, 2, n);
     launch_dgrad<4, 32, 64, 8, 1, 1, false>(net, 2, n);
-    launch_wgrad<5, 16, 32, 2, 1, 3, 32>(net, 1, n);
+    launch_wgrad<5, 16, 32, 4, 1, 1, 32, 1>(net, 1, n);
     launch_dgrad<5, 16, 32, 4, 1, 1, true>(net, 1, n);
-    launch_kernel("cnn_conv_wgrad", conv0_wgrad, dim3(wgrad_rows(0, n)), dim3(kConvLanes), 0,
-                  input_words(net), static_cast<const uint16_t *>(net.dact[1].ptr),
-                  net.partials.ptr + net.off_partial[0], C0Tile<kW0Rows>::chunks(n));
+    const WgradSplit s0 = wgrad_split(0, n);
+    if (s0.per % (kW0Rows * 64) != 0) fail(SITKHIP_ERR_DRIVER, "first-layer splits are not whole chunks");
+    launch_kernel("cnn_conv_wgrad", conv0_wgrad, dim3(s0.rows), dim3(kW0Lanes), 0, input_words(net),
+                  static_cast<const uint16_t *>(net.dact[1].ptr), net.partials.ptr + net.off_partial[0],
+                  s0.per, s0.positions);
     check_launch("conv0_wgrad");
+    BiasLayers bias;
+    for (int l = 0; l < kLayers; ++l)
+        bias.l[l] = {net.dact[l + 1].ptr, net.bias_partials.ptr + net.off_bias_partial[l],
+                     wgrad_split(l, n).positions, kCh[l + 1]};
+    launch_kernel("cnn_bias_grad", bias_grad, dim3(kBiasSplits, kLayers), dim3(kConvLanes), 0, bias);
+    check_launch("bias_grad");
     PartialJobs jobs;
-    jobs.n = kLayers;
+    jobs.n = 0;
     unsigned blocks = 0;
+    auto add = [&](const float *p, float *out, int rows, int len, int inner, int ld) {
+        jobs.j[jobs.n++] = {p, out, rows, len, inner, ld, blocks};
+        blocks += static_cast<unsigned>((len + kPartialLanes - 1) / kPartialLanes);
+    };
     for (int l = 0; l < kLayers; ++l) {
-        PartialRows &q = jobs.j[l];
-        q.p = net.partials.ptr + net.off_partial[l];
-        q.out = net.grads.ptr + net.off_w[l];
-        q.out_bias = net.grads.ptr + net.off_b[l];
-        q.rows = wgrad_rows(l, n);
-        q.total = wgrad_row_len(l);
-        q.len = q.total - kCh[l + 1];
-        q.inner = l == 0 ? kCin0Used : q.len;
-        q.ld = l == 0 ? kCin0 : q.len;
-        q.first_block = blocks;
-        blocks += static_cast<unsigned>((q.total + 63) / 64);
+        const int len = wgrad_row_len(l);
+        add(net.partials.ptr + net.off_partial[l], net.grads.ptr + net.off_w[l], wgrad_split(l, n).rows, len,
+            l == 0 ? kCin0Used : len, l == 0 ? kCin0 : len);
+        add(net.bias_partials.ptr + net.off_bias_partial[l], net.grads.ptr + net.off_b[l], kBiasSplits,
+            kCh[l + 1], kCh[l + 1], kCh[l + 1]);
     }
-    launch_kernel("cnn_sum_partials", reduce_partials, dim3(blocks), dim3(kConvLanes), 0, jobs);
+    launch_kernel("cnn_sum_partials", reduce_partials, dim3(blocks), dim3(kPartialLanes), 0, jobs);
     check_launch("reduce_partials");
     sync();
 }
