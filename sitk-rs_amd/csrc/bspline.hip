@@ -227,15 +227,25 @@ __device__ __forceinline__ void map_point_cell(const BSplineMap &B, const double
     apply_post_stage(B, p);
 }
 
+// Where weight k (of 12) of sample s lies: twelve planes of the n samples in the
+// cell-grouped order (SOA), so that a wave reads each as one run where twelve
+// together per sample would spread its load over 48 cache lines; the twelve
+// together in cells of few samples (below kDenseCell), which span few lines
+// either way and are read in six loads (12 samples a cell, 4,096 cells, 16 starts:
+// bs_value 334 us against 365).
+template <bool SOA>
+__device__ __forceinline__ const double *weights_of(const double *__restrict__ wts, size_t s) {
+    return wts + (SOA ? s : s * 12);
+}
+
 // The support weights of every sample of a cell (they depend only on the
-// fixed point), computed once: w[k][s], twelve planes of the n samples in the
-// cell-grouped order, so that a wave reads each as one run (twelve together per
-// sample spread a wave's load over 48 cache lines).
+// fixed point), computed once, weight k of sample s at s * ss + k * ks.
 // A sample whose support on the device is not its cell's (the grouping was
 // made on the host) raises *mismatch.
 __global__ void bs_weights(FixedGrid F, BSplineMap B, const ChainConst *__restrict__ C,
                            const uint32_t *__restrict__ idx, const int *__restrict__ cell_begin,
-                           int ncells, size_t n, double *__restrict__ wts, int *__restrict__ mismatch) {
+                           int ncells, size_t ss, size_t ks, double *__restrict__ wts,
+                           int *__restrict__ mismatch) {
     const int cell = blockIdx.y;
     const int m0 = B.gs[0] - 3, m1 = B.gs[1] - 3;
     const int sx = cell % m0, sy = (cell / m0) % m1, sz = cell / (m0 * m1);
@@ -250,16 +260,24 @@ __global__ void bs_weights(FixedGrid F, BSplineMap B, const ChainConst *__restri
 #pragma unroll
         for (int d = 0; d < 3; ++d)
 #pragma unroll
-            for (int k = 0; k < 4; ++k) wts[(d * 4 + k) * n + s] = w[d][k];
+            for (int k = 0; k < 4; ++k) wts[s * ss + (d * 4 + k) * ks] = w[d][k];
     }
+}
+
+// Part `part` of `parts` of the samples [b, e).
+__device__ __forceinline__ void cell_part(int &b, int &e, int part, int parts) {
+    const int len = (e - b + parts - 1) / parts;
+    b += part * len;
+    e = min(b + len, e);
 }
 
 // Value pass, `cpb` cells per workgroup (the last bucket, cell == ncells,
 // holds the samples outside the valid region): the cell's support
 // coefficients in LDS, the joint histogram in LDS, one record per sample (the
 // moving value and its index gradient, NaN value = dropped) for the
-// derivative pass. Any grouping gives the same integer histogram.
-template <typename R>
+// derivative pass. Any grouping gives the same integer histogram; with few
+// starts a cell's samples are shared by `parts` workgroups.
+template <typename R, bool SOA>
 __global__ __launch_bounds__(kBlock) void bs_value(FixedGrid F, MovingVol M, BSplineMap B0,
                                                    const double *__restrict__ coef,
                                                    const double *__restrict__ stage,
@@ -281,21 +299,24 @@ __global__ __launch_bounds__(kBlock) void bs_value(FixedGrid F, MovingVol M, BSp
     unsigned long long *h_joint = s_hist, *h_marg = s_hist + P.bins * P.bins;
     SampleRec<R> *r = rec + static_cast<size_t>(st) * n;
     for (int i = threadIdx.x; i < nb; i += kBlock) s_hist[i] = 0ull;
+    const int group = blockIdx.y, part = blockIdx.z, parts = gridDim.z;
     for (int q = 0; q < cpb; ++q) {
-        const int cell = blockIdx.y * cpb + q;
+        const int cell = group * cpb + q;
         if (cell > ncells) break;  // the same for every lane
         __syncthreads();           // the previous cell's coefficients are no longer read
         if (cell < ncells) stage_cell_coefs(B, cell, s_coef);
         __syncthreads();
-        const int e = cell_begin[cell + 1];
-        for (int s = cell_begin[cell] + threadIdx.x; s < e; s += kBlock) {
+        int b = cell_begin[cell], e = cell_begin[cell + 1];
+        if (parts > 1) cell_part(b, e, part, parts);
+        for (int s = b + threadIdx.x; s < e; s += kBlock) {
             const int fb = fbin[s];
             Cell cl;
             bool ok = false;
             if (fb != kNoBin) {
                 double x[3], p[3];
                 fixed_point(F, *C, idx[s], x);
-                map_point_cell(B, x, cell < ncells, wts + s, static_cast<size_t>(n), s_coef, p);
+                map_point_cell(B, x, cell < ncells, weights_of<SOA>(wts, s), SOA ? static_cast<size_t>(n) : 1, s_coef,
+                               p);
                 ok = locate(M, *C, p, cl);
             }
             if (!ok) {
@@ -311,7 +332,7 @@ __global__ __launch_bounds__(kBlock) void bs_value(FixedGrid F, MovingVol M, BSp
         }
     }
     __syncthreads();
-    const unsigned copy = (blockIdx.y * gridDim.x + blockIdx.x) % kHistCopies;
+    const unsigned copy = ((blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x) % kHistCopies;
     g_joint += (static_cast<size_t>(st) * kHistCopies + copy) * P.bins * P.bins;
     g_marg += (static_cast<size_t>(st) * kHistCopies + copy) * P.bins;
     for (int i = threadIdx.x; i < nb; i += kBlock) {
@@ -330,9 +351,25 @@ struct CellMap {
     double Q[9];
 };
 
-// The FP32 path's value pass: the same cells, histogram and records, the
-// displacement and the index composed with fused multiply-adds, kCellU samples
-// per lane. The displacement is summed along x, then y, then z (252 FMAs instead of
+// Displacement in moving voxels below which the composed sum's rounding (some
+// 20 FP64 roundings of terms up to 3 kFar: 1e-7) stays under kGuard.
+constexpr double kFar = 16777216.0;
+
+// Samples per cell (the mean of those that hold any) from which the FP32 value
+// pass below is the faster one, a property of the metric, so that a start gets the
+// same bits alone as among others. A cell of few samples fills only some of its
+// workgroup's lanes and waits for its 192 coefficients, which come faster to LDS in
+// one load per lane than as scalars. Times in us of bs_value (the general pass) / one
+// sample per lane / two, 32 bins: 26 a cell, 729 cells, 16 and 48 starts 70, 183 /
+// 94, 289 / 137, 410; 288 a cell, 729 cells, 4 and 16 starts 51, 158 / 57, 162 / 66,
+// 185; 748 a cell, 729 cells, 4 and 16 starts 92, 308 / 91, 262 / 99, 306; 2,064 a
+// cell, 343 cells, 16 and 64 starts 415, 1,337 / 365, 1,294 / 361, 1,218; 20,192 a
+// cell, 27 cells, 4 and 16 starts 346, 1,293 / 247, 918 / 189, 693.
+constexpr int kDenseCell = 512, kPairCell = 1024;
+
+// The FP32 path's value pass where cells hold many samples (kDenseCell): the same
+// cells, histogram and records, the displacement and the index composed with fused
+// multiply-adds, kCellU samples per lane. The displacement is summed along x, then y, then z (252 FMAs instead of
 // 64 weight products and 192 rounded multiply-adds), and a cell's coefficients
 // come as scalar loads -- a multiply-add takes one operand from a scalar
 // register -- where LDS broadcasts took 192 reads per sample. A sample whose
@@ -344,20 +381,16 @@ struct CellMap {
 // one start 53, now 42. The vector pipes issue 54 % of the many starts' time and
 // the texture path is busy 65 % (the eight corners of 64 scattered samples).
 // Two samples per lane share a coefficient load and take 230 registers, two waves
-// per SIMD; few starts, whose workgroups are short of samples, take one at three
-// waves: one start 42 us against 47, 64 starts 1,290 against 1,240. (A bound of
-// three waves on two samples spills: 2,076; one of two waves costs 1,320.)
-// Displacement in moving voxels below which the composed sum's rounding (some
-// 20 FP64 roundings of terms up to 3 kFar: 1e-7) stays under kGuard.
-constexpr double kFar = 16777216.0;
-
+// per SIMD: worth it from kPairCell samples per cell on and with four starts or
+// more; otherwise one, at three waves. (A bound of three waves on two samples
+// spills: 2,076 us; one of two waves costs 1,320.)
 template <int kCellU>
 __global__ __launch_bounds__(kBlock, kCellU == 1 ? 3 : 1) void bs_value_f32(
     FixedGrid F, MovingVol M, BSplineMap B0, const double *__restrict__ coef,
     const double *__restrict__ stage, const CellMap *__restrict__ maps, CellMap own,
     const int *__restrict__ active, const ChainConst *__restrict__ C, const uint32_t *__restrict__ idx,
     const uint8_t *__restrict__ fbin, const int *__restrict__ cell_begin, const double *__restrict__ wts,
-    int ncells, int cpb, int parts, MattesParams P, unsigned long long *__restrict__ g_joint,
+    int ncells, int cpb, MattesParams P, unsigned long long *__restrict__ g_joint,
     unsigned long long *__restrict__ g_marg, SampleRec<float> *__restrict__ rec, long long n) {
     extern __shared__ unsigned long long s_hist[];
     __shared__ double s_coef[192];
@@ -368,7 +401,7 @@ __global__ __launch_bounds__(kBlock, kCellU == 1 ? 3 : 1) void bs_value_f32(
     unsigned long long *h_joint = s_hist, *h_marg = s_hist + P.bins * P.bins;
     SampleRec<float> *r = rec + static_cast<size_t>(st) * n;
     for (int i = threadIdx.x; i < nb; i += kBlock) s_hist[i] = 0ull;
-    const int group = blockIdx.y / parts, part = blockIdx.y % parts;
+    const int group = blockIdx.y, part = blockIdx.z, parts = gridDim.z;
     const int g0 = B0.gs[0], g01 = B0.gs[0] * B0.gs[1], m0 = B0.gs[0] - 3, m1 = B0.gs[1] - 3;
     double qmax = 0.0;
     for (int k = 0; k < 9; ++k) qmax = fmax(qmax, fabs(cm.Q[k]));
@@ -384,9 +417,8 @@ __global__ __launch_bounds__(kBlock, kCellU == 1 ? 3 : 1) void bs_value_f32(
             if (threadIdx.x < 192) far = !(fabs(s_coef[threadIdx.x]) * qmax < kFar);
         }
         const double unsure = __syncthreads_or(far) ? static_cast<double>(NAN) : 0.0;
-        const int cb = cell_begin[cell], ce = cell_begin[cell + 1];
-        const int len = (ce - cb + parts - 1) / parts;
-        const int b = cb + part * len, e = min(b + len, ce);
+        int b = cell_begin[cell], e = cell_begin[cell + 1];
+        if (parts > 1) cell_part(b, e, part, parts);
         // read-only for the whole launch: constant address space, scalar loads
         typedef const __attribute__((address_space(4))) double *ConstPtr;
         const ConstPtr cf = (ConstPtr)(coef + static_cast<size_t>(st) * 3 * B0.ncp + cell % m0 +
@@ -499,7 +531,7 @@ __global__ __launch_bounds__(kBlock, kCellU == 1 ? 3 : 1) void bs_value_f32(
         }
     }
     __syncthreads();
-    const unsigned copy = (blockIdx.y * gridDim.x + blockIdx.x) % kHistCopies;
+    const unsigned copy = ((blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x) % kHistCopies;
     g_joint += (static_cast<size_t>(st) * kHistCopies + copy) * P.bins * P.bins;
     g_marg += (static_cast<size_t>(st) * kHistCopies + copy) * P.bins;
     for (int i = threadIdx.x; i < nb; i += kBlock) {
@@ -555,7 +587,7 @@ __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_wave_barrier();
 }
 
-template <typename R>
+template <typename R, bool SOA>
 __global__ __launch_bounds__(kBlock) void bs_deriv(FixedGrid F, MovingVol M, BSplineMap B0,
                                                    const double *__restrict__ stage,
                                                    const CellMap *__restrict__ maps, CellMap own,
@@ -600,7 +632,7 @@ __global__ __launch_bounds__(kBlock) void bs_deriv(FixedGrid F, MovingVol M, BSp
             rr = r[s];
             fb = fbin[s];
 #pragma unroll
-            for (int k = 0; k < 12; ++k) w[k] = wts[static_cast<size_t>(k) * n + s];
+            for (int k = 0; k < 12; ++k) w[k] = weights_of<SOA>(wts, s)[SOA ? static_cast<size_t>(k) * n : k];
         };
         if (b < e) fetch(b + threadIdx.x);
         for (int s0 = b; s0 < e; s0 += kBlock) {
@@ -712,6 +744,8 @@ struct BSplineMetric {
     BSplineMap B{};             // coef unused: every evaluation brings its coefficients
     int ncells = 0;
     int parts = 1;              // parts of a cell in the derivative pass
+    int fill = 0;               // samples per cell, over the cells that hold any
+    bool soa = false;           // layout of wts (weights_of): the cells are dense
     SampleSet SS{};             // cell-grouped samples
     DeviceBuffer<uint32_t> idx;
     DeviceBuffer<uint8_t> fbin;
@@ -780,6 +814,9 @@ BSplineMetric *bspline_create(Metric &m, const size_t gs[3], const double origin
             cell[s] = c;
             ++count[c];
         }
+        const auto held = b->ncells - std::count(count.begin(), count.end() - 1, 0);
+        b->fill = held > 0 ? static_cast<int>((n - count[b->ncells]) / held) : 0;
+        b->soa = b->fill >= kDenseCell;
         // about four rounds of a workgroup's lanes per part
         b->parts = std::max(1, std::min(8, (*std::max_element(count.begin(), count.end()) + 4 * kBlock - 1) /
                                                (4 * kBlock)));
@@ -809,8 +846,8 @@ BSplineMetric *bspline_create(Metric &m, const size_t gs[3], const double origin
             DeviceBuffer<int> bad(1);
             HIP_OK(hipMemsetAsync(bad.ptr, 0, sizeof(int), backend().stream));
             hipLaunchKernelGGL(bs_weights, dim3(8, b->ncells), dim3(256), 0, backend().stream, m.F,
-                               b->B, m.chain.ptr, b->idx.ptr, b->cell_begin.ptr, b->ncells, n,
-                               b->wts.ptr, bad.ptr);
+                               b->B, m.chain.ptr, b->idx.ptr, b->cell_begin.ptr, b->ncells,
+                               b->soa ? size_t{1} : size_t{12}, b->soa ? n : size_t{1}, b->wts.ptr, bad.ptr);
             check_launch("bs_weights");
             int flag = 0;
             HIP_OK(hipMemcpyAsync(&flag, bad.ptr, sizeof(int), hipMemcpyDeviceToHost, backend().stream));
@@ -993,22 +1030,25 @@ static void multi_passes(BSplineMulti &u, const int *active, int nact, bool deri
     // so that one start's cells fill the chip
     const int cpb = nact >= 16 ? kCellsPerBlockMany : 1;
     const unsigned groups = static_cast<unsigned>((b.ncells + 1 + cpb - 1) / cpb);
-    if constexpr (sizeof(R) == 4) {
-        const int vparts = nact >= 4 ? 1 : b.parts;
-        auto kernel = nact >= 4 ? bs_value_f32<2> : bs_value_f32<1>;
-        launch_kernel("bs_value", kernel, dim3(nact, groups * vparts), dim3(kBlock), shm, m.F, m.Mv, b.B,
+    const unsigned vparts = nact >= 4 ? 1 : b.parts;
+    if (sizeof(R) == 4 && b.soa) {
+        auto kernel = nact >= 4 && b.fill >= kPairCell ? bs_value_f32<2> : bs_value_f32<1>;
+        launch_kernel("bs_value_f32", kernel, dim3(nact, groups, vparts), dim3(kBlock), shm, m.F, m.Mv, b.B,
                       static_cast<const double *>(u.coef.ptr), stage, maps, own, active,
                       static_cast<const ChainConst *>(m.chain.ptr), static_cast<const uint32_t *>(b.idx.ptr),
                       static_cast<const uint8_t *>(b.fbin.ptr), static_cast<const int *>(b.cell_begin.ptr),
-                      static_cast<const double *>(b.wts.ptr), b.ncells, cpb, vparts, m.P, u.joint.ptr,
-                      u.marg.ptr, rec, b.SS.n);
+                      static_cast<const double *>(b.wts.ptr), b.ncells, cpb, m.P, u.joint.ptr,
+                      u.marg.ptr, reinterpret_cast<SampleRec<float> *>(u.rec.ptr), b.SS.n);
     } else {
-        launch_kernel("bs_value", bs_value<R>, dim3(nact, groups), dim3(kBlock), shm, m.F, m.Mv, b.B,
+        auto kernel = bs_value<R, false>;
+        if constexpr (sizeof(R) == 8)
+            if (b.soa) kernel = bs_value<R, true>;
+        launch_kernel("bs_value", kernel, dim3(nact, groups, vparts), dim3(kBlock), shm, m.F, m.Mv, b.B,
                       static_cast<const double *>(u.coef.ptr), stage, active,
                       static_cast<const ChainConst *>(m.chain.ptr), static_cast<const uint32_t *>(b.idx.ptr),
                       static_cast<const uint8_t *>(b.fbin.ptr), static_cast<const int *>(b.cell_begin.ptr),
-                      static_cast<const double *>(b.wts.ptr), b.ncells, cpb, m.P, u.joint.ptr, u.marg.ptr, rec,
-                      b.SS.n);
+                      static_cast<const double *>(b.wts.ptr), b.ncells, cpb, m.P, u.joint.ptr,
+                      u.marg.ptr, rec, b.SS.n);
     }
     check_launch("bs_value");
     {
@@ -1026,7 +1066,7 @@ static void multi_passes(BSplineMulti &u, const int *active, int nact, bool deri
     const size_t ratio_all = static_cast<size_t>(B) * B * sizeof(R);
     const size_t ratio_bytes = ratio_all <= kRatioLds ? ratio_all : 0;
     if (b.ncells > 0) {
-        launch_kernel("bs_deriv", bs_deriv<R>, dim3(nact, b.ncells * rows), dim3(kBlock), ratio_bytes, m.F, m.Mv, b.B,
+        launch_kernel("bs_deriv", b.soa ? bs_deriv<R, true> : bs_deriv<R, false>, dim3(nact, b.ncells * rows), dim3(kBlock), ratio_bytes, m.F, m.Mv, b.B,
                       stage, maps, own, active, static_cast<const int *>(b.cell_begin.ptr),
                       static_cast<const double *>(b.wts.ptr), static_cast<const uint8_t *>(b.fbin.ptr), m.P, pr,
                       static_cast<const SampleRec<R> *>(rec), b.SS.n, b.parts, rows < b.parts, ratio_bytes > 0,

@@ -303,3 +303,46 @@ def test_cells_cut_into_parts_against_the_oracle(hip, bins, shape, mesh, kind):
         vals, ders, valid = multi.value_and_derivative(np.stack([coeffs] * starts))
         for s in (0, starts - 1):
             assert vals[s] == v and valid[s] == n and np.array_equal(ders[s], d), (starts, s)
+
+
+@pytest.mark.parametrize("precision,shape,mesh,dense",
+                         [(0, (22, 20, 18), (3, 3, 3), False), (0, (36, 32, 34), (7, 6, 7), False),
+                          (0, (24, 24, 24), (3, 3, 2), True), (0, (30, 28, 26), (2, 3, 2), True),
+                          (1, (22, 20, 18), (3, 3, 3), False), (1, (30, 28, 26), (2, 3, 2), True)])
+def test_the_value_pass_by_samples_per_cell(hip, precision, shape, mesh, dense):
+    """Cells of few samples (about 130 and 290) take the general FP32 value pass:
+    the one that reads a cell's coefficients as scalars took up to 2.3 times as
+    long there. Cells of 768 and 1,820 take the latter, with one sample per lane
+    and, for four starts, two in the fuller ones; FP64 always takes the general
+    pass, from either layout of the weights. Each against the oracle, and a start
+    alone with the same bits as among others."""
+    nx, ny, nz = shape
+    f = blob_volume((nz, ny, nx), 8, spacing=SP)
+    m = blob_volume((nz, ny, nx), 9, spacing=SP) * 0.4 + f * 0.6
+    df = hip.DeviceImage.upload(f, spacing=SP, origin=ORG)
+    dm = hip.DeviceImage.upload(m, spacing=SP, origin=ORG)
+    met = hip.ResidentMattes(df, dm, bins=24, precision=precision)
+    ncp = int(np.prod([k + 3 for k in mesh]))
+    coeffs = np.random.default_rng(3).normal(0.0, 0.5, 3 * ncp)
+    t = O.make_bspline(list(shape), SP, ORG, np.eye(3), mesh, coeffs)
+    bs = hip.BSplineMattes(met, list(t.grid_size), list(t.grid_origin), list(t.grid_spacing),
+                           np.array(list(t.grid_direction)).reshape(3, 3))
+    stage = np.concatenate([np.eye(3).reshape(9), np.zeros(3)])
+    bs.set_moving_initial(stage)
+    hip.profile_enable(True)
+    try:
+        hip.profile_reset()
+        v, d, n = bs.value_and_derivative(coeffs)
+        scalar, passes = hip.profile_query("bs_value_f32")[0], hip.profile_query("bs_value")[0]
+    finally:
+        hip.profile_enable(False)
+    assert (scalar, passes) == (1 if dense and precision == 0 else 0, 1)
+    pb = O.MetricProblem(f, SP, ORG, m, SP, ORG)
+    want_v, want_d, want_n = pb.mattes_evaluate(pb.mattes_geometry(24), t)
+    tv, td = (1e-9, 1e-7) if precision == 1 else (1e-6, 1e-4)
+    assert n == want_n and abs(v - want_v) <= tv * abs(want_v), (v, want_v)
+    assert rel_vec(d, want_d) < td, rel_vec(d, want_d)
+    multi = hip.BSplineMulti(bs, 4, np.stack([stage] * 4))
+    vals, ders, valid = multi.value_and_derivative(np.stack([coeffs] * 4))
+    for s in (0, 3):
+        assert vals[s] == v and valid[s] == n and np.array_equal(ders[s], d), s
