@@ -1585,20 +1585,20 @@ void mattes_value_and_moments(Metric &m, const double *stages, int nstage, doubl
     if (valid) *valid = static_cast<size_t>(t.valid);
 }
 
-// The column walk of a grid metric. Its tiles: as many planes each as make
-// about two kGrid workgroups (256^3: 59 us; one kGrid 61), at least the planes
-// of one step.
+// The column walk of a grid metric. Its tiles: as many planes each as make about
+// kGrid workgroups. (Twice as many make the pass of 256^3 2 us shorter, 59 for 61,
+// but the fold of their rows as much longer, and at 96^3, tiles of two planes, pass
+// and fold take 15.4 us against 12.6; ms_range 13.9.)
 template <bool MOM>
 static void launch_ms_columns(Metric &m, const Stages &S) {
     constexpr int NS = MOM ? 14 : 2;
     const ColumnTiles one = column_tiles(m.F, 1);
-    const ColumnTiles T =
-        column_tiles(m.F, std::max(kColumnU, static_cast<int>((one.tiles + 2 * kGrid - 1) / (2 * kGrid))));
+    const ColumnTiles T = column_tiles(m.F, std::max(kColumnU, static_cast<int>((one.tiles + kGrid - 1) / kGrid)));
     const size_t need = static_cast<size_t>(T.tiles) * NS;
     if (m.partials.len < need) m.partials.alloc(need);
     const IndexMap X = make_index_map(m.F, m.Mv, S.s, S.n);
     const dim3 grid((T.tiles + 7) / 8 * 8);
-    const char *name = MOM ? "ms_moments" : "ms_value";
+    const char *name = MOM ? "ms_moments_columns" : "ms_value_columns";
     auto go = [&](const auto &map) {
         using Map = std::decay_t<decltype(map)>;
         launch_kernel(name, ms_columns_pass<MOM, Map>, grid, dim3(kBlock), 0, m.F, m.Mv, map, X,
