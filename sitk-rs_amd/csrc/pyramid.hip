@@ -88,7 +88,9 @@ __device__ __forceinline__ bool resample_cindex(const GridMap &G, const Map &S, 
 // are neither read nor weighed, and voxels that all fall on voxels, as those of a
 // grid placed on its own or on every second voxel do, are read alone. us a call,
 // 256 x 256 x 128: onto itself 51 with each corner behind its test, 62 with all
-// eight, 41 now; finer along x alone (400 x 256 x 128) 75, 92, 71; rotated 88, 76, 63.
+// eight, 48 now; finer along x alone (400 x 256 x 128) 74, 92, 75; rotated 88, 76, 68.
+// (Waves that weigh all eight have a path of their own: with the tests of the
+// others in it the 64 volumes took 126, now 116.)
 template <typename Map>
 __device__ __forceinline__ float linear_voxel(const float *__restrict__ in, const GridMap &G,
                                               const Map &S, double dflt, uint32_t o) {
@@ -104,43 +106,58 @@ __device__ __forceinline__ float linear_voxel(const float *__restrict__ in, cons
             frac[d] = c[d] - f;
         }
         const int n0 = G.in_size[0], n1 = G.in_size[1], n2 = G.in_size[2];
-        // (frac < 1: only an upper corner's weight can be zero)
-        const bool up0 = __any(frac[0] != 0.0), up1 = __any(frac[1] != 0.0), up2 = __any(frac[2] != 0.0);
-        if (!(up0 || up1 || up2))  // voxels on voxels
-            return static_cast<float>(
-                0.0 + static_cast<double>(in[(static_cast<size_t>(base[2]) * n1 + base[1]) * n0 + base[0]]));
         const long long st1 = n0, st2 = static_cast<long long>(n0) * n1;
         const int p = min(max(base[0], 0), max(n0 - 2, 0));
-        const bool row[4] = {true, up1, up2, up1 && up2};
+        const long long y0 = clampi(base[1], 0, n1 - 1) * st1, y1 = clampi(base[1] + 1, 0, n1 - 1) * st1;
+        const long long z0 = clampi(base[2], 0, n2 - 1) * st2, z1 = clampi(base[2] + 1, 0, n2 - 1) * st2;
+        const float *rows[4] = {in + (z0 + y0 + p), in + (z0 + y1 + p), in + (z1 + y0 + p),
+                                in + (z1 + y1 + p)};
+        // (frac < 1: only an upper corner's weight can be zero)
+        const bool up0 = __any(frac[0] != 0.0), up1 = __any(frac[1] != 0.0), up2 = __any(frac[2] != 0.0);
         float q[8];
-        const float *at = in + (clampi(base[1], 0, n1 - 1) * st1 + clampi(base[2], 0, n2 - 1) * st2 + p);
-        // to the upper row along y and z: none past a face
-        const long long dy = base[1] >= 0 && base[1] < n1 - 1 ? st1 : 0;
-        const long long dz = base[2] >= 0 && base[2] < n2 - 1 ? st2 : 0;
-        if (n0 >= 2) {
-            FloatPair w[4] = {};
-#pragma unroll
-            for (int k = 0; k < 4; ++k)
-                if (row[k])
-                    w[k] = *reinterpret_cast<const FloatPair *>(at + (k & 1 ? dy : 0) + (k & 2 ? dz : 0));
-            const bool hi = base[0] > p, lo = base[0] < p;  // both corners the pair's last / first
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                q[2 * k] = hi ? w[k].b : w[k].a;
-                q[2 * k + 1] = lo ? w[k].a : w[k].b;
-            }
-        } else {
-#pragma unroll
-            for (int k = 0; k < 4; ++k) q[2 * k] = q[2 * k + 1] = at[(k & 1 ? dy : 0) + (k & 2 ? dz : 0)];
-        }
         double acc = 0.0;
-#pragma unroll
-        for (int corner = 0; corner < 8; ++corner) {
-            if (!row[corner >> 1] || ((corner & 1) && !up0)) continue;
+        auto pair = [&](int k) {
+            const FloatPair w = *reinterpret_cast<const FloatPair *>(rows[k]);
+            q[2 * k] = w.a;
+            q[2 * k + 1] = w.b;
+        };
+        auto faces = [&](int k) {  // past a face both corners are the pair's last / first
+            const float a = q[2 * k], b = q[2 * k + 1];
+            q[2 * k] = base[0] > p ? b : a;
+            q[2 * k + 1] = base[0] < p ? a : b;
+        };
+        auto weigh = [&](int corner) {
             double weight = 1.0;
 #pragma unroll
             for (int d = 0; d < 3; ++d) weight *= (corner >> d) & 1 ? frac[d] : (1.0 - frac[d]);
             if (weight != 0.0) acc += weight * static_cast<double>(q[corner]);
+        };
+        if (n0 < 2) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) q[2 * k] = q[2 * k + 1] = *rows[k];
+#pragma unroll
+            for (int corner = 0; corner < 8; ++corner) weigh(corner);
+        } else if (up0 && up1 && up2) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) pair(k);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) faces(k);
+#pragma unroll
+            for (int corner = 0; corner < 8; ++corner) weigh(corner);
+        } else if (!(up0 || up1 || up2)) {  // voxels on voxels
+            acc += static_cast<double>(rows[0][base[0] - p]);
+        } else {
+            const bool row[4] = {true, up1, up2, up1 && up2};
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                if (row[k]) pair(k);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                if (!row[k]) continue;
+                faces(k);
+                weigh(2 * k);
+                if (up0) weigh(2 * k + 1);
+            }
         }
         v = acc;
     }
