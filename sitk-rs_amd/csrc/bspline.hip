@@ -171,6 +171,8 @@ __device__ __forceinline__ BSplineMap start_map(const BSplineMap &B0, const doub
     return B;
 }
 
+// Up to this many starts, a cell's parts are workgroups of their own.
+constexpr int kFewStarts = 3;
 // Cells per value-pass workgroup: 4 when many starts fill the chip, else 1.
 constexpr int kCellsPerBlockMany = 4;
 
@@ -559,7 +561,7 @@ __global__ __launch_bounds__(kTail) void bs_tail(const int *__restrict__ active,
 // Derivative pass, one workgroup per (part of a cell, start), from the value
 // pass's records: per valid sample the pRatio-weighted B3' sum a times the moving
 // gradient (through the stage's transposed matrix when there is one), g_d;
-// then out[cell][16 n + m] = sum over the cell's samples of u_m t_n with
+// then out[start's place in the launch][cell][part][16 n + m] = sum over the cell's samples of u_m t_n with
 // u_m = w0[m % 4] w1[m / 4] and t_n = g_{n / 4} w2[n % 4] (n < 12), i.e.
 // out[d * 64 + k * 16 + j * 4 + i] = sum of g_d w0[i] w1[j] w2[k]. The sum
 // is a 16 x 4 by 4 x 16 FP64 matrix product per four samples
@@ -597,18 +599,17 @@ __global__ __launch_bounds__(kBlock) void bs_deriv(FixedGrid F, MovingVol M, BSp
                                                    const uint8_t *__restrict__ fbin,
                                                    MattesParams P, const R *__restrict__ pratio,
                                                    const SampleRec<R> *__restrict__ rec, long long n,
-                                                   int parts, bool together, bool ratio_in_lds,
-                                                   double *__restrict__ out) {
+                                                   int parts, bool ratio_in_lds, double *__restrict__ out) {
     __shared__ double s_x[kBlock / 64][64][17];  // per lane: w[3][4], g[3], pad
     extern __shared__ double s_ratio[];          // pRatio, when the launch has room for it
     const int st = active[blockIdx.x];
     const BSplineMap B = start_map(B0, nullptr, stage, st);
     const SampleRec<R> *r = rec + static_cast<size_t>(st) * n;
     pratio += static_cast<size_t>(st) * P.bins * P.bins;
-    // one part per workgroup, or all parts of a cell in turn (`together`), added
-    // in the same order
-    const int cell = together ? blockIdx.y : blockIdx.y / parts;
-    const int p0 = together ? 0 : blockIdx.y % parts, p1 = together ? parts : p0 + 1;
+    // one part per workgroup (gridDim.z of them), or all parts of a cell in turn,
+    // added in the same order
+    const int cell = blockIdx.y;
+    const int p0 = blockIdx.z, p1 = gridDim.z > 1 ? p0 + 1 : parts;
     const int cb = cell_begin[cell], ce = cell_begin[cell + 1];
     const int len = (ce - cb + parts - 1) / parts;
     const CellMap cm = maps ? maps[st] : own;
@@ -702,7 +703,8 @@ __global__ __launch_bounds__(kBlock) void bs_deriv(FixedGrid F, MovingVol M, BSp
         __syncthreads();  // the next part's samples go where the tiles were
     }
     if (threadIdx.x < 192)
-        out[(static_cast<size_t>(st) * gridDim.y + blockIdx.y) * 192 + threadIdx.x] = total;
+        out[((static_cast<size_t>(blockIdx.x) * gridDim.y + cell) * gridDim.z + blockIdx.z) * 192 +
+            threadIdx.x] = total;
 }
 
 // deriv[d][cp] = sum over the (up to 64) cells whose support holds cp and their
@@ -714,7 +716,7 @@ __global__ __launch_bounds__(256) void bs_gather(BSplineMap B, const int *__rest
                                                  int parts, const double *__restrict__ cellT,
                                                  double *__restrict__ deriv) {
     const int st = active[blockIdx.y];
-    cellT += static_cast<size_t>(st) * ncells * parts * 192;
+    cellT += static_cast<size_t>(blockIdx.y) * ncells * parts * 192;
     deriv += static_cast<size_t>(st) * 3 * B.ncp;
     const int cp = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (cp >= B.ncp) return;
@@ -743,7 +745,7 @@ struct BSplineMetric {
     Metric *m = nullptr;        // the Mattes metric (bins set); not owned
     BSplineMap B{};             // coef unused: every evaluation brings its coefficients
     int ncells = 0;
-    int parts = 1;              // parts of a cell in the derivative pass
+    int parts = 1, value_parts = 1;  // parts of a cell in the derivative and the value pass
     int fill = 0;               // samples per cell, over the cells that hold any
     bool soa = false;           // layout of wts (weights_of): the cells are dense
     SampleSet SS{};             // cell-grouped samples
@@ -817,9 +819,13 @@ BSplineMetric *bspline_create(Metric &m, const size_t gs[3], const double origin
         const auto held = b->ncells - std::count(count.begin(), count.end() - 1, 0);
         b->fill = held > 0 ? static_cast<int>((n - count[b->ncells]) / held) : 0;
         b->soa = b->fill >= kDenseCell;
-        // about four rounds of a workgroup's lanes per part
-        b->parts = std::max(1, std::min(8, (*std::max_element(count.begin(), count.end()) + 4 * kBlock - 1) /
-                                               (4 * kBlock)));
+        // about four rounds of a workgroup's lanes per part; only the value pass
+        // walks the samples outside the valid region
+        auto parts_of = [](int most) { return std::max(1, std::min(8, (most + 4 * kBlock - 1) / (4 * kBlock))); };
+        if (b->ncells > 0)  // (a part's row is 1.5 KB: 100 MB of them at most)
+            b->parts = std::max(1, std::min(parts_of(*std::max_element(count.begin(), count.end() - 1)),
+                                            65536 / b->ncells));
+        b->value_parts = parts_of(*std::max_element(count.begin(), count.end()));
         std::vector<int> begin(b->ncells + 2, 0);
         for (int c = 0; c <= b->ncells; ++c) begin[c + 1] = begin[c] + count[c];
         std::vector<uint32_t> sflat(n);
@@ -986,7 +992,9 @@ BSplineMulti *bspline_multi_create(BSplineMetric &b, int S, const double *stages
         u->stage.alloc(static_cast<size_t>(S) * 12);
         u->pratio.alloc(S * nb);
         u->pratio_f.alloc(S * nb);
-        u->cellT.alloc(static_cast<size_t>(S) * std::max(1, b.ncells) * b.parts * 192);
+        // a row per cell and start of a launch, a row per part where few start
+        u->cellT.alloc(static_cast<size_t>(std::max(S, std::min(S, kFewStarts) * b.parts)) *
+                       std::max(1, b.ncells) * 192);
         u->deriv.alloc(S * u->np);
         u->joint.alloc(static_cast<size_t>(S) * kHistCopies * nb);
         u->marg.alloc(static_cast<size_t>(S) * kHistCopies * B);
@@ -1030,9 +1038,9 @@ static void multi_passes(BSplineMulti &u, const int *active, int nact, bool deri
     // so that one start's cells fill the chip
     const int cpb = nact >= 16 ? kCellsPerBlockMany : 1;
     const unsigned groups = static_cast<unsigned>((b.ncells + 1 + cpb - 1) / cpb);
-    const unsigned vparts = nact >= 4 ? 1 : b.parts;
+    const unsigned vparts = nact > kFewStarts ? 1 : b.value_parts;
     if (sizeof(R) == 4 && b.soa) {
-        auto kernel = nact >= 4 && b.fill >= kPairCell ? bs_value_f32<2> : bs_value_f32<1>;
+        auto kernel = nact > kFewStarts && b.fill >= kPairCell ? bs_value_f32<2> : bs_value_f32<1>;
         launch_kernel("bs_value_f32", kernel, dim3(nact, groups, vparts), dim3(kBlock), shm, m.F, m.Mv, b.B,
                       static_cast<const double *>(u.coef.ptr), stage, maps, own, active,
                       static_cast<const ChainConst *>(m.chain.ptr), static_cast<const uint32_t *>(b.idx.ptr),
@@ -1062,15 +1070,14 @@ static void multi_passes(BSplineMulti &u, const int *active, int nact, bool deri
                                  : reinterpret_cast<const R *>(u.pratio.ptr);
     // one start's parts fill the chip as workgroups of their own; many starts do
     // without, and leave the gather a third of the rows to read
-    const int rows = nact >= 4 ? 1 : b.parts;
+    const int rows = nact > kFewStarts ? 1 : b.parts;
     const size_t ratio_all = static_cast<size_t>(B) * B * sizeof(R);
     const size_t ratio_bytes = ratio_all <= kRatioLds ? ratio_all : 0;
     if (b.ncells > 0) {
-        launch_kernel("bs_deriv", b.soa ? bs_deriv<R, true> : bs_deriv<R, false>, dim3(nact, b.ncells * rows), dim3(kBlock), ratio_bytes, m.F, m.Mv, b.B,
+        launch_kernel("bs_deriv", b.soa ? bs_deriv<R, true> : bs_deriv<R, false>, dim3(nact, b.ncells, rows), dim3(kBlock), ratio_bytes, m.F, m.Mv, b.B,
                       stage, maps, own, active, static_cast<const int *>(b.cell_begin.ptr),
                       static_cast<const double *>(b.wts.ptr), static_cast<const uint8_t *>(b.fbin.ptr), m.P, pr,
-                      static_cast<const SampleRec<R> *>(rec), b.SS.n, b.parts, rows < b.parts, ratio_bytes > 0,
-                      u.cellT.ptr);
+                      static_cast<const SampleRec<R> *>(rec), b.SS.n, b.parts, ratio_bytes > 0, u.cellT.ptr);
         check_launch("bs_deriv");
     }
     launch_kernel("bs_gather", bs_gather, dim3((b.B.ncp + 3) / 4, nact), dim3(256), 0, b.B, active, b.ncells,
