@@ -654,7 +654,7 @@ __global__ __launch_bounds__(kBlock) void bs_deriv(FixedGrid F, MovingVol M, BSp
                                         cm.Q[d] * static_cast<double>(rr.gi[0])));
                 } else {
                     R gp[3];
-                    physical_gradient<R>(M, rr.gi, gp);
+                    physical_gradient(M, rr.gi, gp);
 #pragma unroll
                     for (int d = 0; d < 3; ++d) gq[d] = gp[d];
                     if (B.post) {

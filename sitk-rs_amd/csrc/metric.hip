@@ -1020,7 +1020,6 @@ static Metric *metric_create_impl(int kind, const Image &fixed, const int64_t *i
         index_to_physical(mg, mi2p);
         invert3_host(mi2p, m->Mv.p2i);
         if (opt.m_p2i) std::memcpy(m->Mv.p2i, opt.m_p2i, sizeof(m->Mv.p2i));
-        for (int i = 0; i < 9; ++i) m->Mv.p2i_f[i] = static_cast<float>(m->Mv.p2i[i]);
         {
             ChainConst cc;
             for (int d = 0; d < 3; ++d) {

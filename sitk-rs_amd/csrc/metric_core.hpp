@@ -484,7 +484,7 @@ __device__ __forceinline__ void moment_gradient(const MovingVol &M, const R gi[3
 #pragma unroll
         for (int d = 0; d < 3; ++d) g[d] = gi[d];
     } else {
-        physical_gradient<R>(M, gi, g);
+        physical_gradient(M, gi, g);
     }
 }
 

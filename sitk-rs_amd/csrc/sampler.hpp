@@ -72,7 +72,6 @@ struct MovingVol {
     long long stride1, stride2;
     double origin[3];
     double p2i[9];
-    float p2i_f[9];       // p2i rounded to float (the FP32 path's gradient)
     // Cubic B-spline coefficients of the volume (the moving image's cubic
     // interpolator, interpolator.rs:170-190): float for the FP32 path, double
     // for the FP64 path; nullptr with linear interpolation.
@@ -599,25 +598,15 @@ struct Interp {
 };
 
 // Index-space gradient -> physical gradient: g_d = sum_j gi_j * P[j][d].
-template <typename R>
-__device__ __forceinline__ void physical_gradient(const MovingVol &M, const R gi[3], R gp[3]) {
+__device__ __forceinline__ void physical_gradient(const MovingVol &M, const double gi[3], double gp[3]) {
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
-        R acc = static_cast<R>(-0.0);
-        acc += gi[0] * static_cast<R>(M.p2i[0 * 3 + d]);
-        acc += gi[1] * static_cast<R>(M.p2i[1 * 3 + d]);
-        acc += gi[2] * static_cast<R>(M.p2i[2 * 3 + d]);
+        double acc = -0.0;
+        acc += gi[0] * M.p2i[0 * 3 + d];
+        acc += gi[1] * M.p2i[1 * 3 + d];
+        acc += gi[2] * M.p2i[2 * 3 + d];
         gp[d] = acc;
     }
-}
-
-// FP32: the same sum with fused multiply-adds (three instructions per axis)
-template <>
-__device__ __forceinline__ void physical_gradient<float>(const MovingVol &M, const float gi[3],
-                                                         float gp[3]) {
-#pragma unroll
-    for (int d = 0; d < 3; ++d)
-        gp[d] = fmaf(gi[2], M.p2i_f[2 * 3 + d], fmaf(gi[1], M.p2i_f[1 * 3 + d], gi[0] * M.p2i_f[0 * 3 + d]));
 }
 
 }  // namespace sitkhip
