@@ -445,7 +445,8 @@ void batch_set_tiling(BatchEngine &b, const BatchTiling &t) {
     build_tiles(b);
 }
 
-// The five launches of one evaluation, in stream order. `profile`: time each launch with events (never under capture).
+// The five launches of one evaluation, in stream order. `profile`: time each
+// launch with events (never under capture).
 template <typename R>
 static void enqueue(BatchEngine &b, bool profile) {
     hipStream_t st = backend().stream;

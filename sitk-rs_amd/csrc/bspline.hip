@@ -1074,9 +1074,10 @@ static void multi_passes(BSplineMulti &u, const int *active, int nact, bool deri
     const size_t ratio_all = static_cast<size_t>(B) * B * sizeof(R);
     const size_t ratio_bytes = ratio_all <= kRatioLds ? ratio_all : 0;
     if (b.ncells > 0) {
-        launch_kernel("bs_deriv", b.soa ? bs_deriv<R, true> : bs_deriv<R, false>, dim3(nact, b.ncells, rows), dim3(kBlock), ratio_bytes, m.F, m.Mv, b.B,
-                      stage, maps, own, active, static_cast<const int *>(b.cell_begin.ptr),
-                      static_cast<const double *>(b.wts.ptr), static_cast<const uint8_t *>(b.fbin.ptr), m.P, pr,
+        launch_kernel("bs_deriv", b.soa ? bs_deriv<R, true> : bs_deriv<R, false>, dim3(nact, b.ncells, rows),
+                      dim3(kBlock), ratio_bytes, m.F, m.Mv, b.B, stage, maps, own, active,
+                      static_cast<const int *>(b.cell_begin.ptr), static_cast<const double *>(b.wts.ptr),
+                      static_cast<const uint8_t *>(b.fbin.ptr), m.P, pr,
                       static_cast<const SampleRec<R> *>(rec), b.SS.n, b.parts, ratio_bytes > 0, u.cellT.ptr);
         check_launch("bs_deriv");
     }
